@@ -105,6 +105,7 @@ class _Inputs:
     def __init__(self, seed: int):
         self.dev = torch.device("cuda", torch.cuda.current_device())
         self.gen = torch.Generator(device=self.dev).manual_seed(seed)
+        self.made = None    # a list: the operand triples, in the order they are made (for ``exact``)
 
     def normal(self, *shape, scale: float = 1.0, dtype=torch.bfloat16) -> torch.Tensor:
         return torch.randn(shape, generator=self.gen, device=self.dev, dtype=dtype).mul_(scale)
@@ -120,7 +121,10 @@ class _Inputs:
         qzeros = self.words(N, (groups + 7) // 8)
         if groups % 8:
             qzeros[:, -1] &= (1 << (4 * (groups % 8))) - 1
-        return self.words(N, K // 8), scales.to(torch.bfloat16), qzeros
+        triple = self.words(N, K // 8), scales.to(torch.bfloat16), qzeros
+        if self.made is not None:
+            self.made.append((*triple, G))
+        return triple
 
     def linear(self, K: int, N: int, G: int = 128, scale: float = 0.02, prepack: bool = True) -> Int4Linear:
         module = Int4Linear.from_packed(*self.packed(K, N, G, scale), G)
@@ -191,11 +195,12 @@ def _prepare_decode(case: dict, inp: _Inputs):
     mask = torch.ones((rows, length), dtype=torch.uint8, device=inp.dev)
     pad = torch.randint(0, min(slots, PROMPT) // 2, (rows, 1), generator=inp.gen, device=inp.dev)
     mask[torch.arange(length, device=inp.dev)[None] < pad] = 0          # prompts are padded on the left
-    step = NativeDecodeTrunk(trunk, cache, inp.normal(rows, 1, case["hidden"]), mask,
+    embedded = inp.normal(rows, 1, case["hidden"])
+    step = NativeDecodeTrunk(trunk, cache, embedded, mask,
                              torch.full((1,), slots, dtype=torch.int64, device=inp.dev))
     head = inp.linear(case["hidden"], HEAD, scale=_TRUNK_SCALE)
     appended = [t[:, :, slots] for layer in cache.layers for t in (layer.keys, layer.values)]
-    return {"trunk": trunk, "step": step, "short": step.short_form(slots), "head": head, "appended": appended}
+    return {"trunk": trunk, "cache": cache, "mask": mask, "embedded": embedded, "step": step, "short": step.short_form(slots), "head": head, "appended": appended}
 
 
 def _prepare_modules(case: dict, inp: _Inputs):
@@ -217,7 +222,10 @@ def _prepare_modules(case: dict, inp: _Inputs):
 
 
 def prepare(case: dict, seed: int):
-    inp = _Inputs(seed)
+    return _prepare(case, _Inputs(seed))
+
+
+def _prepare(case: dict, inp: _Inputs):
     kind = case["kind"]
     if kind == "linear":
         M, K, N, G = case["M"], case["K"], case["N"], case["G"]
@@ -237,7 +245,7 @@ def prepare(case: dict, seed: int):
             problems += [(d, weight(inter, hidden), False)]
         if case["head"]:
             problems.append((inp.normal(M, hidden), weight(hidden, HEAD), False))
-        return {"plan": ops.GroupedGemv(problems)}
+        return {"rows": [x for x, _, _ in problems], "plan": ops.GroupedGemv(problems)}
     if kind == "decode":
         return _prepare_decode(case, inp)
     if kind == "sample":
@@ -294,10 +302,10 @@ def work(case: dict) -> dict:
     if kind in ("linear", "sample"):
         M, K = (case["M"], case["K"]) if kind == "linear" else (2 * case["B"], case["K"])
         N = case["N"] if kind == "linear" else case["V"]
-        rows = 2 * N if case.get("form") == "gate_up" else N
+        columns = N // 2 if case.get("form") == "gate_up" else N
         extra = case["B"] * N * 2 if kind == "sample" else 0            # the draws
-        return {"bytes": _weight_bytes(K, rows, case.get("G", 128)) + 2 * M * (K + N) + extra,
-                "flops": 2 * M * K * rows}
+        return {"bytes": _weight_bytes(K, N, case.get("G", 128)) + 2 * M * (K + columns) + extra,
+                "flops": 2 * M * K * N}
     shapes = _layer_shapes(case) * case["layers"]
     if case.get("head") or kind == "decode":
         shapes.append((case["hidden"], HEAD))
@@ -328,3 +336,79 @@ def tolerance(case: dict):
     if case["kind"] in ("prompt", "replay"):
         return {"rel": 0.01, "max": 0.1}
     return {"rel": 0.004, "max": 0.05}
+
+
+# ------------------------------------------------------------------------------------------------ in 64 bits
+def _dense(qweight, scales, qzeros, G: int) -> torch.Tensor:
+    """The weight an operand triple stands for: ``(q - z) * s`` rounded to bf16 once, as float64 ``[N, K]``."""
+    shifts = torch.arange(0, 32, 4, device=qweight.device, dtype=torch.int32)
+    nibbles = lambda t: ((t[..., None] >> shifts) & 15).flatten(1)
+    q, z = nibbles(qweight), nibbles(qzeros)[:, :scales.shape[1]]
+    q = q.unflatten(1, (-1, G)) - z[..., None]
+    return (q.float() * scales.float()[..., None]).to(torch.bfloat16).flatten(1).double()
+
+
+def _rms(x, norm):
+    return norm.weight.double() * x * torch.rsqrt(x.square().mean(-1, keepdim=True) + norm.variance_epsilon)
+
+
+def _adapted(x, weight, module):
+    y = x @ weight.T
+    if isinstance(module, _Adapted):
+        a, b = (p["default"].weight.data.double() for p in (module.lora_A, module.lora_B))
+        y = y + module.scaling["default"] * (x @ a.T @ b.T)
+    return y
+
+
+def _exact_decode(case: dict, state, made) -> dict:
+    slot, heads, kv_heads = case["slots"], case["heads"], case["kv_heads"]
+    dim = case["hidden"] // heads
+    trunk, hidden = state["trunk"], state["embedded"][:, 0].double()
+    cos, sin = (t[0].double() for t in trunk.rotary_emb(state["embedded"], torch.full((1, 1), slot,
+                                                                                     device=hidden.device)))
+    turn = lambda t: t * cos + torch.cat([-t[..., dim // 2:], t[..., :dim // 2]], -1) * sin
+    seen, appended = state["mask"][:, None, :slot + 1] != 0, []
+    for layer, cached in zip(trunk.layers, state["cache"].layers):
+        at, x = layer.self_attn, _rms(hidden, layer.input_layernorm)
+        q, k, v = (_adapted(x, _dense(*next(made)), m).unflatten(1, (-1, dim)) for m in (at.q_proj, at.k_proj, at.v_proj))
+        q, k = turn(q), turn(k)
+        appended += [k, v]
+        keys, values = (torch.cat([c[:, :, :slot].double(), new[:, :, None]], 2).repeat_interleave(heads // kv_heads, 1)
+                        for c, new in ((cached.keys, k), (cached.values, v)))
+        scores = (keys * q[:, :, None]).sum(-1) * at.scaling
+        probs = scores.masked_fill(~seen, -math.inf).softmax(-1)
+        mixed = (probs[..., None] * values).sum(2).flatten(1)
+        hidden = hidden + _adapted(mixed, _dense(*next(made)), at.o_proj)
+        x = _rms(hidden, layer.post_attention_layernorm)
+        gate, up, down = (_dense(*next(made)) for _ in range(3))
+        hidden = hidden + (torch.nn.functional.silu(x @ gate.T) * (x @ up.T)) @ down.T
+    hidden = _rms(hidden, trunk.norm)
+    return {"hidden": hidden, "logits": hidden @ _dense(*next(made)).T, "appended": appended}
+
+
+def exact(case: dict, seed: int):
+    """What ``run`` returns for these inputs, in 64 bits (the dequantised weights are bf16 by definition)."""
+    inp = _Inputs(seed)
+    inp.made = []
+    state, kind = _prepare(case, inp), case["kind"]
+    made = iter(inp.made)
+    if kind == "decode":
+        return _exact_decode(case, state, made)
+    if kind == "linear":
+        y = state["x"].double() @ _dense(*next(made)).T
+        if case["form"] == "gate_up":
+            gate, up = y.chunk(2, dim=1)
+            y = torch.nn.functional.silu(gate) * up
+        return y
+    if kind == "grouped":
+        return [x.double() @ _dense(*m).T for x, m in zip(state["rows"], made)]
+    if kind == "sample":
+        return {"token": None, "logprob": None, "logits": state["x"].double() @ _dense(*next(made)).T}
+    out = []
+    for n, inputs in enumerate(state["x"]):
+        x, a, h = (t.double().requires_grad_(kind == "replay") for t in inputs)
+        q, k, v, o, gate, up, down = (_dense(*next(made)) for _ in range(7))
+        ys = (x @ q.T, x @ k.T, x @ v.T, a @ o.T, (torch.nn.functional.silu(h @ gate.T) * (h @ up.T)) @ down.T)
+        grads = torch.autograd.grad(ys, (x, a, h), [g.double() for g in state["grads"][n]]) if kind == "replay" else ()
+        out.append((*(y.detach() for y in ys), *grads))
+    return out
