@@ -128,6 +128,16 @@ typedef struct vrl_int4_problem {
     int32_t reserved[2];   /* 0 */
 } vrl_int4_problem;
 
+/*
+ * The products of a prompt pass: y[M,N] = x[M,K] . dequant(W)^T (or the fused gate||up form) for any number of
+ * activation rows, over the canonical operands, up to 8 problems in one launch (the q|k|v linears of a layer,
+ * policy.py:640-672).  Every problem has prepacked = 0 and the same K, G and fused_gate_up.  Shapes that the
+ * launch has no build for return VRL_INT4_ELIMIT and nothing is enqueued (it needs K % 128 == 0, G a power of two
+ * >= 32, and 512 bytes of LDS per group of a 128-row weight tile): rebuild the weight with
+ * vrl_int4_dequant_bf16() and use a library product, which is also the faster form from about 2048 rows on.
+ */
+int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_problems, void *hip_stream);
+
 typedef struct vrl_int4_plan_info {
     int32_t n_problems;    /* records in the blob */
     int32_t total_tiles;   /* 16-column output tiles over all problems */

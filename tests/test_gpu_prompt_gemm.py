@@ -1,0 +1,175 @@
+"""Prompt-sized int4 products (``vrl_int4_gemm_bf16``) against the same product over the dequantised weight.
+
+The weight tile is bit-exact (``test_gpu_parity``), so the reference is a float64 product over it.  Tolerance: one
+bf16 rounding of the result (2^-8 relative covers it) and the worst case of K fp32 additions, K 2^-24 sum |x w|;
+the fused form carries both operands' sums through ``silu(g) * u`` (|silu'| < 1.1) and 2^-18 for exp and divide.
+"""
+
+import ctypes
+
+import pytest
+import torch
+
+from visionrl_amd import _lib, ops
+from visionrl_amd import linear as linear_mod
+from visionrl_amd.linear import Int4GateUpSiLU, Int4Linear
+
+
+def _triple(gen, K, N, G, dev):
+    groups = K // G
+    words = lambda *s: torch.randint(-2 ** 31, 2 ** 31, s, generator=gen, dtype=torch.int64).to(torch.int32)
+    zeros = words(N, (groups + 7) // 8)
+    if groups % 8:
+        zeros[:, -1] &= (1 << (4 * (groups % 8))) - 1
+    scales = (torch.randn(N, groups, generator=gen) * 0.02).to(torch.bfloat16)      # negative scales are legal
+    return tuple(t.to(dev) for t in (words(N, K // 8), scales, zeros))
+
+
+def _reference(x, triple, G, fused):
+    w = ops.int4_dequant(*triple, G).double()
+    K = x.shape[1]
+    ref, eps = x.double() @ w.T, K * 2.0 ** -24 * (x.double().abs() @ w.abs().T)
+    if fused:
+        (g, u), (eg, eu) = ref.chunk(2, 1), eps.chunk(2, 1)
+        s = torch.nn.functional.silu(g)
+        ref, eps = s * u, 1.1 * eg * (u.abs() + eu) + s.abs() * eu + 2.0 ** -18 * (s * u).abs()
+    return ref, eps + 2.0 ** -8 * ref.abs()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,G,fused,n", [
+    (33, 64, 256, 128, False, 1),       # 32x64 tiles, one row into the second
+    (64, 2048, 2048, 128, False, 1),
+    (65, 2050, 512, 32, False, 1),      # odd widths: narrow stores, a ragged last tile
+    (40, 17, 256, 64, False, 3),
+    (500, 2048, 256, 128, False, 1),    # 64x64 tiles
+    (512, 3000, 512, 64, False, 2),     # 64x128 and 128x128 tiles by tile count
+    (200, 2 * 1000, 256, 128, True, 1),
+    (129, 2 * 77, 512, 32, True, 1),
+    (33, 2 * 5632, 2048, 128, True, 1),
+    (300, 1000, 384, 128, False, 1),    # K not a multiple of 256: the tiles with shorter chunks
+    (130, 1000, 128, 128, False, 1),    # one chunk
+    (48, 96, 128, 32, True, 1),
+    (1664, 2048, 512, 128, False, 3),   # more tiles than CUs
+    (2047, 2 * 1500, 256, 256, True, 1),
+    (70, 128, 4096, 32, False, 1),      # the largest tables of scales
+    (600, 2500, 5632, 32, False, 1),
+])
+def test_prompt_gemm_matches_dequantised_product(M, N, K, G, fused, n):
+    gen = torch.Generator().manual_seed(M + N + K)
+    dev = torch.device("cuda:0")
+    triples = [_triple(gen, K, N + 16 * i, G, dev) for i in range(n)]
+    x = torch.randn(M, K, generator=gen).to(torch.bfloat16).to(dev)
+    ys = ops.int4_gemm(x, triples, G, fused)
+    assert ys is not None
+    again = ops.int4_gemm(x, triples, G, fused)
+    for y, y2, t in zip(ys, again, triples):
+        ref, tol = _reference(x, t, G, fused)
+        assert y.shape == ref.shape and torch.equal(y, y2)
+        assert bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+def test_prompt_gemm_leaves_other_operands_to_the_general_route():
+    gen, dev = torch.Generator().manual_seed(3), torch.device("cuda:0")
+    x = torch.randn(64, 360, generator=gen).to(torch.bfloat16).to(dev)
+    assert ops.int4_gemm(x, [_triple(gen, 360, 32, 40, dev)], 40) is None            # no MFMA form
+    flat = torch.randn(64 * 256 + 1, generator=gen).to(torch.bfloat16).to(dev)
+    triple = _triple(gen, 256, 32, 128, dev)
+    shifted = flat[1:].view(64, 256)
+    assert ops.int4_gemm(shifted, [triple], 128) is None                             # misaligned view
+    module = Int4Linear.from_packed(*triple, 128)
+    assert torch.equal(module(shifted), torch.nn.functional.linear(shifted, module.dequantize()))
+    big = _triple(gen, 16384, 40000, 32, dev)                                        # scales beyond LDS
+    x = torch.randn(400, 16384, generator=gen).to(torch.bfloat16).to(dev)
+    assert ops.int4_gemm(x, [big], 32) is None
+
+
+@pytest.mark.gpu
+def test_prompt_calls_of_a_group_share_one_launch(monkeypatch):
+    gen, dev = torch.Generator().manual_seed(5), torch.device("cuda:0")
+    q, k, v = (Int4Linear.from_packed(*_triple(gen, 256, n, 128, dev), 128).prepack_() for n in (256, 64, 64))
+    x = torch.randn(2, 50, 256, generator=gen).to(torch.bfloat16).to(dev)
+    alone = [m(x) for m in (q, k, v)]
+    q.group_with(k, v)
+    calls = []
+    real = ops.int4_gemm
+    monkeypatch.setattr(linear_mod.ops, "int4_gemm", lambda *a: calls.append(1) or real(*a))
+    for want, m in zip(alone, (q, k, v)):
+        assert torch.equal(m(x), want)
+    assert len(calls) == 1
+    q(x)
+    x.mul_(2)                                   # the input changed: nothing is handed over
+    assert torch.equal(k(x), real(x.view(100, 256), [k._canonical()], 128)[0].view(2, 50, 64))
+    q(x)
+    k.scales.mul_(2)                            # the sibling's weight changed
+    assert torch.equal(k(x), real(x.view(100, 256), [k._canonical()], 128)[0].view(2, 50, 64))
+    side = torch.cuda.Stream()
+    q(x)
+    side.wait_stream(torch.cuda.current_stream())
+    n = len(calls)
+    with torch.cuda.stream(side):               # a call on another stream computes its own
+        v(x)
+    assert len(calls) == n + 1
+    torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_watched_prompt_calls_stay_on_the_general_route():
+    """Transforms and modes see torch operators: a tangent, a batch dimension and a dispatch mode get through."""
+    gen, dev = torch.Generator().manual_seed(7), torch.device("cuda:0")
+    m = Int4Linear.from_packed(*_triple(gen, 256, 64, 128, dev), 128)
+    x, t = (torch.randn(40, 256, generator=gen).to(torch.bfloat16).to(dev) for _ in range(2))
+    with torch.no_grad():
+        dense = torch.nn.functional.linear(t, m.dequantize())
+        _, tangent = torch.func.jvp(m, (x,), (t,))
+        assert torch.equal(tangent, dense)
+        batched = torch.func.vmap(m)(torch.stack([x, t]))
+        assert torch.allclose(batched[1].float(), dense.float(), rtol=2.0 ** -7, atol=1e-3)
+        from torch.utils.flop_counter import FlopCounterMode
+        with FlopCounterMode(display=False) as flops:
+            m(x)
+        assert flops.get_total_flops() == 2 * 40 * 256 * 64
+
+
+@pytest.mark.gpu
+def test_prompt_gemm_replays_in_a_graph():
+    gen, dev = torch.Generator().manual_seed(9), torch.device("cuda:0")
+    gate, up = (Int4Linear.from_packed(*_triple(gen, 256, 128, 128, dev), 128) for _ in range(2))
+    mlp = Int4GateUpSiLU(gate, up)
+    x = torch.randn(40, 256, generator=gen).to(torch.bfloat16).to(dev)
+    with torch.no_grad():
+        mlp(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = mlp(x)
+        for seed in range(3):
+            x.copy_(torch.randn(40, 256, generator=gen).to(torch.bfloat16))
+            graph.replay()
+            want = mlp(x)
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+
+
+def test_prompt_gemm_rejects_bad_calls():
+    lib = _lib.load()
+    raw = ctypes.create_string_buffer(4096 + 64)
+    p = (ctypes.addressof(raw) + 15) & ~15
+    table = (_lib.Problem * 2)()
+
+    def call(n=1, **fields):
+        for rec in table:
+            rec.x = rec.qweight = rec.scales = rec.qzeros = rec.y = p
+            rec.M, rec.N, rec.K, rec.G, rec.fused_gate_up, rec.prepacked = 64, 32, 256, 128, 0, 0
+        for name, value in fields.items():
+            setattr(table[n - 1], name, value)
+        return lib.vrl_int4_gemm_bf16(table, n, None)
+
+    assert lib.vrl_int4_gemm_bf16(None, 1, None) == 1003
+    assert call(0) == 1001 and lib.vrl_int4_gemm_bf16(table, 9, None) == 1001
+    assert call(x=None) == 1003 and call(y=p + 2) == 1002
+    assert call(M=0) == 1001 and call(prepacked=1) == 1001
+    assert call(2, K=512) == 1001 and call(2, G=64) == 1001 and call(2, fused_gate_up=1) == 1001
+    assert call(N=33, fused_gate_up=1) == 1001
+    assert call(K=264, G=8) == 1005 and call(K=192, G=64) == 1005 and call(K=384, G=96) == 1005

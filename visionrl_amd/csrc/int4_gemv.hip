@@ -34,6 +34,7 @@
 
 #include <atomic>
 
+#include "host_checks.hpp"
 #include "stream_kernel.hpp"
 #include "rows32.hpp"
 
@@ -55,21 +56,6 @@ constexpr StreamShape STREAM_SHAPES[3] = {{4, 15, 32 * 1024}, {8, 2, 72 * 1024},
 constexpr size_t LDS_PER_CU = 160 * 1024;
 constexpr size_t STREAM_LDS_CAP = LDS_PER_CU - 1024;   // dynamic LDS a grouped launch may ask for (the kernels hold a few static words)
 constexpr size_t DIRECT_LDS_CAP = 150 * 1024;   // plan-free launches: staged activations + partial tiles
-
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-int check_problem(const void *x, const void *qw, const void *sc, const void *qz, const void *y,
-                  long M, long N, long K, long G) {
-    if (!x || !qw || !sc || !qz || !y) return VRL_INT4_ENULL;
-    if (M < 1 || N < 1 || K < 8 || G < 8) return VRL_INT4_ESHAPE;
-    if (K % 8 != 0 || G % 8 != 0 || K % G != 0) return VRL_INT4_ESHAPE;
-    if (N * K >= (1L << 40) || M * K >= (1L << 31) || M * N >= (1L << 31)) return VRL_INT4_ESHAPE;
-    if (!aligned16(x) || !aligned16(qw) || !aligned16(sc) || !aligned16(qz) || !aligned16(y))
-        return VRL_INT4_EALIGN;
-    return VRL_INT4_OK;
-}
-
-bool pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 
 // shapes the MFMA kernels take; everything else goes to the generic kernel
 bool tile_path_ok(const DevProblem &p) {
@@ -117,16 +103,6 @@ size_t tile_smem_bytes(int M, int kc) {
     const size_t xbytes = (size_t)M * (kc + XPAD) * 2;
     const size_t rbytes = (size_t)TileCfg<R, MB, TILE_WPB>::RED_FLOATS * 4;
     return xbytes > rbytes ? xbytes : rbytes;
-}
-
-int device_cu_count() {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            cus = v;
-    }
-    return cus;
 }
 
 template <int R, int MB>

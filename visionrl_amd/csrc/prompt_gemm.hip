@@ -1,0 +1,402 @@
+// Prompt-sized products over the canonical int4 operands: y[M,N] = x[M,K] . dequant(W)^T for more activation
+// rows than the GEMV launches take (the prompt pass, vrl/models/families/janus_pro/policy.py:640-672, and the
+// forward of a training replay, policy.py:419-424).
+//
+// One launch covers up to GEMM_MAX problems (q|k|v of a layer; gate|up with the SiLU epilogue is one problem).
+// A workgroup owns BM activation rows x BN weight rows and walks K in chunks of KC.  Both operands reach LDS by
+// direct loads (no registers in flight): the activations as bf16, the weights as the packed words, a quarter of
+// the bytes.  Every wave reads its own weight rows from LDS, rebuilds the exactly rounded bf16 weights in
+// registers (as the GEMV kernels do) and feeds them to v_mfma_f32_16x16x32_bf16 as the A operand, the
+// activations as the B operand: a lane then holds four neighbouring output columns of one row.  No bf16 copy of
+// the weight is ever written.
+//
+// Layout in LDS: activation rows are KC bf16 with their 16-byte pieces permuted within the row (piece j of row r
+// sits at j ^ f(r)), so that the 16 rows a fragment read touches fall on different banks; the direct loads
+// permute the global addresses instead of the LDS side, which they fill in lane order.  Scales and zero-points of
+// all of K are laid down once per workgroup as one word each.
+#include <atomic>
+
+#include "canonical.hpp"
+#include "host_checks.hpp"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
+
+constexpr int GEMM_MAX = 8;
+
+struct GemmRec {
+    const uint16_t *x;
+    const uint32_t *qweight;
+    const uint16_t *scales;
+    const uint32_t *qzeros;
+    uint16_t *y;
+    int32_t M, N;        // N: weight rows (gate||up: both halves)
+    int32_t tile_begin;  // first tile of the record in the launch
+    int32_t mtiles;
+};
+struct GemmArgs {
+    GemmRec recs[GEMM_MAX];
+    int32_t n, K, gshift, tiles;   // every record shares K and the group size 1 << gshift
+};
+
+// One packed word -> eight exactly rounded bf16 weights in k order.  float(q) by the byte converter, then
+// fma(q, s, -z s): both products are exact (4 by 8 bits), so the sum is the exact (q - z) s and the conversion
+// is the one rounding of the contract.  Plain instructions, so that the compiler can issue them between MFMAs:
+// 23 against the 19 of the GEMV kernels' asm block, which cannot be split.
+struct ScaleZero { float s, zs; };
+
+__device__ __forceinline__ ScaleZero scale_zero(uint32_t meta) {   // (scale bits << 16) | zero
+    const float s = bf16_bits_to_f32(meta >> 16);
+    return {s, -s * (float)(meta & 0xFFu)};
+}
+
+__device__ __forceinline__ bf16x8_t dequant_natural(uint32_t v, const ScaleZero &c) {
+    const uint32_t even = v & 0x0F0F0F0Fu, odd = (v >> 4) & 0x0F0F0F0Fu;
+    u32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        o[i] = pack_bf16_rne(__builtin_fmaf((float)((even >> (8 * i)) & 0xFFu), c.s, c.zs),
+                             __builtin_fmaf((float)((odd >> (8 * i)) & 0xFFu), c.s, c.zs));
+    return __builtin_bit_cast(bf16x8_t, o);
+}
+
+// 16 bytes per lane from global memory to LDS at `lds` + 16 * lane; counted by vmcnt, touches no register.
+__device__ __forceinline__ void dma16(uint8_t *lds, const uint8_t *g) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(uintptr_t)g,
+                                     (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
+}
+
+// WM x WN x WK waves share a tile: WM and WN split its rows and columns, WK the k of every chunk (their partial
+// tiles meet in LDS at the end).  A wave owns MB x NB blocks of 16 x 16.  S chunks of KC k are in LDS at a time.
+template <int WM_, int WN_, int WK_, int MB_, int NB_, int KC_, int S_>
+struct GemmCfg {
+    static constexpr int WM = WM_, WN = WN_, WK = WK_, MB = MB_, NB = NB_, KC = KC_, S = S_;
+    static constexpr int WAVES = WM * WN * WK, THREADS = WAVES * WAVE;
+    static constexpr int BM = 16 * MB * WM, BN = 16 * NB * WN;
+    static constexpr int T = KC / 32 / WK;                // MFMA steps per wave and chunk = packed words a lane reads per row
+    static constexpr int XP = KC / 8, WP = KC / 32;       // 16-byte pieces of a staged activation row, of a weight row
+    static constexpr int X_BYTES = BM * KC * 2, W_BYTES = BN * KC / 2;
+    // direct loads per wave and chunk (where the words are fewer loads than waves, waves repeat each other's)
+    static constexpr int W_UNITS = W_BYTES / 1024;
+    static constexpr int X_LOADS = X_BYTES / 1024 / WAVES, W_LOADS = W_UNITS < WAVES ? 1 : W_UNITS / WAVES;
+    static constexpr int STAGE = X_BYTES + W_BYTES;
+    static_assert(X_BYTES % (1024 * WAVES) == 0 && (WAVES % W_UNITS == 0 || W_UNITS % WAVES == 0), "whole direct loads");
+    static_assert(T == 2 || T == 4, "a lane's words are one 8- or 16-byte read, inside one group of 32 k");
+    static_assert(MB % WK == 0, "the waves that split K finish a share of the row blocks each");
+    static constexpr size_t PARTIAL = WK > 1 ? (size_t)WAVES * MB * NB * 1024 : 0;   // over the stages, once they are done
+    static constexpr size_t lds(int groups) {
+        const size_t loop = (size_t)S * STAGE + (size_t)BN * groups * 4;
+        return loop > PARTIAL ? loop : PARTIAL;
+    }
+};
+
+// Piece j of staged row r sits at j ^ f(r).  LDS has 64 banks; a 16-byte read goes in four turns of sixteen lanes,
+// lanes {0-3, 12-15, 20-27} and {4-11, 16-19, 28-31} of each half of the wave, an 8-byte read in two turns of half
+// a wave.  f is chosen per row length (P pieces) and per distance T of two lane quarters' pieces so that a turn's
+// lanes cover the banks once: where a turn mixes two quarters, flipping the piece bit that tells them apart must
+// not change which of the two sets a row belongs to (its bits 2 and 3).  Half of the LDS cycles were conflicts
+// with f(r) = r & 15.
+template <int P, int T>
+__device__ __forceinline__ int activation_swizzle(int r) {
+    if (P == 8) return (r >> 1 & 4) | (r & 2) | (r >> 2 & 1);
+    return T == 4 ? (r & 10) | (r & 1) << 2 | (r >> 2 & 1) : r & 15;
+}
+template <int P>
+__device__ __forceinline__ int weight_swizzle(int r) {
+    return P == 2 ? r >> 3 & 1 : P == 4 ? -(r >> 2) & 3 : r >> 1 & 7;
+}
+
+// The weight row behind local row r of column tile nt.  Fused records: a wave's first NB/2 blocks of 16 rows are
+// gate rows, the others the up rows of the same columns.  Clamped: what lies past the end is never stored.
+template <class C, bool FUSED>
+__device__ __forceinline__ int weight_row(int r, int nt, int N) {
+    if (!FUSED) return min(nt * C::BN + r, N - 1);
+    constexpr int HB = C::NB > 1 ? C::NB / 2 : 1;
+    const int half = (r / (16 * HB)) & 1;
+    const int col = nt * (C::BN / 2) + (r / (32 * HB)) * (16 * HB) + r % (16 * HB);
+    return half * (N / 2) + min(col, N / 2 - 1);
+}
+
+template <class C, bool FUSED>
+__global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 ? 2 : 1) void gemm_int4_kernel(GemmArgs args) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lc = lane & 15, kq = lane >> 4;
+    const int wn = wave % C::WN, wm = wave / C::WN % C::WM, wk = wave / (C::WN * C::WM);
+
+    // Consecutive workgroups go to the eight XCDs in turn: each XCD gets one contiguous range of tiles, walked in
+    // bands of GROUP_M row tiles, so that what its L2 holds is read by several of its workgroups.
+    constexpr int XCDS = 8, GROUP_M = 8;
+    const int xcd = blockIdx.x % XCDS, per = args.tiles / XCDS, rest = args.tiles % XCDS;
+    const int tile = xcd * per + min(xcd, rest) + blockIdx.x / XCDS;
+    int ri = 0;
+    for (int i = 1; i < args.n; ++i)
+        if (tile >= args.recs[i].tile_begin) ri = i;
+    const GemmRec p = args.recs[ri];
+    const int K = args.K, kwords = K >> 3, groups = K >> args.gshift, zwords = (groups + 7) >> 3;
+    const int out_cols = FUSED ? p.N / 2 : p.N;
+    constexpr int COLS = FUSED ? C::BN / 2 : C::BN;
+    int mt, nt;
+    {
+        const int local = tile - p.tile_begin, ntiles = (out_cols + COLS - 1) / COLS;
+        const int band = local / (GROUP_M * ntiles), rows = min(GROUP_M, p.mtiles - band * GROUP_M);
+        const int in = local - band * GROUP_M * ntiles;
+        mt = band * GROUP_M + in % rows;
+        nt = in / rows;
+    }
+
+    uint32_t *table = reinterpret_cast<uint32_t *>(smem + C::S * C::STAGE);
+
+    // addresses of this wave's direct loads; a chunk is KC k further on
+    const uint8_t *xsrc[C::X_LOADS], *wsrc[C::W_LOADS];
+#pragma unroll
+    for (int i = 0; i < C::X_LOADS; ++i) {
+        const int at = (wave * C::X_LOADS + i) * 64 + lane;              // 16-byte piece of the staged tile
+        const int r = at / C::XP, j = (at % C::XP) ^ activation_swizzle<C::XP, C::T>(r);
+        xsrc[i] = reinterpret_cast<const uint8_t *>(p.x + (long)min(mt * C::BM + r, p.M - 1) * K + 8 * j);
+    }
+#pragma unroll
+    for (int i = 0; i < C::W_LOADS; ++i) {
+        const int at = (wave * C::W_LOADS + i) % C::W_UNITS * 64 + lane;
+        const int r = at / C::WP, j = (at % C::WP) ^ weight_swizzle<C::WP>(r);
+        wsrc[i] = reinterpret_cast<const uint8_t *>(p.qweight + (long)weight_row<C, FUSED>(r, nt, p.N) * kwords + 4 * j);
+    }
+    const int chunks = K / C::KC;
+    auto issue = [&](int chunk, int slot) {
+        const long c = min(chunk, chunks - 1);   // past the end: a repeat nobody reads, so that every chunk counts alike
+        uint8_t *base = smem + slot * C::STAGE + wave * (C::X_LOADS * 1024);
+#pragma unroll
+        for (int i = 0; i < C::X_LOADS; ++i) dma16(base + i * 1024, xsrc[i] + c * (C::KC * 2));
+        uint8_t *wbase = smem + slot * C::STAGE + C::X_BYTES + wave * C::W_LOADS % C::W_UNITS * 1024;
+#pragma unroll
+        for (int i = 0; i < C::W_LOADS; ++i) dma16(wbase + i * 1024, wsrc[i] + c * (C::KC / 2));
+    };
+
+    // scales and zero-points of the tile's rows, (scale bits << 16) | zero, group-major
+    for (int idx = tid; idx < C::BN * groups; idx += C::THREADS) {
+        const int r = idx / groups, g = idx - r * groups;
+        const long row = weight_row<C, FUSED>(r, nt, p.N);
+        const uint32_t sb = as_global(p.scales)[row * groups + g];
+        const uint32_t z = ((gptr_cu32)(uintptr_t)p.qzeros)[row * zwords + (g >> 3)] >> (4 * (g & 7)) & 0xFu;
+        table[g * C::BN + r] = (sb << 16) | z;
+    }
+#pragma unroll
+    for (int s = 0; s < C::S - 1; ++s) issue(s, s);
+
+    f32x4_t acc[C::MB][C::NB];
+#pragma unroll
+    for (int b = 0; b < C::MB; ++b)
+#pragma unroll
+        for (int n = 0; n < C::NB; ++n) acc[b][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    const int xrow0 = wm * 16 * C::MB + lc, wrow0 = wn * 16 * C::NB + lc;
+    // rows of the other blocks differ by multiples of 16, which no swizzle sees
+    const int xswz = activation_swizzle<C::XP, C::T>(lc), xpiece = 4 * C::T * wk + C::T * kq;
+    const int wbyte = 16 * C::T * wk + 4 * C::T * kq;
+    const int woff = wrow0 * (C::KC / 2) + (((wbyte >> 4) ^ weight_swizzle<C::WP>(lc)) << 4) + (wbyte & 15);
+    const int xoff = xrow0 * (C::KC * 2);
+    int slot = 0;
+    for (int c = 0; c < chunks; ++c) {
+        // chunk c has arrived for every wave, and every wave is done with the slot that is filled next
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"((C::S - 2) * (C::X_LOADS + C::W_LOADS)) : "memory");
+        const uint8_t *xs = smem + slot * C::STAGE + xoff;
+        const uint8_t *ws = smem + slot * C::STAGE + C::X_BYTES + woff;
+        uint32_t w[C::NB][C::T];
+        ScaleZero sz[C::NB];
+        const int g = (c * C::KC + 32 * C::T * wk + 8 * C::T * kq) >> args.gshift;
+#pragma unroll
+        for (int n = 0; n < C::NB; ++n) {
+            typedef __attribute__((ext_vector_type(C::T))) uint32_t words_t;
+            const words_t v = *reinterpret_cast<const words_t *>(ws + n * (16 * C::KC / 2));
+#pragma unroll
+            for (int t = 0; t < C::T; ++t) w[n][t] = v[t];
+            sz[n] = scale_zero(table[g * C::BN + wrow0 + 16 * n]);
+        }
+        bf16x8_t xb[C::MB];
+        auto fetch = [&](int t, int b) {
+            return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t *>(
+                xs + b * (16 * C::KC * 2) + (((xpiece + t) ^ xswz) << 4)));
+        };
+#pragma unroll
+        for (int b = 0; b < C::MB; ++b) xb[b] = fetch(0, b);
+        issue(c + C::S - 1, slot == 0 ? C::S - 1 : slot - 1);
+        // the next block's weights are rebuilt between this block's MFMAs, and the next step's activations are
+        // requested as soon as the last block has used this step's
+        bf16x8_t wa = dequant_natural(w[0][0], sz[0]);
+#pragma unroll
+        for (int i = 0; i < C::T * C::NB; ++i) {
+            const int t = i / C::NB, n = i % C::NB;
+            bf16x8_t next = wa;
+            if (i + 1 < C::T * C::NB) next = dequant_natural(w[(i + 1) % C::NB][(i + 1) / C::NB], sz[(i + 1) % C::NB]);
+#pragma unroll
+            for (int b = 0; b < C::MB; ++b) {
+                acc[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, xb[b], acc[b][n], 0, 0, 0);
+                if (n == C::NB - 1 && t + 1 < C::T) xb[b] = fetch(t + 1, b);
+            }
+            wa = next;
+        }
+        slot = slot + 1 == C::S ? 0 : slot + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the repeats must not land in another workgroup's LDS
+
+    int b0 = 0;
+    constexpr int OWN = C::MB / C::WK;   // row blocks a wave finishes
+    if constexpr (C::WK > 1) {
+        // partial tiles meet in LDS: wave wk finishes blocks wk * OWN ...
+        __syncthreads();
+        f32x4_t *red = reinterpret_cast<f32x4_t *>(smem);
+        b0 = wk * OWN;
+        const int base = (wm * C::WN + wn) * C::MB * C::NB, step = C::WM * C::WN * C::MB * C::NB;
+#pragma unroll
+        for (int b = 0; b < C::MB; ++b)
+#pragma unroll
+            for (int n = 0; n < C::NB; ++n) red[(wk * step + base + b * C::NB + n) * WAVE + lane] = acc[b][n];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < OWN; ++b)
+#pragma unroll
+            for (int n = 0; n < C::NB; ++n) {
+                f32x4_t sum = red[(base + (b0 + b) * C::NB + n) * WAVE + lane];
+#pragma unroll
+                for (int k = 1; k < C::WK; ++k) sum += red[(k * step + base + (b0 + b) * C::NB + n) * WAVE + lane];
+                acc[b][n] = sum;
+            }
+    }
+
+    // lane: row lc of each row block, columns 4 kq .. 4 kq + 3 of each column block
+    constexpr int OB = FUSED ? C::NB / 2 : C::NB;
+    const bool wide = (out_cols & 3) == 0;
+#pragma unroll
+    for (int b = 0; b < OWN; ++b) {
+        const int m = mt * C::BM + xrow0 + 16 * (b0 + b);
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int n = 0; n < OB; ++n) {
+            const int col = nt * COLS + wn * (16 * OB) + 16 * n + 4 * kq;
+            f32x4_t v = acc[b][n];
+            if constexpr (FUSED) {
+                const f32x4_t u = acc[b][n + OB];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = (v[i] / (1.0f + __expf(-v[i]))) * u[i];
+            }
+            uint16_t *y = p.y + (long)m * out_cols + col;
+            const u32x2_t o = {pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3])};
+            if (wide) {
+                if (col < out_cols) *reinterpret_cast<u32x2_t *>(y) = o;
+            } else {
+                if (col < out_cols) y[0] = (uint16_t)o[0];
+                if (col + 1 < out_cols) y[1] = (uint16_t)(o[0] >> 16);
+                if (col + 2 < out_cols) y[2] = (uint16_t)o[1];
+                if (col + 3 < out_cols) y[3] = (uint16_t)(o[1] >> 16);
+            }
+        }
+    }
+}
+
+constexpr size_t GEMM_LDS_CAP = 160 * 1024;
+
+template <class C, bool FUSED>
+long gemm_tiles(GemmArgs &args) {
+    constexpr int COLS = FUSED ? C::BN / 2 : C::BN;
+    long tiles = 0;
+    for (int i = 0; i < args.n; ++i) {
+        GemmRec &r = args.recs[i];
+        r.mtiles = (r.M + C::BM - 1) / C::BM;
+        r.tile_begin = (int)tiles;
+        tiles += (long)r.mtiles * (((FUSED ? r.N / 2 : r.N) + COLS - 1) / COLS);
+        if (tiles > (1L << 24)) return tiles;
+    }
+    args.tiles = (int)tiles;
+    return tiles;
+}
+
+template <class C>
+bool gemm_fits(const GemmArgs &args) {
+    return args.K % C::KC == 0 && C::lds(args.K >> args.gshift) <= GEMM_LDS_CAP;
+}
+
+template <class C, bool FUSED>
+int launch_gemm(GemmArgs &args, hipStream_t stream) {
+    const long tiles = gemm_tiles<C, FUSED>(args);
+    if (tiles > (1L << 24)) return VRL_INT4_ESHAPE;
+    if (!gemm_fits<C>(args)) return VRL_INT4_ELIMIT;
+    const size_t lds = C::lds(args.K >> args.gshift);
+    auto kernel = &gemm_int4_kernel<C, FUSED>;
+    if (lds > 64 * 1024) {   // once per build and device, at the largest size a launch may ask for
+        static std::atomic<uint64_t> raised{0};
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+        const uint64_t bit = 1ull << (dev & 63);
+        if (!(raised.load(std::memory_order_relaxed) & bit)) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_LDS_CAP);
+            if (e != hipSuccess) return (int)e;
+            raised.fetch_or(bit, std::memory_order_relaxed);
+        }
+    }
+    return vrl_launch(kernel, dim3((unsigned)tiles), dim3(C::THREADS), lds, stream, args);
+}
+
+// Whether the launch takes this tile: all its tiles run at once, one workgroup per CU.
+template <class C, bool FUSED>
+bool gemm_one_round(GemmArgs &args, long cus) {
+    return gemm_fits<C>(args) && gemm_tiles<C, FUSED>(args) <= cus;
+}
+
+using Gemm32x64 = GemmCfg<1, 4, 2, 2, 1, 256, 2>;
+using Gemm64x64 = GemmCfg<1, 4, 4, 4, 1, 256, 2>;
+using Gemm64x128 = GemmCfg<1, 4, 4, 4, 2, 256, 2>;
+using Gemm128x128Split = GemmCfg<1, 4, 2, 8, 2, 128, 3>;
+using Gemm128x128 = GemmCfg<1, 4, 1, 8, 2, 64, 2>;
+
+// The smallest tile whose launch is one round of workgroups: until the chip is full a launch takes as long as one
+// tile does, and a smaller tile is done sooner (K = 2048, one round: 8.5 / 9.4 / 15.0 / 20.7 us in the order
+// below; its waves split K, since a tile alone on its CU is bound by the latency of its own chain).  Beyond that
+// the 128x128 tile whose waves split nothing, three or four workgroups per CU (25.2 us alone, but 60.7 us for
+// 1664 rows of q|k|v against 72.1 with the K split).  Measured at 48 to 1664 rows of q|k|v (3 x 2048), o_proj,
+// gate|up (11264) and down_proj (K = 5632): the rule's choice was the best or within 2 % of it at every one.
+template <bool FUSED>
+int dispatch_gemm(GemmArgs &args, hipStream_t stream) {
+    const long cus = device_cu_count();
+    if constexpr (!FUSED) {   // a wave of these holds one block of columns, a fused one needs gate and up
+        if (gemm_one_round<Gemm32x64, false>(args, cus)) return launch_gemm<Gemm32x64, false>(args, stream);
+        if (gemm_one_round<Gemm64x64, false>(args, cus)) return launch_gemm<Gemm64x64, false>(args, stream);
+    }
+    if (gemm_one_round<Gemm64x128, FUSED>(args, cus)) return launch_gemm<Gemm64x128, FUSED>(args, stream);
+    if (gemm_one_round<Gemm128x128Split, FUSED>(args, cus)) return launch_gemm<Gemm128x128Split, FUSED>(args, stream);
+    return launch_gemm<Gemm128x128, FUSED>(args, stream);
+}
+
+}  // namespace
+
+extern "C" int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_problems, void *hip_stream) {
+    if (!problems) return VRL_INT4_ENULL;
+    if (n_problems < 1 || n_problems > GEMM_MAX) return VRL_INT4_ESHAPE;
+    GemmArgs args;
+    memset(&args, 0, sizeof args);
+    const vrl_int4_problem &q0 = problems[0];
+    const bool fused = q0.fused_gate_up != 0;
+    for (int i = 0; i < n_problems; ++i) {
+        const vrl_int4_problem &q = problems[i];
+        const int rc = check_problem(q.x, q.qweight, q.scales, q.qzeros, q.y, q.M, q.N, q.K, q.G);
+        if (rc != VRL_INT4_OK) return rc;
+        if (q.prepacked || q.K != q0.K || q.G != q0.G || (q.fused_gate_up != 0) != fused || (fused && q.N % 2 != 0))
+            return VRL_INT4_ESHAPE;
+        if (q.K % 128 != 0 || q.G % 32 != 0 || !pow2(q.G)) return VRL_INT4_ELIMIT;
+        GemmRec &r = args.recs[i];
+        r.x = static_cast<const uint16_t *>(q.x);
+        r.qweight = static_cast<const uint32_t *>(q.qweight);
+        r.scales = static_cast<const uint16_t *>(q.scales);
+        r.qzeros = static_cast<const uint32_t *>(q.qzeros);
+        r.y = static_cast<uint16_t *>(q.y);
+        r.M = q.M;
+        r.N = q.N;
+    }
+    args.n = n_problems;
+    args.K = q0.K;
+    args.gshift = __builtin_ctz((unsigned)q0.G);
+    hipStream_t stream = reinterpret_cast<hipStream_t>(hip_stream);
+    return fused ? dispatch_gemm<true>(args, stream) : dispatch_gemm<false>(args, stream);
+}

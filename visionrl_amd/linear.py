@@ -21,14 +21,31 @@ from torch import nn
 from . import ops
 from .int4_format import check_packed, pack_nibbles, quantize_minmax
 
-# Calls with more activation rows than this (the prompt pass) rebuild the bf16 weight (bit-exact
-# tile, one launch) and hand the product to the library GEMM; the GEMV kernels are for decode.
+# Calls with more activation rows than this (the prompt pass) are matrix products; the GEMV kernels are for
+# decode.  Up to PROMPT_ROWS rows they go through the launch that rebuilds the weight in registers
+# (``ops.int4_gemm``: q|k|v of 512 rows by 2048 in 24 us against 3 x (7 + 12) us); beyond that, and wherever that
+# launch does not apply, the bf16 weight is rebuilt (bit-exact tile, one launch) and handed to the library GEMM,
+# whose rate makes up for the extra pass from there on (2048 x 5632 -> 2048: 55 against 7 + 47 us at 2048 rows,
+# 226 against 7 + 121 us at 8192).
 GEMM_ROWS = 32
+PROMPT_ROWS = 2048
+_PLAIN = (torch.Tensor, nn.Parameter)
 
 
 def _wants_grad(x: torch.Tensor) -> bool:
     """The HIP launches are not recorded by autograd: such calls take the dequant + GEMM route."""
     return torch.is_grad_enabled() and x.requires_grad
+
+
+def _launchable(x: torch.Tensor) -> bool:
+    """Whether a prompt-sized call may leave the torch operators: nothing watches them (a trace, a dispatch mode,
+    a functorch transform, forward-mode differentiation, an autocast to another type), and ``x`` is a plain
+    tensor.  The general route goes through ``F.linear`` and serves all of those."""
+    return type(x) in _PLAIN and x.is_cuda and not torch.jit.is_tracing() \
+        and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 \
+        and torch._C._functorch.peek_interpreter_stack() is None \
+        and torch.autograd.forward_ad._current_level < 0 \
+        and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
 
 
 def _version(t: torch.Tensor):
@@ -201,6 +218,25 @@ class Int4Linear(nn.Module):
             self._dense = kept
         return kept[1]
 
+    def _canonical(self):
+        return self.qweight, self.scales, self.qzeros
+
+    def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
+        """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
+        if rows.shape[0] > PROMPT_ROWS or getattr(self, "_keep_dense", False) or not _launchable(x):
+            return None
+        group, version = getattr(self, "_group", None), _version(x)
+        if group is not None and version is not None and all(
+                m.group_size == self.group_size and not getattr(m, "_keep_dense", False) for m in group[1:]):
+            ys = ops.int4_gemm(rows, [m._canonical() for m in group], self.group_size)
+            if ys is not None:
+                stream = torch.cuda.current_stream(x.device)
+                for m, ym in zip(group[1:], ys[1:]):
+                    m._handed = (x, version, ym, stream, _source_state(*m._canonical()))
+                return ys[0]
+        ys = ops.int4_gemm(rows, [self._canonical()], self.group_size)
+        return None if ys is None else ys[0]
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         rows = _rows(x, self.in_features)
         handed = getattr(self, "_handed", None)
@@ -214,7 +250,9 @@ class Int4Linear(nn.Module):
             y = ops.int4_gemv(rows, self.qweight, self.scales, self.qzeros, self.group_size)
         elif _wants_grad(x):
             y = F.linear(rows, self._dense_weight())
-        elif handed is not None and handed[0] is x and handed[1] == _version(x):
+        elif handed is not None and handed[0] is x and handed[1] == _version(x) and \
+                (len(handed) == 3 or (handed[3] == torch.cuda.current_stream(x.device) and
+                                      not _source_changed(handed[4], *self._canonical()))):
             y = handed[2]   # computed by the group leader's launch from this very tensor, unchanged since
         else:  # eager decode: skip the operator dispatcher, it costs more than the kernel
             packed = self._fresh_packed()
@@ -237,7 +275,9 @@ class Int4Linear(nn.Module):
                 packed = None
             if packed is None and M > GEMM_ROWS:
                 # prompt-sized call: the GEMV kernels would stream the weight once per 16 rows
-                y = F.linear(rows, self._dense_weight())
+                y = self._prompt_gemm(x, rows)
+                if y is None:
+                    y = F.linear(rows, self._dense_weight())
             elif packed is None:
                 y = torch.empty((M, self.out_features), dtype=torch.bfloat16, device=rows.device)
                 ops.int4_gemv_into(y, rows, self.qweight, self.scales, self.qzeros, self.group_size)
@@ -290,6 +330,10 @@ class Int4GateUpSiLU(nn.Module):
         if packed is not None and not grad and not torch.compiler.is_compiling() \
                 and rows.shape[0] <= self._direct_rows and packed.blob.device == rows.device:
             y = self._call(rows)[0]
+        elif not grad and GEMM_ROWS < rows.shape[0] <= PROMPT_ROWS and not torch.compiler.is_compiling() \
+                and not getattr(self, "_keep_dense", False) and _launchable(x) and \
+                (ys := ops.int4_gemm(rows, [(self.qweight, self.scales, self.qzeros)], self.group_size, True)):
+            y = ys[0]
         elif (grad or rows.shape[0] > GEMM_ROWS) and not torch.compiler.is_compiling():
             gate, up = F.linear(rows, self._dense_weight()).chunk(2, dim=-1)   # prompt-sized call: one library GEMM
             y = F.silu(gate) * up

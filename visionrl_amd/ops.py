@@ -23,7 +23,7 @@ import torch
 from . import _lib
 from .int4_format import check_packed
 
-__all__ = ["int4_gemv", "int4_dequant", "int4_gate_up_silu", "int4_gemv_into", "int4_prepack",
+__all__ = ["int4_gemv", "int4_dequant", "int4_gate_up_silu", "int4_gemv_into", "int4_gemm", "int4_prepack",
            "PrepackedWeight", "GroupedGemv", "DirectGemv", "int4_gemv_prepacked_into",
            "int4_gemv_prepacked_multi_into", "DirectCall", "cfg_sample", "head_sample", "head_sample_supported",
            "head_sample_workspace", "EpilogueGemv", "add_rmsnorm", "rope_attn_split_workspace",
@@ -122,6 +122,39 @@ def int4_gemv_into(y: torch.Tensor, x: torch.Tensor, qweight: torch.Tensor, scal
                                         _stream_handle(dev))
     _lib.check(rc, "vrl_int4_gemv_bf16")
     return y
+
+
+def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
+    """Prompt-sized products of one input with several canonical weights in one launch, or ``None``.
+
+    ``x`` is a contiguous bf16 ``[M, K]`` device tensor, ``weights`` a list of ``(qweight, scales, qzeros)``
+    triples of one group size (``fused``: gate||up triples, SiLU applied).  Returns one bf16 tensor per weight;
+    ``None`` for operands the launch has no build for (an odd group size, a misaligned view, scales that do not
+    fit its LDS), in which case nothing was enqueued and the caller takes its general route.
+    """
+    M, K = x.shape
+    dev, G = x.device, int(group_size)
+    groups = K // G
+    table = (_lib.Problem * len(weights))()
+    outs = []
+    for rec, (qweight, scales, qzeros) in zip(table, weights):
+        N = qweight.shape[0]
+        if qweight.dtype != torch.int32 or qzeros.dtype != torch.int32 or scales.dtype != torch.bfloat16 or \
+                qweight.shape != (N, K // 8) or scales.shape != (N, groups) or \
+                qzeros.shape != (N, (groups + 7) // 8) or \
+                any(t.device != dev or not t.is_contiguous() for t in (qweight, scales, qzeros)):
+            return None
+        y = torch.empty((M, N // 2 if fused else N), dtype=torch.bfloat16, device=dev)
+        rec.x, rec.y, rec.M, rec.N, rec.K, rec.G = x.data_ptr(), y.data_ptr(), M, N, K, G
+        rec.qweight, rec.scales, rec.qzeros = qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr()
+        rec.fused_gate_up = 1 if fused else 0
+        outs.append(y)
+    with _on(dev):
+        rc = _lib.load().vrl_int4_gemm_bf16(table, len(table), _stream_handle(dev))
+    if rc >= 1000:
+        return None
+    _lib.check(rc, "vrl_int4_gemm_bf16")
+    return outs
 
 
 @torch.library.custom_op("vrl_hip::int4_dequant", mutates_args=())
