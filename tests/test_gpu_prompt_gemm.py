@@ -78,7 +78,7 @@ def test_prompt_gemm_leaves_other_operands_to_the_general_route():
     triple = _triple(gen, 256, 32, 128, dev)
     shifted = flat[1:].view(64, 256)
     assert ops.int4_gemm(shifted, [triple], 128) is None                             # misaligned view
-    module = Int4Linear.from_packed(*triple, 128)
+    module = Int4Linear.from_packed(*_triple(gen, 256, 512, 128, dev), 128)
     assert torch.equal(module(shifted), torch.nn.functional.linear(shifted, module.dequantize()))
     big = _triple(gen, 16384, 40000, 32, dev)                                        # scales beyond LDS
     x = torch.randn(400, 16384, generator=gen).to(torch.bfloat16).to(dev)
@@ -88,7 +88,7 @@ def test_prompt_gemm_leaves_other_operands_to_the_general_route():
 @pytest.mark.gpu
 def test_prompt_calls_of_a_group_share_one_launch(monkeypatch):
     gen, dev = torch.Generator().manual_seed(5), torch.device("cuda:0")
-    q, k, v = (Int4Linear.from_packed(*_triple(gen, 256, n, 128, dev), 128).prepack_() for n in (256, 64, 64))
+    q, k, v = (Int4Linear.from_packed(*_triple(gen, 256, n, 128, dev), 128).prepack_() for n in (768, 512, 512))
     x = torch.randn(2, 50, 256, generator=gen).to(torch.bfloat16).to(dev)
     alone = [m(x) for m in (q, k, v)]
     q.group_with(k, v)
@@ -100,10 +100,10 @@ def test_prompt_calls_of_a_group_share_one_launch(monkeypatch):
     assert len(calls) == 1
     q(x)
     x.mul_(2)                                   # the input changed: nothing is handed over
-    assert torch.equal(k(x), real(x.view(100, 256), [k._canonical()], 128)[0].view(2, 50, 64))
+    assert torch.equal(k(x), real(x.view(100, 256), [k._canonical()], 128)[0].view(2, 50, 512))
     q(x)
     k.scales.mul_(2)                            # the sibling's weight changed
-    assert torch.equal(k(x), real(x.view(100, 256), [k._canonical()], 128)[0].view(2, 50, 64))
+    assert torch.equal(k(x), real(x.view(100, 256), [k._canonical()], 128)[0].view(2, 50, 512))
     side = torch.cuda.Stream()
     q(x)
     side.wait_stream(torch.cuda.current_stream())
@@ -118,7 +118,7 @@ def test_prompt_calls_of_a_group_share_one_launch(monkeypatch):
 def test_watched_prompt_calls_stay_on_the_general_route():
     """Transforms and modes see torch operators: a tangent, a batch dimension and a dispatch mode get through."""
     gen, dev = torch.Generator().manual_seed(7), torch.device("cuda:0")
-    m = Int4Linear.from_packed(*_triple(gen, 256, 64, 128, dev), 128)
+    m = Int4Linear.from_packed(*_triple(gen, 256, 512, 128, dev), 128)
     x, t = (torch.randn(40, 256, generator=gen).to(torch.bfloat16).to(dev) for _ in range(2))
     with torch.no_grad():
         dense = torch.nn.functional.linear(t, m.dequantize())
@@ -129,13 +129,13 @@ def test_watched_prompt_calls_stay_on_the_general_route():
         from torch.utils.flop_counter import FlopCounterMode
         with FlopCounterMode(display=False) as flops:
             m(x)
-        assert flops.get_total_flops() == 2 * 40 * 256 * 64
+        assert flops.get_total_flops() == 2 * 40 * 256 * 512
 
 
 @pytest.mark.gpu
 def test_prompt_gemm_replays_in_a_graph():
     gen, dev = torch.Generator().manual_seed(9), torch.device("cuda:0")
-    gate, up = (Int4Linear.from_packed(*_triple(gen, 256, 128, 128, dev), 128) for _ in range(2))
+    gate, up = (Int4Linear.from_packed(*_triple(gen, 256, 512, 128, dev), 128) for _ in range(2))
     mlp = Int4GateUpSiLU(gate, up)
     x = torch.randn(40, 256, generator=gen).to(torch.bfloat16).to(dev)
     with torch.no_grad():
@@ -150,6 +150,18 @@ def test_prompt_gemm_replays_in_a_graph():
             want = mlp(x)
             torch.cuda.synchronize()
             assert torch.equal(y, want)
+
+
+@pytest.mark.gpu
+def test_narrow_weights_stay_on_the_library_route(monkeypatch):
+    gen, dev = torch.Generator().manual_seed(11), torch.device("cuda:0")
+    narrow, wide = (Int4Linear.from_packed(*_triple(gen, 256, n, 128, dev), 128) for n in (511, 512))
+    x = torch.randn(40, 256, generator=gen).to(torch.bfloat16).to(dev)
+    calls, real = [], ops.int4_gemm
+    monkeypatch.setattr(linear_mod.ops, "int4_gemm", lambda *a: calls.append(1) or real(*a))
+    assert torch.equal(narrow(x), torch.nn.functional.linear(x, narrow.dequantize())) and not calls
+    wide(x)
+    assert len(calls) == 1
 
 
 def test_prompt_gemm_rejects_bad_calls():

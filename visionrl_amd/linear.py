@@ -27,8 +27,11 @@ from .int4_format import check_packed, pack_nibbles, quantize_minmax
 # launch does not apply, the bf16 weight is rebuilt (bit-exact tile, one launch) and handed to the library GEMM,
 # whose rate makes up for the extra pass from there on (2048 x 5632 -> 2048: 55 against 7 + 47 us at 2048 rows,
 # 226 against 7 + 121 us at 8192).
+# Weights of fewer than PROMPT_COLUMNS outputs stay on the library's route at every row count: rebuilding them
+# costs next to nothing, and their results are pinned bit for bit to the library's product.
 GEMM_ROWS = 32
 PROMPT_ROWS = 2048
+PROMPT_COLUMNS = 512
 _PLAIN = (torch.Tensor, nn.Parameter)
 
 
@@ -223,11 +226,13 @@ class Int4Linear(nn.Module):
 
     def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
         """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
-        if rows.shape[0] > PROMPT_ROWS or getattr(self, "_keep_dense", False) or not _launchable(x):
+        if rows.shape[0] > PROMPT_ROWS or self.out_features < PROMPT_COLUMNS or \
+                getattr(self, "_keep_dense", False) or not _launchable(x):
             return None
         group, version = getattr(self, "_group", None), _version(x)
         if group is not None and version is not None and all(
-                m.group_size == self.group_size and not getattr(m, "_keep_dense", False) for m in group[1:]):
+                m.group_size == self.group_size and m.out_features >= PROMPT_COLUMNS and
+                not getattr(m, "_keep_dense", False) for m in group[1:]):
             ys = ops.int4_gemm(rows, [m._canonical() for m in group], self.group_size)
             if ys is not None:
                 stream = torch.cuda.current_stream(x.device)
@@ -331,7 +336,8 @@ class Int4GateUpSiLU(nn.Module):
                 and rows.shape[0] <= self._direct_rows and packed.blob.device == rows.device:
             y = self._call(rows)[0]
         elif not grad and GEMM_ROWS < rows.shape[0] <= PROMPT_ROWS and not torch.compiler.is_compiling() \
-                and not getattr(self, "_keep_dense", False) and _launchable(x) and \
+                and self.intermediate_size >= PROMPT_COLUMNS and not getattr(self, "_keep_dense", False) \
+                and _launchable(x) and \
                 (ys := ops.int4_gemm(rows, [(self.qweight, self.scales, self.qzeros)], self.group_size, True)):
             y = ys[0]
         elif (grad or rows.shape[0] > GEMM_ROWS) and not torch.compiler.is_compiling():
