@@ -138,6 +138,17 @@ typedef struct vrl_int4_problem {
  */
 int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_problems, void *hip_stream);
 
+/*
+ * The middle of LlamaMLP over a product that is already there (act_fn(gate_proj(x)) * up_proj(x), policy.py:419-424):
+ * gate_up bf16 [M, 2 * inter] holds gate columns, then up columns.
+ *   y[m,i] = bf16( silu(gate) * up )                                     y bf16 [M, inter]
+ * and its gradient: grad_gate_up bf16 [M, 2 * inter] from gate_up and grad_y.  fp32 arithmetic, one rounding per
+ * result.  inter % 8 == 0, M * inter < 2^31.
+ */
+int vrl_silu_mul_bf16(const void *gate_up, void *y, int M, int inter, void *hip_stream);
+int vrl_silu_mul_backward_bf16(const void *gate_up, const void *grad_y, void *grad_gate_up, int M, int inter,
+                               void *hip_stream);
+
 typedef struct vrl_int4_plan_info {
     int32_t n_problems;    /* records in the blob */
     int32_t total_tiles;   /* 16-column output tiles over all problems */

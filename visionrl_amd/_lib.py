@@ -22,6 +22,8 @@ SYMBOLS = (
     "vrl_int4_dequant_bf16",
     "vrl_int4_gate_up_silu_bf16",
     "vrl_int4_gemm_bf16",
+    "vrl_silu_mul_bf16",
+    "vrl_silu_mul_backward_bf16",
     "vrl_int4_prepacked_bytes",
     "vrl_int4_prepack",
     "vrl_int4_gemv_prepacked_bf16",
@@ -231,6 +233,9 @@ def _bind(lib):
     lib.vrl_int4_dequant_bf16.argtypes = [vp, vp, vp, vp, ci, ci, ci, vp]
     lib.vrl_int4_gate_up_silu_bf16.restype = ci
     lib.vrl_int4_gate_up_silu_bf16.argtypes = [vp, vp, vp, vp, vp, ci, ci, ci, ci, vp]
+    lib.vrl_silu_mul_bf16.restype = lib.vrl_silu_mul_backward_bf16.restype = ci
+    lib.vrl_silu_mul_bf16.argtypes = [vp, vp, ci, ci, vp]
+    lib.vrl_silu_mul_backward_bf16.argtypes = [vp, vp, vp, ci, ci, vp]
     lib.vrl_int4_gemm_bf16.restype = ci
     lib.vrl_int4_gemm_bf16.argtypes = [ctypes.POINTER(Problem), ci, vp]
     lib.vrl_int4_prepacked_bytes.restype = ctypes.c_size_t

@@ -47,6 +47,7 @@ def _launchable(x: torch.Tensor) -> bool:
     return type(x) in _PLAIN and x.is_cuda and not torch.jit.is_tracing() \
         and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 \
         and torch._C._functorch.peek_interpreter_stack() is None \
+        and not torch._C._functorch.is_legacy_batchedtensor(x) \
         and torch.autograd.forward_ad._current_level < 0 \
         and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
 
@@ -295,6 +296,44 @@ class Int4Linear(nn.Module):
                 f"group_size={self.group_size}, bias={self.bias is not None}")
 
 
+def _silu_mul_ops(gate_up: torch.Tensor) -> torch.Tensor:
+    gate, up = gate_up.chunk(2, dim=-1)
+    return F.silu(gate) * up
+
+
+class _SiLUMul(torch.autograd.Function):
+    """``silu(gate) * up`` with its gradient as one launch each; only the product itself is saved.  A backward
+    that is itself recorded, or watched by a transform, goes through the torch operators."""
+
+    @staticmethod
+    def forward(ctx, gate_up):
+        ctx.save_for_backward(gate_up)
+        return ops.silu_mul(gate_up)
+
+    @staticmethod
+    def backward(ctx, grad):
+        gate_up, = ctx.saved_tensors
+        if torch.is_grad_enabled() or not (_launchable(grad) and _launchable(gate_up)):
+            recorded = torch.is_grad_enabled()
+            with torch.enable_grad():
+                return torch.autograd.grad(_silu_mul_ops(gate_up), gate_up, grad, create_graph=recorded)[0]
+        return ops.silu_mul_backward(gate_up, _aligned(grad))
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t`` itself if it is contiguous and starts on a 16-byte boundary, a copy otherwise."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
+    inter = gate_up.shape[-1] // 2
+    if not _launchable(gate_up) or gate_up.dtype != torch.bfloat16 or inter < PROMPT_COLUMNS or inter % 8 != 0 \
+            or gate_up.numel() >= 2 ** 31 or not gate_up.is_contiguous() or gate_up.data_ptr() % 16 != 0:
+        return _silu_mul_ops(gate_up)
+    return _SiLUMul.apply(gate_up) if _wants_grad(gate_up) else ops.silu_mul(gate_up)
+
+
 class Int4GateUpSiLU(nn.Module):
     """Fused ``silu(gate_proj(x)) * up_proj(x)`` over one packed gate||up operand."""
 
@@ -341,8 +380,7 @@ class Int4GateUpSiLU(nn.Module):
                 (ys := ops.int4_gemm(rows, [(self.qweight, self.scales, self.qzeros)], self.group_size, True)):
             y = ys[0]
         elif (grad or rows.shape[0] > GEMM_ROWS) and not torch.compiler.is_compiling():
-            gate, up = F.linear(rows, self._dense_weight()).chunk(2, dim=-1)   # prompt-sized call: one library GEMM
-            y = F.silu(gate) * up
+            y = _silu_mul(F.linear(rows, self._dense_weight()))   # prompt-sized call: one library GEMM
         else:
             y = ops.int4_gate_up_silu(rows, self.qweight, self.scales, self.qzeros, self.group_size)
         return y.reshape(*x.shape[:-1], self.intermediate_size)

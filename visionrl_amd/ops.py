@@ -23,7 +23,8 @@ import torch
 from . import _lib
 from .int4_format import check_packed
 
-__all__ = ["int4_gemv", "int4_dequant", "int4_gate_up_silu", "int4_gemv_into", "int4_gemm", "int4_prepack",
+__all__ = ["int4_gemv", "int4_dequant", "int4_gate_up_silu", "int4_gemv_into", "int4_gemm", "silu_mul",
+           "silu_mul_backward", "int4_prepack",
            "PrepackedWeight", "GroupedGemv", "DirectGemv", "int4_gemv_prepacked_into",
            "int4_gemv_prepacked_multi_into", "DirectCall", "cfg_sample", "head_sample", "head_sample_supported",
            "head_sample_workspace", "EpilogueGemv", "add_rmsnorm", "rope_attn_split_workspace",
@@ -155,6 +156,34 @@ def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
         return None
     _lib.check(rc, "vrl_int4_gemm_bf16")
     return outs
+
+
+def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
+    """``silu(gate) * up`` of a contiguous bf16 ``[M, 2 I]`` product (``I % 8 == 0``) in one launch."""
+    M, I = gate_up.shape[0], gate_up.shape[1] // 2
+    dev = _require_device("gate_up", gate_up)
+    if gate_up.dtype != torch.bfloat16:
+        raise TypeError(f"gate_up must be bfloat16, got {gate_up.dtype}")
+    y = torch.empty((M, I), dtype=torch.bfloat16, device=dev)
+    with _on(dev):
+        rc = _lib.load().vrl_silu_mul_bf16(gate_up.data_ptr(), y.data_ptr(), M, I, _stream_handle(dev))
+    _lib.check(rc, "vrl_silu_mul_bf16")
+    return y
+
+
+def silu_mul_backward(gate_up: torch.Tensor, grad: torch.Tensor) -> torch.Tensor:
+    """The gradient of :func:`silu_mul` with respect to ``gate_up``, in one launch."""
+    M, I = gate_up.shape[0], gate_up.shape[1] // 2
+    dev = _require_device("gate_up", gate_up)
+    _require_device("grad", grad, dev)
+    if gate_up.dtype != torch.bfloat16 or grad.dtype != torch.bfloat16 or grad.shape != (M, I):
+        raise ValueError(f"gate_up and grad must be bfloat16 [M, 2 I] and [M, I], got {tuple(grad.shape)}")
+    out = torch.empty_like(gate_up)
+    with _on(dev):
+        rc = _lib.load().vrl_silu_mul_backward_bf16(gate_up.data_ptr(), grad.data_ptr(), out.data_ptr(), M, I,
+                                                    _stream_handle(dev))
+    _lib.check(rc, "vrl_silu_mul_backward_bf16")
+    return out
 
 
 @torch.library.custom_op("vrl_hip::int4_dequant", mutates_args=())
