@@ -435,14 +435,18 @@ int vrl_int4_dequant_bf16(const void *qweight, const void *scales, const void *q
                           int N, int K, int G, void *hip_stream) {
     int rc = check_problem(qweight, qweight, scales, qzeros, w, 1, N, K, G);
     if (rc != VRL_INT4_OK) return rc;
-    const long total = (long)N * (K >> 3);
-    long blocks = (total + 255) / 256;
-    const long cap = (long)device_cu_count() * 32;
-    if (blocks > cap) blocks = cap;
+    // threads per row: the power of two that covers its words, 256 at most (then the row is cut into segments)
+    const int kwords = K >> 3;
+    int tshift = 0;
+    while (tshift < 8 && (1 << tshift) < kwords) ++tshift;
+    const long segments = (kwords + (1 << tshift) - 1) >> tshift, rows = DEQUANT_ROWS * (256 >> tshift);
+    const long blocks = (N + rows - 1) / rows * segments;
+    if (blocks >= (1L << 31)) return VRL_INT4_ESHAPE;
     return vrl_launch(&dequant_kernel, dim3((unsigned)blocks), dim3(256), 0,
                        reinterpret_cast<hipStream_t>(hip_stream),
                        static_cast<const uint32_t *>(qweight), static_cast<const uint16_t *>(scales),
-                       static_cast<const uint32_t *>(qzeros), static_cast<uint16_t *>(w), N, K, G);
+                       static_cast<const uint32_t *>(qzeros), static_cast<uint16_t *>(w), N, K, G, tshift,
+                       (int)segments);
 }
 
 size_t vrl_int4_prepacked_bytes(int N, int K, int G) {
