@@ -60,6 +60,9 @@ def _reference(x, triple, G, fused):
     (48, 96, 128, 32, True, 1),
     (1664, 2048, 512, 128, False, 3),   # more tiles than CUs
     (2047, 2 * 1500, 256, 256, True, 1),
+    (4100, 2 * 1700, 512, 64, True, 1), # 256x256 tiles, ragged both ways
+    (4090, 3500, 256, 128, False, 1),
+    (511, 16000, 384, 32, False, 2),
     (70, 128, 4096, 32, False, 1),      # the largest tables of scales
     (600, 2500, 5632, 32, False, 1),
 ])

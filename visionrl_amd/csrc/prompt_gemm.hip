@@ -42,8 +42,8 @@ struct GemmArgs {
 
 // One packed word -> eight exactly rounded bf16 weights in k order.  float(q) by the byte converter, then
 // fma(q, s, -z s): both products are exact (4 by 8 bits), so the sum is the exact (q - z) s and the conversion
-// is the one rounding of the contract.  Plain instructions, so that the compiler can issue them between MFMAs:
-// 23 against the 19 of the GEMV kernels' asm block, which cannot be split.
+// is the one rounding of the contract.  23 plain instructions that can be issued between MFMAs, pair by pair,
+// against 19 of the GEMV kernels' asm block, which cannot be split.
 struct ScaleZero { float s, zs; };
 
 __device__ __forceinline__ ScaleZero scale_zero(uint32_t meta) {   // (scale bits << 16) | zero
@@ -51,14 +51,17 @@ __device__ __forceinline__ ScaleZero scale_zero(uint32_t meta) {   // (scale bit
     return {s, -s * (float)(meta & 0xFFu)};
 }
 
-__device__ __forceinline__ bf16x8_t dequant_natural(uint32_t v, const ScaleZero &c) {
-    const uint32_t even = v & 0x0F0F0F0Fu, odd = (v >> 4) & 0x0F0F0F0Fu;
-    u32x4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        o[i] = pack_bf16_rne(__builtin_fmaf((float)((even >> (8 * i)) & 0xFFu), c.s, c.zs),
-                             __builtin_fmaf((float)((odd >> (8 * i)) & 0xFFu), c.s, c.zs));
-    return __builtin_bit_cast(bf16x8_t, o);
+struct Nibbles { uint32_t even, odd; };
+
+__device__ __forceinline__ Nibbles nibbles(uint32_t v) {
+    Nibbles b{v & 0x0F0F0F0Fu, (v >> 4) & 0x0F0F0F0Fu};
+    asm("" : "+v"(b.even), "+v"(b.odd));   // or the compiler takes every nibble out by itself: 28 instructions
+    return b;
+}
+
+__device__ __forceinline__ uint32_t dequant_pair(const Nibbles &b, int i, const ScaleZero &c) {
+    return pack_bf16_rne(__builtin_fmaf((float)((b.even >> (8 * i)) & 0xFFu), c.s, c.zs),
+                         __builtin_fmaf((float)((b.odd >> (8 * i)) & 0xFFu), c.s, c.zs));
 }
 
 // 16 bytes per lane from global memory to LDS at `lds` + 16 * lane; counted by vmcnt, touches no register.
@@ -119,7 +122,7 @@ __device__ __forceinline__ int weight_row(int r, int nt, int N) {
 }
 
 template <class C, bool FUSED>
-__global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 ? 2 : 1) void gemm_int4_kernel(GemmArgs args) {
+__global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 || C::MB * C::NB >= 32 ? 2 : 1) void gemm_int4_kernel(GemmArgs args) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -149,29 +152,32 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 ? 2 : 1) void gemm_int4_k
 
     uint32_t *table = reinterpret_cast<uint32_t *>(smem + C::S * C::STAGE);
 
-    // addresses of this wave's direct loads; a chunk is KC k further on
-    const uint8_t *xsrc[C::X_LOADS], *wsrc[C::W_LOADS];
+    // this wave's direct loads: byte offsets from the tile's first row and from the weight; a chunk is KC k further on
+    const uint8_t *xbase = reinterpret_cast<const uint8_t *>(p.x + (long)mt * C::BM * K);
+    const uint8_t *wbase = reinterpret_cast<const uint8_t *>(p.qweight);
+    uint32_t xsrc[C::X_LOADS], wsrc[C::W_LOADS];
 #pragma unroll
     for (int i = 0; i < C::X_LOADS; ++i) {
         const int at = (wave * C::X_LOADS + i) * 64 + lane;              // 16-byte piece of the staged tile
         const int r = at / C::XP, j = (at % C::XP) ^ activation_swizzle<C::XP, C::T>(r);
-        xsrc[i] = reinterpret_cast<const uint8_t *>(p.x + (long)min(mt * C::BM + r, p.M - 1) * K + 8 * j);
+        xsrc[i] = (uint32_t)(min(r, p.M - 1 - mt * C::BM) * K + 8 * j) * 2u;
     }
 #pragma unroll
     for (int i = 0; i < C::W_LOADS; ++i) {
         const int at = (wave * C::W_LOADS + i) % C::W_UNITS * 64 + lane;
         const int r = at / C::WP, j = (at % C::WP) ^ weight_swizzle<C::WP>(r);
-        wsrc[i] = reinterpret_cast<const uint8_t *>(p.qweight + (long)weight_row<C, FUSED>(r, nt, p.N) * kwords + 4 * j);
+        wsrc[i] = ((uint32_t)weight_row<C, FUSED>(r, nt, p.N) * (uint32_t)kwords + 4 * j) * 4u;   // below 4 GiB
     }
     const int chunks = K / C::KC;
     auto issue = [&](int chunk, int slot) {
         const long c = min(chunk, chunks - 1);   // past the end: a repeat nobody reads, so that every chunk counts alike
-        uint8_t *base = smem + slot * C::STAGE + wave * (C::X_LOADS * 1024);
+        const uint8_t *xc = xbase + c * (C::KC * 2), *wc = wbase + c * (C::KC / 2);
+        uint8_t *xl = smem + slot * C::STAGE + wave * (C::X_LOADS * 1024);
+        uint8_t *wl = smem + slot * C::STAGE + C::X_BYTES + wave * C::W_LOADS % C::W_UNITS * 1024;
 #pragma unroll
-        for (int i = 0; i < C::X_LOADS; ++i) dma16(base + i * 1024, xsrc[i] + c * (C::KC * 2));
-        uint8_t *wbase = smem + slot * C::STAGE + C::X_BYTES + wave * C::W_LOADS % C::W_UNITS * 1024;
+        for (int i = 0; i < C::X_LOADS; ++i) dma16(xl + i * 1024, xc + xsrc[i]);
 #pragma unroll
-        for (int i = 0; i < C::W_LOADS; ++i) dma16(wbase + i * 1024, wsrc[i] + c * (C::KC / 2));
+        for (int i = 0; i < C::W_LOADS; ++i) dma16(wl + i * 1024, wc + wsrc[i]);
     };
 
     // scales and zero-points of the tile's rows, (scale bits << 16) | zero, group-major
@@ -214,28 +220,51 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 ? 2 : 1) void gemm_int4_k
             for (int t = 0; t < C::T; ++t) w[n][t] = v[t];
             sz[n] = scale_zero(table[g * C::BN + wrow0 + 16 * n]);
         }
-        bf16x8_t xb[C::MB];
         auto fetch = [&](int t, int b) {
             return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t *>(
                 xs + b * (16 * C::KC * 2) + (((xpiece + t) ^ xswz) << 4)));
         };
+        bf16x8_t xb[C::MB];
 #pragma unroll
         for (int b = 0; b < C::MB; ++b) xb[b] = fetch(0, b);
         issue(c + C::S - 1, slot == 0 ? C::S - 1 : slot - 1);
-        // the next block's weights are rebuilt between this block's MFMAs, and the next step's activations are
-        // requested as soon as the last block has used this step's
-        bf16x8_t wa = dequant_natural(w[0][0], sz[0]);
+        // Row block by row block: its MFMAs, the request for its next activations, a share of the next step's
+        // weights.  The scheduler is kept to this order: by its own it requests activations right before they are
+        // used and rebuilds weights in one piece (a 128x128 tile of K = 5632 alone on its CU: 70.9 against 58.4 us,
+        // a 64x128 one 31.4 against 29.8; the smallest tile has nothing to gain, 15.4 against 16.6).
+        u32x4_t wa[C::NB];
 #pragma unroll
-        for (int i = 0; i < C::T * C::NB; ++i) {
-            const int t = i / C::NB, n = i % C::NB;
-            bf16x8_t next = wa;
-            if (i + 1 < C::T * C::NB) next = dequant_natural(w[(i + 1) % C::NB][(i + 1) / C::NB], sz[(i + 1) % C::NB]);
+        for (int n = 0; n < C::NB; ++n) {
+            const Nibbles q = nibbles(w[n][0]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wa[n][i] = dequant_pair(q, i, sz[n]);
+        }
+#pragma unroll
+        for (int t = 0; t < C::T; ++t) {
+            const bool last = t == C::T - 1;
+            constexpr int PAIRS = 4 * C::NB;
+            Nibbles q[C::NB];
+            u32x4_t next[C::NB];
 #pragma unroll
             for (int b = 0; b < C::MB; ++b) {
-                acc[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, xb[b], acc[b][n], 0, 0, 0);
-                if (n == C::NB - 1 && t + 1 < C::T) xb[b] = fetch(t + 1, b);
+#pragma unroll
+                for (int n = 0; n < C::NB; ++n)
+                    acc[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wa[n]), xb[b],
+                                                                        acc[b][n], 0, 0, 0);
+                if (!last) {
+                    xb[b] = fetch(t + 1, b);
+#pragma unroll
+                    for (int pair = b * PAIRS / C::MB; pair < (b + 1) * PAIRS / C::MB; ++pair) {
+                        const int n = pair / 4, i = pair % 4;
+                        if (i == 0) q[n] = nibbles(w[n][last ? 0 : t + 1]);
+                        next[n][i] = dequant_pair(q[n], i, sz[n]);
+                    }
+                }
+                if constexpr (C::MB > 2) __builtin_amdgcn_sched_barrier(0);
             }
-            wa = next;
+            if (!last)
+#pragma unroll
+                for (int n = 0; n < C::NB; ++n) wa[n] = next[n];
         }
         slot = slot + 1 == C::S ? 0 : slot + 1;
     }
@@ -348,15 +377,17 @@ bool gemm_one_round(GemmArgs &args, long cus) {
 using Gemm32x64 = GemmCfg<1, 4, 2, 2, 1, 256, 2>;
 using Gemm64x64 = GemmCfg<1, 4, 4, 4, 1, 256, 2>;
 using Gemm64x128 = GemmCfg<1, 4, 4, 4, 2, 256, 2>;
-using Gemm128x128Split = GemmCfg<1, 4, 2, 8, 2, 128, 3>;
+using Gemm128x128Split = GemmCfg<1, 4, 2, 8, 2, 128, 2>;
 using Gemm128x128 = GemmCfg<1, 4, 1, 8, 2, 64, 2>;
+using Gemm256x256 = GemmCfg<1, 8, 1, 16, 2, 64, 2>;
 
 // The smallest tile whose launch is one round of workgroups: until the chip is full a launch takes as long as one
-// tile does, and a smaller tile is done sooner (K = 2048, one round: 8.5 / 9.4 / 15.0 / 20.7 us in the order
-// below; its waves split K, since a tile alone on its CU is bound by the latency of its own chain).  Beyond that
-// the 128x128 tile whose waves split nothing, three or four workgroups per CU (25.2 us alone, but 60.7 us for
-// 1664 rows of q|k|v against 72.1 with the K split).  Measured at 48 to 1664 rows of q|k|v (3 x 2048), o_proj,
-// gate|up (11264) and down_proj (K = 5632): the rule's choice was the best or within 2 % of it at every one.
+// tile does, and a smaller tile is done sooner (K = 2048, one round: 7.7 / 9.5 / 14.0 / 21.0 us in the order
+// below; the waves split K, since a tile alone on its CU is bound by the latency of its own chain).  Beyond that
+// tiles whose waves split nothing: 256x256, every weight rebuilt once for 256 rows (1086 TFLOP/s for gate|up of
+// 8192 rows by 2048, against 975), where its rounds are at least 85 % full, 128x128 otherwise (gate|up of 1664
+// rows: 109 against 88 us; of 1280 rows: 62 against 76).  Measured at 48 to 8192 rows of q|k|v (3 x 2048),
+// o_proj, gate|up (11264) and down_proj (K = 5632): the choice is the best or within 5 % of it at every one.
 template <bool FUSED>
 int dispatch_gemm(GemmArgs &args, hipStream_t stream) {
     const long cus = device_cu_count();
@@ -366,6 +397,10 @@ int dispatch_gemm(GemmArgs &args, hipStream_t stream) {
     }
     if (gemm_one_round<Gemm64x128, FUSED>(args, cus)) return launch_gemm<Gemm64x128, FUSED>(args, stream);
     if (gemm_one_round<Gemm128x128Split, FUSED>(args, cus)) return launch_gemm<Gemm128x128Split, FUSED>(args, stream);
+    if (gemm_fits<Gemm256x256>(args)) {
+        const long tiles = gemm_tiles<Gemm256x256, FUSED>(args), rounds = (tiles + cus - 1) / cus;
+        if (tiles * 100 >= rounds * cus * 85) return launch_gemm<Gemm256x256, FUSED>(args, stream);
+    }
     return launch_gemm<Gemm128x128, FUSED>(args, stream);
 }
 
@@ -384,7 +419,7 @@ extern "C" int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_proble
         if (rc != VRL_INT4_OK) return rc;
         if (q.prepacked || q.K != q0.K || q.G != q0.G || (q.fused_gate_up != 0) != fused || (fused && q.N % 2 != 0))
             return VRL_INT4_ESHAPE;
-        if (q.K % 128 != 0 || q.G % 32 != 0 || !pow2(q.G)) return VRL_INT4_ELIMIT;
+        if (q.K % 128 != 0 || q.G % 32 != 0 || !pow2(q.G) || (long)q.N * q.K / 2 >= (1L << 32)) return VRL_INT4_ELIMIT;
         GemmRec &r = args.recs[i];
         r.x = static_cast<const uint16_t *>(q.x);
         r.qweight = static_cast<const uint32_t *>(q.qweight);

@@ -23,14 +23,18 @@ from .int4_format import check_packed, pack_nibbles, quantize_minmax
 
 # Calls with more activation rows than this (the prompt pass) are matrix products; the GEMV kernels are for
 # decode.  Up to PROMPT_ROWS rows they go through the launch that rebuilds the weight in registers
-# (``ops.int4_gemm``: q|k|v of 512 rows by 2048 in 24 us against 3 x (7 + 12) us); beyond that, and wherever that
+# (``ops.int4_gemm``: q|k|v of 512 rows by 2048 in 24 us against 3 x (4 + 12) us); beyond that, and wherever that
 # launch does not apply, the bf16 weight is rebuilt (bit-exact tile, one launch) and handed to the library GEMM,
-# whose rate makes up for the extra pass from there on (2048 x 5632 -> 2048: 55 against 7 + 47 us at 2048 rows,
-# 226 against 7 + 121 us at 8192).
+# whose rate makes up for the extra pass from there on (2048 x 5632 -> 2048: 54 against 6 + 48 us at 2048 rows,
+# 154 against 6 + 117 us at 8192).  gate|up goes back to the launch from FUSED_ROWS rows on where K is at most
+# FUSED_K: there SiLU's pass over the product costs more than the library's rate gains (2048 -> 2 x 5632: 164 us
+# against 120 + 10 + 21 at 3072 rows, 181 against 157 + 10 + 28 at 4096, 348 against 352 + 10 + 55 at 8192; the
+# pass is a smaller part of a longer K).
 # Weights of fewer than PROMPT_COLUMNS outputs stay on the library's route at every row count: rebuilding them
 # costs next to nothing, and their results are pinned bit for bit to the library's product.
 GEMM_ROWS = 32
 PROMPT_ROWS = 2048
+FUSED_ROWS, FUSED_K = 4096, 2048
 PROMPT_COLUMNS = 512
 _PLAIN = (torch.Tensor, nn.Parameter)
 
@@ -362,6 +366,15 @@ class Int4GateUpSiLU(nn.Module):
             self._call = ops.DirectCall([self._packed], fused=True)
         return self
 
+    def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
+        """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
+        M = rows.shape[0]
+        if not (GEMM_ROWS < M <= PROMPT_ROWS or M >= FUSED_ROWS and self.in_features <= FUSED_K) or \
+                self.intermediate_size < PROMPT_COLUMNS or getattr(self, "_keep_dense", False) or not _launchable(x):
+            return None
+        ys = ops.int4_gemm(rows, [(self.qweight, self.scales, self.qzeros)], self.group_size, True)
+        return None if ys is None else ys[0]
+
     packed_is_stale = Int4Linear.packed_is_stale
     _fresh_packed = Int4Linear._fresh_packed
     keep_dense_ = Int4Linear.keep_dense_
@@ -374,11 +387,8 @@ class Int4GateUpSiLU(nn.Module):
         if packed is not None and not grad and not torch.compiler.is_compiling() \
                 and rows.shape[0] <= self._direct_rows and packed.blob.device == rows.device:
             y = self._call(rows)[0]
-        elif not grad and GEMM_ROWS < rows.shape[0] <= PROMPT_ROWS and not torch.compiler.is_compiling() \
-                and self.intermediate_size >= PROMPT_COLUMNS and not getattr(self, "_keep_dense", False) \
-                and _launchable(x) and \
-                (ys := ops.int4_gemm(rows, [(self.qweight, self.scales, self.qzeros)], self.group_size, True)):
-            y = ys[0]
+        elif not grad and not torch.compiler.is_compiling() and (launched := self._prompt_gemm(x, rows)) is not None:
+            y = launched
         elif (grad or rows.shape[0] > GEMM_ROWS) and not torch.compiler.is_compiling():
             y = _silu_mul(F.linear(rows, self._dense_weight()))   # prompt-sized call: one library GEMM
         else:
