@@ -425,7 +425,7 @@ class NativeDecodeTrunk:
         """Enqueue the step on the current stream; returns the ``[rows, hidden]`` output buffer.  ``short``: the
         list :meth:`short_form` speaks of (the caller vouches that no row has as many cached slots as the split
         form begins at; the results are those of the default list either way, up to the order of fp32 sums)."""
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = ops._stream_handle(self.device)
         short = short and self._table_short is not None
         table, calls = (self._table_short, self._calls_short) if short else (self._table, self._calls)
         with ops._on(self.device):

@@ -89,7 +89,7 @@ def _rows(x: torch.Tensor, in_features: int) -> torch.Tensor:
         raise TypeError(f"Int4Linear runs in bfloat16 like the policy it replaces, got {x.dtype}")
     if x.shape[-1] != in_features:
         raise ValueError(f"last dimension {x.shape[-1]} != in_features {in_features}")
-    return x.reshape(-1, in_features).contiguous()
+    return x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, in_features).contiguous()
 
 
 class Int4Linear(nn.Module):
@@ -171,8 +171,8 @@ class Int4Linear(nn.Module):
 
     def _fresh_packed(self):
         """The prepacked copy, made again first if the canonical buffers changed under it."""
-        packed = getattr(self, "_packed", None)
-        if packed is not None and _source_changed(self._packed_from, self.qweight, self.scales, self.qzeros):
+        packed = self.__dict__.get("_packed")
+        if packed is not None and _source_changed(self._packed_from, *self._canonical()):
             if self.qweight.is_cuda and torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("the int4 weight changed after prepack_(): call prepack_() again before "
                                    "recording a graph over this module")
@@ -215,10 +215,11 @@ class Int4Linear(nn.Module):
         self._dense = None
         return self
 
-    def _dense_weight(self) -> torch.Tensor:
-        """The bf16 weight for a library GEMM: the kept copy if there is one and it is current."""
+    def _dense_weight(self, x: torch.Tensor) -> torch.Tensor:
+        """The bf16 weight for a library GEMM over ``x``: the kept copy if there is one and it is current."""
         if not getattr(self, "_keep_dense", False):
-            return ops.int4_dequant(self.qweight, self.scales, self.qzeros, self.group_size)
+            dequant = ops.dequant_eager if _launchable(x) else ops.int4_dequant
+            return dequant(*self._canonical(), self.group_size)
         kept = getattr(self, "_dense", None)
         if kept is None or _source_changed(kept[0], self.qweight, self.scales, self.qzeros):
             kept = (_source_state(self.qweight, self.scales, self.qzeros),
@@ -227,55 +228,63 @@ class Int4Linear(nn.Module):
         return kept[1]
 
     def _canonical(self):
-        return self.qweight, self.scales, self.qzeros
+        buffers = self._buffers   # (looked up through the module, a buffer costs three times as much)
+        try:
+            return buffers["qweight"], buffers["scales"], buffers["qzeros"]
+        except KeyError:          # replaced by plain attributes
+            return self.qweight, self.scales, self.qzeros
 
     def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
         """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
         if rows.shape[0] > PROMPT_ROWS or self.out_features < PROMPT_COLUMNS or \
                 getattr(self, "_keep_dense", False) or not _launchable(x):
             return None
-        group, version = getattr(self, "_group", None), _version(x)
-        if group is not None and version is not None and all(
+        group = self.__dict__.get("_group")
+        version = _version(x) if group is not None else None
+        if version is not None and all(
                 m.group_size == self.group_size and m.out_features >= PROMPT_COLUMNS and
-                not getattr(m, "_keep_dense", False) for m in group[1:]):
-            ys = ops.int4_gemm(rows, [m._canonical() for m in group], self.group_size)
+                not m.__dict__.get("_keep_dense", False) for m in group[1:]):
+            weights = [m._canonical() for m in group]
+            ys = ops.int4_gemm(rows, weights, self.group_size)
             if ys is not None:
-                stream = torch.cuda.current_stream(x.device)
-                for m, ym in zip(group[1:], ys[1:]):
-                    m._handed = (x, version, ym, stream, _source_state(*m._canonical()))
+                stream = ops._stream_handle(x.device)
+                for m, ym, weight in zip(group[1:], ys[1:], weights[1:]):
+                    m.__dict__["_handed"] = (x, version, ym, stream, _source_state(*weight))
                 return ys[0]
         ys = ops.int4_gemm(rows, [self._canonical()], self.group_size)
         return None if ys is None else ys[0]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         rows = _rows(x, self.in_features)
-        handed = getattr(self, "_handed", None)
-        if handed is not None:
-            self._handed = None
-        group = getattr(self, "_group", None)
-        if group is not None:   # a new call of the leader: whatever it handed over before is void
-            for m in group[1:]:
-                m._handed = None
         if torch.compiler.is_compiling():
             y = ops.int4_gemv(rows, self.qweight, self.scales, self.qzeros, self.group_size)
-        elif _wants_grad(x):
-            y = F.linear(rows, self._dense_weight())
+            return self._finish(y, x, rows)
+        own = self.__dict__   # plain attributes: nn.Module's own lookups and assignments cost microseconds
+        handed = own.get("_handed")
+        if handed is not None:
+            own["_handed"] = None
+        group = own.get("_group")
+        if group is not None:   # a new call of the leader: whatever it handed over before is void
+            for m in group[1:]:
+                m.__dict__["_handed"] = None
+        if _wants_grad(x):
+            y = F.linear(rows, self._dense_weight(x))
         elif handed is not None and handed[0] is x and handed[1] == _version(x) and \
-                (len(handed) == 3 or (handed[3] == torch.cuda.current_stream(x.device) and
+                (len(handed) == 3 or (handed[3] == ops._stream_handle(x.device) and
                                       not _source_changed(handed[4], *self._canonical()))):
             y = handed[2]   # computed by the group leader's launch from this very tensor, unchanged since
         else:  # eager decode: skip the operator dispatcher, it costs more than the kernel
             packed = self._fresh_packed()
             M = rows.shape[0]
             if packed is not None and packed.blob.device == rows.device:
-                call = getattr(self, "_group_call", None)
+                call = own.get("_group_call")
                 version = _version(x) if call is not None else None
                 if call is not None and M <= call.max_rows and version is not None and \
                         not any(m.packed_is_stale() for m in group[1:]):
                     # (an input without a modification counter cannot be recognised later: no hand-over)
                     ys = call(rows)
                     for m, ym in zip(group[1:], ys[1:]):
-                        m._handed = (x, version, ym)
+                        m.__dict__["_handed"] = (x, version, ym)
                     y = ys[0]
                 elif M <= self._direct_rows:
                     y = self._call(rows)[0]
@@ -287,13 +296,16 @@ class Int4Linear(nn.Module):
                 # prompt-sized call: the GEMV kernels would stream the weight once per 16 rows
                 y = self._prompt_gemm(x, rows)
                 if y is None:
-                    y = F.linear(rows, self._dense_weight())
+                    y = F.linear(rows, self._dense_weight(x))
             elif packed is None:
                 y = torch.empty((M, self.out_features), dtype=torch.bfloat16, device=rows.device)
                 ops.int4_gemv_into(y, rows, self.qweight, self.scales, self.qzeros, self.group_size)
+        return self._finish(y, x, rows)
+
+    def _finish(self, y: torch.Tensor, x: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
         if self.bias is not None:
             y = y + self.bias
-        return y.reshape(*x.shape[:-1], self.out_features)
+        return y if rows is x else y.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, "
@@ -372,9 +384,10 @@ class Int4GateUpSiLU(nn.Module):
         if not (GEMM_ROWS < M <= PROMPT_ROWS or M >= FUSED_ROWS and self.in_features <= FUSED_K) or \
                 self.intermediate_size < PROMPT_COLUMNS or getattr(self, "_keep_dense", False) or not _launchable(x):
             return None
-        ys = ops.int4_gemm(rows, [(self.qweight, self.scales, self.qzeros)], self.group_size, True)
+        ys = ops.int4_gemm(rows, [self._canonical()], self.group_size, True)
         return None if ys is None else ys[0]
 
+    _canonical = Int4Linear._canonical
     packed_is_stale = Int4Linear.packed_is_stale
     _fresh_packed = Int4Linear._fresh_packed
     keep_dense_ = Int4Linear.keep_dense_
@@ -390,10 +403,10 @@ class Int4GateUpSiLU(nn.Module):
         elif not grad and not torch.compiler.is_compiling() and (launched := self._prompt_gemm(x, rows)) is not None:
             y = launched
         elif (grad or rows.shape[0] > GEMM_ROWS) and not torch.compiler.is_compiling():
-            y = _silu_mul(F.linear(rows, self._dense_weight()))   # prompt-sized call: one library GEMM
+            y = _silu_mul(F.linear(rows, self._dense_weight(x)))   # prompt-sized call: one library GEMM
         else:
             y = ops.int4_gate_up_silu(rows, self.qweight, self.scales, self.qzeros, self.group_size)
-        return y.reshape(*x.shape[:-1], self.intermediate_size)
+        return y if rows is x else y.reshape(*x.shape[:-1], self.intermediate_size)
 
 
 class Int4LlamaMLP(nn.Module):

@@ -32,7 +32,8 @@ __all__ = ["int4_gemv", "int4_dequant", "int4_gate_up_silu", "int4_gemv_into", "
 
 
 def _stream_handle(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream of ``device`` as the library takes it (no stream object is built: 3 us of a call)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 _NULL = contextlib.nullcontext()
@@ -40,7 +41,7 @@ _NULL = contextlib.nullcontext()
 
 def _on(device: torch.device):
     """Context that makes ``device`` current; free when it already is (the decode-loop case)."""
-    if device.index is None or torch.cuda.current_device() == device.index:
+    if device.index is None or torch._C._cuda_getDevice() == device.index:
         return _NULL
     return torch.cuda.device(device)
 
@@ -78,7 +79,7 @@ def int4_gemv(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     M, N, K, dev = _check_call(x, qweight, scales, qzeros, group_size)
     lib = _lib.load()
     y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.vrl_int4_gemv_bf16(x.data_ptr(), qweight.data_ptr(), scales.data_ptr(),
                                     qzeros.data_ptr(), y.data_ptr(), M, N, K, int(group_size),
                                     _stream_handle(dev))
@@ -135,23 +136,24 @@ def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
     """
     M, K = x.shape
     dev, G = x.device, int(group_size)
-    groups = K // G
+    words, groups = K // 8, K // G
+    zwords = (groups + 7) // 8
     table = (_lib.Problem * len(weights))()
-    outs = []
+    xp, flag, outs = x.data_ptr(), 1 if fused else 0, []
     for rec, (qweight, scales, qzeros) in zip(table, weights):
         N = qweight.shape[0]
         if qweight.dtype != torch.int32 or qzeros.dtype != torch.int32 or scales.dtype != torch.bfloat16 or \
-                qweight.shape != (N, K // 8) or scales.shape != (N, groups) or \
-                qzeros.shape != (N, (groups + 7) // 8) or \
-                any(t.device != dev or not t.is_contiguous() for t in (qweight, scales, qzeros)):
+                qweight.shape != (N, words) or scales.shape != (N, groups) or qzeros.shape != (N, zwords) or \
+                not (qweight.is_contiguous() and scales.is_contiguous() and qzeros.is_contiguous()) or \
+                not (qweight.device == dev and scales.device == dev and qzeros.device == dev):
             return None
         y = torch.empty((M, N // 2 if fused else N), dtype=torch.bfloat16, device=dev)
-        rec.x, rec.y, rec.M, rec.N, rec.K, rec.G = x.data_ptr(), y.data_ptr(), M, N, K, G
-        rec.qweight, rec.scales, rec.qzeros = qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr()
-        rec.fused_gate_up = 1 if fused else 0
+        rec.x, rec.qweight, rec.scales, rec.qzeros, rec.y = \
+            xp, qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), y.data_ptr()
+        rec.M, rec.N, rec.K, rec.G, rec.fused_gate_up = M, N, K, G, flag
         outs.append(y)
     with _on(dev):
-        rc = _lib.load().vrl_int4_gemm_bf16(table, len(table), _stream_handle(dev))
+        rc = _lib.load().vrl_int4_gemm_bf16(table, len(outs), _stream_handle(dev))
     if rc >= 1000:
         return None
     _lib.check(rc, "vrl_int4_gemm_bf16")
@@ -186,20 +188,26 @@ def silu_mul_backward(gate_up: torch.Tensor, grad: torch.Tensor) -> torch.Tensor
     return out
 
 
-@torch.library.custom_op("vrl_hip::int4_dequant", mutates_args=())
-def int4_dequant(qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
-                 group_size: int) -> torch.Tensor:
+def dequant_eager(qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
+                  group_size: int) -> torch.Tensor:
+    """``int4_dequant`` without the operator dispatcher, which costs an eager call more than the kernel does."""
     N, K, _ = check_packed(qweight, scales, qzeros, group_size)
     dev = _require_device("qweight", qweight)
     _require_device("scales", scales, dev)
     _require_device("qzeros", qzeros, dev)
     lib = _lib.load()
     w = torch.empty((N, K), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.vrl_int4_dequant_bf16(qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(),
                                        w.data_ptr(), N, K, int(group_size), _stream_handle(dev))
     _lib.check(rc, "vrl_int4_dequant_bf16")
     return w
+
+
+@torch.library.custom_op("vrl_hip::int4_dequant", mutates_args=())
+def int4_dequant(qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
+                 group_size: int) -> torch.Tensor:
+    return dequant_eager(qweight, scales, qzeros, group_size)
 
 
 @int4_dequant.register_fake
@@ -216,7 +224,7 @@ def int4_gate_up_silu(x: torch.Tensor, qweight_gu: torch.Tensor, scales_gu: torc
     inter = N2 // 2
     lib = _lib.load()
     y = torch.empty((M, inter), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.vrl_int4_gate_up_silu_bf16(x.data_ptr(), qweight_gu.data_ptr(), scales_gu.data_ptr(),
                                             qzeros_gu.data_ptr(), y.data_ptr(), M, inter, K,
                                             int(group_size), _stream_handle(dev))
@@ -279,7 +287,7 @@ def int4_prepack(qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tens
         raise ValueError(f"no prepacked form for N={N}, K={K}, group_size={group_size} "
                          "(needs group_size 128)")
     blob = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.vrl_int4_prepack(qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(),
                                   blob.data_ptr(), N, K, int(group_size), _stream_handle(dev))
     _lib.check(rc, "vrl_int4_prepack")
@@ -784,7 +792,7 @@ class DirectCall:
             rec = self.table[0]
             rec.x, rec.y, rec.M = x2d.data_ptr(), y.data_ptr(), M
             with _on(self.device):
-                rc = self._fn(self.table, 1, torch.cuda.current_stream(self.device).cuda_stream)
+                rc = self._fn(self.table, 1, _stream_handle(self.device))
             if rc:
                 _lib.check(rc, "vrl_int4_gemv_prepacked_bf16")
             return [y]
@@ -797,7 +805,7 @@ class DirectCall:
             outs.append(buf[off:off + M * c].view(M, c))
             off += size
         with _on(self.device):
-            rc = self._fn(self.table, self._n, torch.cuda.current_stream(self.device).cuda_stream)
+            rc = self._fn(self.table, self._n, _stream_handle(self.device))
         if rc:
             _lib.check(rc, "vrl_int4_gemv_prepacked_bf16")
         return outs
