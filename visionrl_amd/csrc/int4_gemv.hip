@@ -964,33 +964,50 @@ int vrl_int4_grouped_plan_build(const vrl_int4_problem *problems, int n_problems
         // pays for its stagings and barriers on top (measured: the workgroups that hold such tiles
         // ended 28 % after the others at equal weight; 1.45 is the best of a sweep from 1.0 to 2.4 on
         // the 1B set at 32 rows, and is worth 7-8 % on the 7B-class sets at 8 and 16 rows)
-        const double pass_factor = 1.45;
+        auto in_passes = [&](const DevProblem &p) { return p.prepacked && p.kc < pp_nsc(p.K) * PP_SC; };
+        double pass_factor = 1.45;
         auto tile_cost = [&](const DevProblem &p) {
-            const bool passes = p.prepacked && p.kc < pp_nsc(p.K) * PP_SC;
-            return ((double)p.K * (p.fused ? 2 : 1) + 512.0) * (passes ? pass_factor : 1.0);
+            return ((double)p.K * (p.fused ? 2 : 1) + 512.0) * (in_passes(p) ? pass_factor : 1.0);
         };
-        for (int i = 0; i < n_problems; ++i) {
-            const DevProblem &p = recs[i];
-            total_cost += (double)(((p.fused ? p.N / 2 : p.N) + 15) / 16) * tile_cost(p);
+        auto plan_cost = [&] {
+            double sum = 0.0;
+            for (int i = 0; i < n_problems; ++i)
+                sum += (double)(((recs[i].fused ? recs[i].N / 2 : recs[i].N) + 15) / 16) * tile_cost(recs[i]);
+            return sum;
+        };
+        total_cost = plan_cost();
+        // A record walked in staged passes deals its tiles to the waves in lock-step, one per wave at a time: a
+        // range inside it is cut at a multiple of the workgroup's waves.  In a plan of few tiles such a piece is
+        // more than a workgroup's share and the launch waits for it: then half as many tiles, which cost more
+        // each (half the waves share a staging; three layers of 2048 x 5632 at 32 rows 42.7 against 32.0 us,
+        // four at 24 rows 42.7 against 36.2; from a share of 5/8 of a piece on whole pieces are as good or
+        // better: 60.8 against 65.4 us for seven layers and the head at 24 rows).
+        int pass_cut = wpb;
+        for (int i = 0; i < n_problems; ++i)
+            if (in_passes(recs[i]) && wpb * tile_cost(recs[i]) > 1.6 * total_cost / (double)grid) pass_cut = wpb / 2;
+        if (pass_cut < wpb) {
+            pass_factor = 1.8;
+            total_cost = plan_cost();
         }
+        // A range ends at the cut nearest to its share of what is left, so that one that had to take more than its
+        // share does not leave a neighbour empty, and one whose piece is just short of it does not take two.
         int b = 0;
-        double acc_cost = 0.0;
+        double left = total_cost, held = 0.0;   // cost from the current range on, cost it holds so far
         block_begin[0] = 0;
         for (int i = 0; i < n_problems; ++i) {
             const DevProblem &p = recs[i];
             const int out_cols = p.fused ? p.N / 2 : p.N;
             const int nt = (out_cols + 15) / 16;
             const double c = tile_cost(p);
-            // a record walked in staged passes deals its tiles to the waves in lock-step, one per
-            // wave at a time: a range inside it is cut at a multiple of the workgroup's waves
-            const int cut = (p.prepacked && p.kc < pp_nsc(p.K) * PP_SC) ? wpb : 1;
+            const int cut = in_passes(p) ? pass_cut : 1;
             for (int t = 0; t < nt; ++t) {
-                // tile (p.tile_begin + t) starts block b+1 once the blocks so far hold their share
-                while (b + 1 < grid && t % cut == 0 && acc_cost >= total_cost * (b + 1) / (double)grid) {
-                    ++b;
-                    block_begin[b] = p.tile_begin + t;
+                if (b + 1 < grid && t % cut == 0 && held > 0.0 &&
+                    held + 0.5 * c * std::min(cut, nt - t) >= left / (double)(grid - b)) {
+                    left -= held;
+                    held = 0.0;
+                    block_begin[++b] = p.tile_begin + t;
                 }
-                acc_cost += c;
+                held += c;
             }
         }
         while (b < grid) {
