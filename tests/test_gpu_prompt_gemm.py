@@ -6,21 +6,12 @@ the fused form carries both operands' sums through ``silu(g) * u`` (|silu'| < 1.
 """
 
 import ctypes
-import gc
-
 import pytest
 import torch
 
 from visionrl_amd import _lib, ops
 from visionrl_amd import linear as linear_mod
 from visionrl_amd.linear import Int4GateUpSiLU, Int4Linear
-
-
-@pytest.fixture(autouse=True)
-def _collect_cycles():
-    """Grouped modules and graphs hold GPU tensors in cycles: a later test's memory account is its own."""
-    yield
-    gc.collect()
 
 
 def _triple(gen, K, N, G, dev):

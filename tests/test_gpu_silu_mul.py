@@ -4,20 +4,11 @@ Tolerance: one bf16 rounding (2^-8 relative covers it) and 2^-17 of the terms' m
 fp32 products; where exp leaves fp32 (|gate| > 88) the result is below 2^-118 and may be zero.
 """
 
-import gc
-
 import pytest
 import torch
 
 from visionrl_amd import _lib, ops
 from visionrl_amd.linear import Int4GateUpSiLU, Int4Linear, _silu_mul, _silu_mul_ops
-
-
-@pytest.fixture(autouse=True)
-def _collect_cycles():
-    """Grouped modules and graphs hold GPU tensors in cycles: a later test's memory account is its own."""
-    yield
-    gc.collect()
 
 
 @pytest.mark.gpu
