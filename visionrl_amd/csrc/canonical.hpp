@@ -68,8 +68,8 @@ __device__ __forceinline__ void dequant_word(uint32_t v, const GroupConst &g, ui
 // dequant: one thread per packed word of four rows, natural k order out
 // -------------------------------------------------------------------------
 // A wave's loads and 16-byte stores are contiguous; the four rows' loads are independent, which is what keeps
-// enough of them in flight (one word per thread and a 64-bit division for its row: 6.0 us for 2048 x 2048, 8.4 for
-// 2048 x 5632, 14.2 for 11264 x 2048).  A block covers one of
+// enough of them in flight (2048 x 2048 / 2048 x 5632 / 11264 x 2048: 4.0 / 6.5 / 10.4 us against 4.5 / 7.8 / 11.8
+// with one word per thread and a 64-bit division for its row).  A block covers one of
 // the `segments` of a row, 1 << tshift words; threads beyond that are on the next rows.
 constexpr int DEQUANT_ROWS = 4;
 

@@ -989,8 +989,11 @@ int vrl_int4_grouped_plan_build(const vrl_int4_problem *problems, int n_problems
             pass_factor = 1.8;
             total_cost = plan_cost();
         }
-        // A range ends at the cut nearest to its share of what is left, so that one that had to take more than its
-        // share does not leave a neighbour empty, and one whose piece is just short of it does not take two.
+        // With such pieces a range ends at the cut nearest to its share of what is left, so that one that had to take
+        // more than its share does not leave a neighbour empty, and one whose piece is just short of it does not
+        // take two (eight layers and the head at 32 rows: 79.4 against 61.4 us).  Plans without them are cut tile by
+        // tile where the ranges so far hold their share (nearest cuts: 46.4 against 44.7 us for nine layers at one row).
+        const bool pieces = std::any_of(recs, recs + n_problems, in_passes);
         int b = 0;
         double left = total_cost, held = 0.0;   // cost from the current range on, cost it holds so far
         block_begin[0] = 0;
@@ -1000,9 +1003,12 @@ int vrl_int4_grouped_plan_build(const vrl_int4_problem *problems, int n_problems
             const int nt = (out_cols + 15) / 16;
             const double c = tile_cost(p);
             const int cut = in_passes(p) ? pass_cut : 1;
+            auto full = [&](int t) {
+                if (!pieces) return total_cost - left + held >= total_cost * (b + 1) / (double)grid;
+                return held > 0.0 && held + 0.5 * c * std::min(cut, nt - t) >= left / (double)(grid - b);
+            };
             for (int t = 0; t < nt; ++t) {
-                if (b + 1 < grid && t % cut == 0 && held > 0.0 &&
-                    held + 0.5 * c * std::min(cut, nt - t) >= left / (double)(grid - b)) {
+                while (b + 1 < grid && t % cut == 0 && full(t)) {
                     left -= held;
                     held = 0.0;
                     block_begin[++b] = p.tile_begin + t;
