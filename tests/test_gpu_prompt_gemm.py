@@ -187,3 +187,15 @@ def test_prompt_gemm_rejects_bad_calls():
     assert call(2, K=512) == 1001 and call(2, G=64) == 1001 and call(2, fused_gate_up=1) == 1001
     assert call(N=33, fused_gate_up=1) == 1001
     assert call(K=264, G=8) == 1005 and call(K=192, G=64) == 1005 and call(K=384, G=96) == 1005
+
+
+def test_prompt_gemm_refuses_inputs_it_would_misread(monkeypatch):
+    """The library is handed an address: what lies there is bf16, dense and on the device, or the call ends here."""
+    monkeypatch.setattr(ops._lib, "load", lambda: pytest.fail("the library was reached"))
+    triple = _triple(torch.Generator().manual_seed(1), 256, 32, 128, "cpu")
+    x = torch.zeros(64, 256, dtype=torch.bfloat16)
+    for bad, error in ((x, ValueError), (x.half(), TypeError), (x.float(), TypeError), (x[None], ValueError),
+                       (torch.zeros(64, 512, dtype=torch.bfloat16)[:, ::2], ValueError),
+                       (x[:1].expand(64, 256), ValueError)):
+        with pytest.raises(error):
+            ops.int4_gemm(bad, [triple], 128)

@@ -84,3 +84,22 @@ def test_silu_mul_rejects_bad_calls():
     assert lib.vrl_silu_mul_bf16(p, p + 8, 1, 8, None) == 1002
     assert lib.vrl_silu_mul_backward_bf16(p, None, p, 1, 8, None) == 1003
     assert lib.vrl_silu_mul_backward_bf16(p, p, p, 1 << 20, 1 << 11, None) == 1001
+
+
+def test_silu_mul_refuses_products_it_would_misread(monkeypatch):
+    """An odd width would shift every row after the first; half, strided and host tensors are refused alike."""
+    monkeypatch.setattr(ops._lib, "load", lambda: pytest.fail("the library was reached"))
+    gu, grad = torch.zeros(4, 32, dtype=torch.bfloat16), torch.zeros(4, 16, dtype=torch.bfloat16)
+    wide = torch.zeros(4, 64, dtype=torch.bfloat16)
+    for bad, error in ((gu, ValueError), (gu.half(), TypeError), (wide[:, ::2], ValueError), (gu[None], ValueError),
+                       (torch.zeros(4, 33, dtype=torch.bfloat16), ValueError)):
+        with pytest.raises(error):
+            ops.silu_mul(bad)
+        with pytest.raises(error):
+            ops.silu_mul_backward(bad, grad)
+    for bad in (grad.half(), grad[:, :8], grad[:2]):
+        with pytest.raises(ValueError):
+            ops.silu_mul_backward(gu, bad)
+    # the checks in their order: the odd width is what stops a device tensor of it
+    with pytest.raises(ValueError, match="odd width"):
+        ops.silu_mul(torch.zeros(4, 33, dtype=torch.bfloat16))

@@ -57,6 +57,15 @@ def _require_device(name: str, t: torch.Tensor, device: torch.device | None = No
     return t.device
 
 
+def _require_rows(name: str, t: torch.Tensor) -> None:
+    if t.dtype != torch.bfloat16:
+        raise TypeError(f"{name} must be bfloat16, got {t.dtype}")
+    if t.dim() != 2:
+        raise ValueError(f"{name} must be two-dimensional, got {list(t.shape)}")
+    if not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous")
+
+
 def _check_call(x, qweight, scales, qzeros, group_size):
     if x.dtype != torch.bfloat16:
         raise TypeError(f"x must be bfloat16, got {x.dtype}")
@@ -132,10 +141,12 @@ def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
     ``x`` is a contiguous bf16 ``[M, K]`` device tensor, ``weights`` a list of ``(qweight, scales, qzeros)``
     triples of one group size (``fused``: gate||up triples, SiLU applied).  Returns one bf16 tensor per weight;
     ``None`` for operands the launch has no build for (an odd group size, a misaligned view, scales that do not
-    fit its LDS), in which case nothing was enqueued and the caller takes its general route.
+    fit its LDS), in which case nothing was enqueued and the caller takes its general route.  Another ``x`` is
+    refused: the launch reads ``M * K`` bf16 values from its address.
     """
+    _require_rows("x", x)
     M, K = x.shape
-    dev, G = x.device, int(group_size)
+    dev, G = _require_device("x", x), int(group_size)
     words, groups = K // 8, K // G
     zwords = (groups + 7) // 8
     table = (_lib.Problem * len(weights))()
@@ -160,12 +171,18 @@ def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
     return outs
 
 
+def _halves(gate_up: torch.Tensor) -> tuple[int, int]:
+    """``(M, I)`` of a bf16 ``[M, 2 I]`` product."""
+    _require_rows("gate_up", gate_up)
+    if gate_up.shape[1] % 2:
+        raise ValueError(f"gate_up holds gate and up columns side by side, got an odd width {gate_up.shape[1]}")
+    return gate_up.shape[0], gate_up.shape[1] // 2
+
+
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` of a contiguous bf16 ``[M, 2 I]`` product (``I % 8 == 0``) in one launch."""
-    M, I = gate_up.shape[0], gate_up.shape[1] // 2
+    M, I = _halves(gate_up)
     dev = _require_device("gate_up", gate_up)
-    if gate_up.dtype != torch.bfloat16:
-        raise TypeError(f"gate_up must be bfloat16, got {gate_up.dtype}")
     y = torch.empty((M, I), dtype=torch.bfloat16, device=dev)
     with _on(dev):
         rc = _lib.load().vrl_silu_mul_bf16(gate_up.data_ptr(), y.data_ptr(), M, I, _stream_handle(dev))
@@ -175,11 +192,11 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 def silu_mul_backward(gate_up: torch.Tensor, grad: torch.Tensor) -> torch.Tensor:
     """The gradient of :func:`silu_mul` with respect to ``gate_up``, in one launch."""
-    M, I = gate_up.shape[0], gate_up.shape[1] // 2
+    M, I = _halves(gate_up)
+    if grad.dtype != torch.bfloat16 or grad.shape != (M, I):
+        raise ValueError(f"grad must be bfloat16 {[M, I]}, got {grad.dtype} {list(grad.shape)}")
     dev = _require_device("gate_up", gate_up)
     _require_device("grad", grad, dev)
-    if gate_up.dtype != torch.bfloat16 or grad.dtype != torch.bfloat16 or grad.shape != (M, I):
-        raise ValueError(f"gate_up and grad must be bfloat16 [M, 2 I] and [M, I], got {tuple(grad.shape)}")
     out = torch.empty_like(gate_up)
     with _on(dev):
         rc = _lib.load().vrl_silu_mul_backward_bf16(gate_up.data_ptr(), grad.data_ptr(), out.data_ptr(), M, I,
