@@ -72,6 +72,20 @@ def test_replay_of_the_fused_module_matches_the_explicit_product():
     assert rel(got, want) < 2.0 ** -7 and rel(x.grad, ref.grad) < 2.0 ** -6     # bf16 results, three of them in a row
 
 
+@pytest.mark.gpu
+def test_an_empty_batch_passes_forward_and_backward():
+    gen, dev = torch.Generator().manual_seed(4), torch.device("cuda:0")
+    linear = lambda: Int4Linear.from_linear(torch.nn.Linear(256, 512, bias=False).to(torch.bfloat16).to(dev), 128)
+    mlp, proj = Int4GateUpSiLU(linear(), linear()), linear()
+    for shape in ((0, 256), (2, 0, 256)):
+        for module in (mlp, proj):
+            x = torch.randn(shape, generator=gen).to(torch.bfloat16).to(dev).requires_grad_()
+            y = module(x)
+            assert y.shape == (*shape[:-1], 512)
+            y.float().sum().backward()
+            assert x.grad.shape == x.shape
+
+
 def test_silu_mul_rejects_bad_calls():
     import ctypes
 

@@ -345,7 +345,7 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 def _silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     inter = gate_up.shape[-1] // 2
     if not _launchable(gate_up) or gate_up.dtype != torch.bfloat16 or inter < PROMPT_COLUMNS or inter % 8 != 0 \
-            or gate_up.numel() >= 2 ** 31 or not gate_up.is_contiguous() or gate_up.data_ptr() % 16 != 0:
+            or not 0 < gate_up.numel() < 2 ** 31 or not gate_up.is_contiguous() or gate_up.data_ptr() % 16 != 0:
         return _silu_mul_ops(gate_up)
     return _SiLUMul.apply(gate_up) if _wants_grad(gate_up) else ops.silu_mul(gate_up)
 
