@@ -73,6 +73,26 @@ def test_replay_of_the_fused_module_matches_the_explicit_product():
 
 
 @pytest.mark.gpu
+def test_saved_tensor_hooks_may_hand_back_views():
+    """A strided view, and one that starts between 16-byte boundaries: the gradient is that of the dense tensor."""
+    gen, dev = torch.Generator().manual_seed(3), torch.device("cuda:0")
+    gu = torch.randn(6, 1024, generator=gen).to(torch.bfloat16).to(dev).requires_grad_()
+    grad = torch.randn(6, 512, generator=gen).to(torch.bfloat16).to(dev)
+    want, = torch.autograd.grad(_silu_mul(gu), gu, grad)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.flatten()
+        return flat[1:].view(t.shape)
+
+    for unpack in (lambda t: t.t().contiguous().t(), shifted):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), unpack):
+            y = _silu_mul(gu * 1)
+        got, = torch.autograd.grad(y, gu, grad)
+        assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
 def test_an_empty_batch_passes_forward_and_backward():
     gen, dev = torch.Generator().manual_seed(4), torch.device("cuda:0")
     linear = lambda: Int4Linear.from_linear(torch.nn.Linear(256, 512, bias=False).to(torch.bfloat16).to(dev), 128)

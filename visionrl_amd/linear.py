@@ -333,7 +333,7 @@ class _SiLUMul(torch.autograd.Function):
             recorded = torch.is_grad_enabled()
             with torch.enable_grad():
                 return torch.autograd.grad(_silu_mul_ops(gate_up), gate_up, grad, create_graph=recorded)[0]
-        return ops.silu_mul_backward(gate_up, _aligned(grad))
+        return ops.silu_mul_backward(_aligned(gate_up), _aligned(grad))   # (a saved-tensor hook may have made a view)
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
