@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "dequant_grid.hpp"
 
 namespace {
 
@@ -65,39 +66,37 @@ __device__ __forceinline__ void dequant_word(uint32_t v, const GroupConst &g, ui
 }
 
 // -------------------------------------------------------------------------
-// dequant: one thread per packed word of four rows, natural k order out
+// dequant: one thread per packed word of ROWS rows, natural k order out
 // -------------------------------------------------------------------------
-// A wave's loads and 16-byte stores are contiguous; the four rows' loads are independent, which is what keeps
-// enough of them in flight (2048 x 2048 / 2048 x 5632 / 11264 x 2048: 4.0 / 6.5 / 10.4 us against 4.5 / 7.8 / 11.8
-// with one word per thread and a 64-bit division for its row).  A block covers one of
-// the `segments` of a row, 1 << tshift words; threads beyond that are on the next rows.
-constexpr int DEQUANT_ROWS = 4;
-
-__global__ __launch_bounds__(256) void dequant_kernel(const uint32_t *__restrict__ qweight,
-                                                      const uint16_t *__restrict__ scales,
-                                                      const uint32_t *__restrict__ qzeros,
-                                                      uint16_t *__restrict__ w, int N, int K, int G, int tshift,
-                                                      int segments) {
-    const int kwords = K >> 3;
-    const int groups = K / G;
+// A wave's loads and 16-byte stores are contiguous; the rows' loads are independent, which is what keeps enough of
+// them in flight.  A block covers one segment of a row, blockIdx.x; threads beyond it are on the next rows.  Calls
+// queued back to back, 512 x 2048 / 2048 x 2048 / 2048 x 5632 / 11264 x 2048: 2.4 / 3.9 / 7.3 / 10.9 us, against
+// 3.2 / 4.2 / 8.2 / 11.8 with the segment found by a division and four rows at every size, and 2.7 / 4.4 / 8.1 / 12.1
+// with one word per thread and a 64-bit division for its row.
+template <int ROWS>
+__global__ __launch_bounds__(DEQUANT_THREADS) void dequant_kernel(const uint32_t *__restrict__ qweight,
+                                                                  const uint16_t *__restrict__ scales,
+                                                                  const uint32_t *__restrict__ qzeros,
+                                                                  uint16_t *__restrict__ w, int N, int kwords,
+                                                                  int groups, int G, int tshift) {
     const int zwords = (groups + 7) >> 3;
-    const int step = 256 >> tshift;   // rows the block covers at a time
-    const long n0 = (long)((int)blockIdx.x / segments) * (DEQUANT_ROWS * step) + ((int)threadIdx.x >> tshift);
-    const int r = ((int)blockIdx.x % segments << tshift) + ((int)threadIdx.x & ((1 << tshift) - 1));
+    const int step = DEQUANT_THREADS >> tshift;   // rows the block covers at a time
+    const int n0 = (int)blockIdx.y * (ROWS * step) + ((int)threadIdx.x >> tshift);
+    const int r = ((int)blockIdx.x << tshift) + ((int)threadIdx.x & ((1 << tshift) - 1));
     if (r >= kwords) return;
     const int g = (r << 3) / G;
-    uint32_t v[DEQUANT_ROWS], z[DEQUANT_ROWS];
-    float s[DEQUANT_ROWS];
+    uint32_t v[ROWS], z[ROWS];
+    float s[ROWS];
 #pragma unroll
-    for (int j = 0; j < DEQUANT_ROWS; ++j) {
-        const long n = min(n0 + j * step, (long)N - 1);
+    for (int j = 0; j < ROWS; ++j) {
+        const long n = min(n0 + j * step, N - 1);
         v[j] = qweight[n * kwords + r];
         s[j] = bf16_bits_to_f32(scales[n * groups + g]);
         z[j] = qzeros[n * zwords + (g >> 3)];
     }
 #pragma unroll
-    for (int j = 0; j < DEQUANT_ROWS; ++j) {
-        const long n = n0 + j * step;
+    for (int j = 0; j < ROWS; ++j) {
+        const int n = n0 + j * step;
         if (n >= N) break;
         const int zero = (z[j] >> (4 * (g & 7))) & 0xF;
         u32x4_t o;
@@ -107,7 +106,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t *__restrict
             const int q1 = (v[j] >> (8 * i + 4)) & 0xF;
             o[i] = pack_bf16_rne((float)(q0 - zero) * s[j], (float)(q1 - zero) * s[j]);
         }
-        *reinterpret_cast<u32x4_t *>(w + (n * kwords + r) * 8) = o;
+        *reinterpret_cast<u32x4_t *>(w + ((long)n * kwords + r) * 8) = o;
     }
 }
 

@@ -435,18 +435,18 @@ int vrl_int4_dequant_bf16(const void *qweight, const void *scales, const void *q
                           int N, int K, int G, void *hip_stream) {
     int rc = check_problem(qweight, qweight, scales, qzeros, w, 1, N, K, G);
     if (rc != VRL_INT4_OK) return rc;
-    // threads per row: the power of two that covers its words, 256 at most (then the row is cut into segments)
-    const int kwords = K >> 3;
-    int tshift = 0;
-    while (tshift < 8 && (1 << tshift) < kwords) ++tshift;
-    const long segments = (kwords + (1 << tshift) - 1) >> tshift, rows = DEQUANT_ROWS * (256 >> tshift);
-    const long blocks = (N + rows - 1) / rows * segments;
-    if (blocks >= (1L << 31)) return VRL_INT4_ESHAPE;
-    return vrl_launch(&dequant_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(hip_stream),
-                       static_cast<const uint32_t *>(qweight), static_cast<const uint16_t *>(scales),
-                       static_cast<const uint32_t *>(qzeros), static_cast<uint16_t *>(w), N, K, G, tshift,
-                       (int)segments);
+    const DequantGrid grid = dequant_grid(N, K);
+    const long kwords = K >> 3, groups = K / G, zwords = (groups + 7) >> 3;
+    auto kernel = grid.rows == 1 ? &dequant_kernel<1> : &dequant_kernel<4>;
+    for (int tile = 0; rc == VRL_INT4_OK && tile < grid.tiles; tile += DEQUANT_TILES) {
+        const long n = (long)tile * grid.span;
+        rc = vrl_launch(kernel, dim3((unsigned)grid.segments, (unsigned)std::min(grid.tiles - tile, DEQUANT_TILES)),
+                        dim3(DEQUANT_THREADS), 0, reinterpret_cast<hipStream_t>(hip_stream),
+                        static_cast<const uint32_t *>(qweight) + n * kwords, static_cast<const uint16_t *>(scales) + n * groups,
+                        static_cast<const uint32_t *>(qzeros) + n * zwords, static_cast<uint16_t *>(w) + n * K,
+                        (int)(N - n), (int)kwords, (int)groups, G, grid.tshift);
+    }
+    return rc;
 }
 
 size_t vrl_int4_prepacked_bytes(int N, int K, int G) {
