@@ -134,7 +134,8 @@ typedef struct vrl_int4_problem {
  * policy.py:640-672).  Every problem has prepacked = 0 and the same K, G and fused_gate_up.  Shapes that the
  * launch has no build for return VRL_INT4_ELIMIT and nothing is enqueued (it needs K % 128 == 0, G a power of two
  * >= 32, and 512 bytes of LDS per group of a 128-row weight tile): rebuild the weight with
- * vrl_int4_dequant_bf16() and use a library product, which is also the faster form from about 2048 rows on.
+ * vrl_int4_dequant_bf16() and use a library product.  That is also the faster form of large products, from 512 to
+ * 2048 rows on depending on K, N and G.
  */
 int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_problems, void *hip_stream);
 

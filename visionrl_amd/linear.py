@@ -22,20 +22,57 @@ from . import ops
 from .int4_format import check_packed, pack_nibbles, quantize_minmax
 
 # Calls with more activation rows than this (the prompt pass) are matrix products; the GEMV kernels are for
-# decode.  Up to PROMPT_ROWS rows they go through the launch that rebuilds the weight in registers
-# (``ops.int4_gemm``: q|k|v of 512 rows by 2048 in 24 us against 3 x (4 + 12) us); beyond that, and wherever that
-# launch does not apply, the bf16 weight is rebuilt (bit-exact tile, one launch) and handed to the library GEMM,
-# whose rate makes up for the extra pass from there on (2048 x 5632 -> 2048: 54 against 6 + 48 us at 2048 rows,
-# 154 against 6 + 117 us at 8192).  gate|up goes back to the launch from FUSED_ROWS rows on where K is at most
-# FUSED_K: there SiLU's pass over the product costs more than the library's rate gains (2048 -> 2 x 5632: 164 us
-# against 120 + 10 + 21 at 3072 rows, 181 against 157 + 10 + 28 at 4096, 348 against 352 + 10 + 55 at 8192; the
-# pass is a smaller part of a longer K).
-# Weights of fewer than PROMPT_COLUMNS outputs stay on the library's route at every row count: rebuilding them
-# costs next to nothing, and their results are pinned bit for bit to the library's product.
+# decode.  They go through the launch that rebuilds the weight in registers (``ops.int4_gemm``) where that is the
+# faster form, :func:`_launch_pays`; elsewhere, and wherever that launch does not apply, the bf16 weight is rebuilt
+# (bit-exact tile, one launch) and handed to the library GEMM.
 GEMM_ROWS = 32
 PROMPT_ROWS = 2048
-FUSED_ROWS, FUSED_K = 4096, 2048
+FUSED_ROWS = 4096
+# Weights of fewer than PROMPT_COLUMNS outputs stay on the library's route at every row count, because their results
+# are pinned bit for bit to the library's product.  That is not the faster form (64 to 384 outputs by 2048, 33 to 2048
+# rows: 11.7 to 14 us against 8 to 9 for the launch), but a fraction of a layer of 100 us and more.
 PROMPT_COLUMNS = 512
+CUS = 256
+
+
+def _launch_pays(rows: int, K: int, columns: int, group_size: int, products: int = 1, fused: bool = False) -> bool:
+    """Whether one ``ops.int4_gemm`` launch beats rebuilding the weight and a library product per weight.
+
+    Both routes were timed, queued back to back on the GPU, at 33 to 8192 rows, K of 1024 to 11008, up to 22016 weight
+    rows and groups of 32, 64 and 128.  The library's rate is 1.2 to 1.4 times the launch's once its products are
+    large; what the launch saves is the pass that writes the weight, SiLU's pass and the launches of a group.  A group
+    costs as much again for each halving of the group size below 128, in the table of scales of every tile: ``k``
+    is the K of equal cost.
+    """
+    groups = K // group_size
+    k = max(K, 128 * groups)
+    work = rows * columns * k
+    if fused:
+        # 2048 -> 2 x 5632: 44 against 52 us at 512 rows, 96 against 109 at 1792; 3072 -> 2 x 8192: 96 against 109 at
+        # 1024, 165 against 155 at 1536; 4096 -> 2 x 11008: 83 against 102 at 256, 236 against 209 at 1024.  From
+        # FUSED_ROWS on a short K is faster again, for SiLU's pass (K = 2048: 193 against 192 us at 4096 rows, 373
+        # against 408 at 8192; K = 3072: 365 against 335 and 708 against 639).
+        return rows <= PROMPT_ROWS and work <= 48 << 30 or rows >= FUSED_ROWS and K <= 2048 and k <= 4096
+    if rows > PROMPT_ROWS:
+        return False
+    tiles = lambda bm, bn: -(-rows // bm) * -(-columns // bn)
+    if products > 1:
+        # q|k|v of 2048 / 3072 / 4096 outputs each: 61 / 108 / 207 us against 87 / 150 / 194 at 1664 rows (the last
+        # stays with the library), 26 / 64 / 84 against 63 / 93 / 120 at 512.  Beyond 80 groups only one workgroup
+        # fits a CU and more than a round of them is slow (groups of 32, K = 4096: 56 against 98 us at 256 rows, one
+        # round; 144 against 117 at 512).
+        return work < 72 << 30 if groups <= 80 else tiles(128, 128) <= CUS
+    # One weight: worth it while its tiles are one round of workgroups of the builds that split K (5632 -> 2048: 38
+    # against 46 us at 1024 rows, 58 against 51 at 1152; 11008 -> 4096: 67 against 85 at 512, 110 against 94 at 768),
+    # as far as their tables fit.  Beyond that with two of: one round of 128 x 128 tiles, a short K, few rows
+    # (2048 -> 2048: 26 against 30 us at 2048 rows; 4096 -> 16384: 48 against 76 at 256; 2048 -> 16384: 48 against 54
+    # at 512; 4096 -> 4096: 45 against 42 at 768, where only the first holds).
+    for bm, bn, most in ((32, 64, 448), (64, 64, 320), (64, 128, 128)):
+        if groups <= most and tiles(bm, bn) <= CUS:
+            return True
+    return (groups <= 160 and tiles(128, 128) <= CUS) + (k <= 3072) + (rows <= 512) >= 2
+
+
 _PLAIN = (torch.Tensor, nn.Parameter)
 
 
@@ -236,22 +273,26 @@ class Int4Linear(nn.Module):
 
     def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
         """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
-        if rows.shape[0] > PROMPT_ROWS or self.out_features < PROMPT_COLUMNS or \
-                getattr(self, "_keep_dense", False) or not _launchable(x):
+        M, K, G = rows.shape[0], self.in_features, self.group_size
+        if M > PROMPT_ROWS or self.out_features < PROMPT_COLUMNS or getattr(self, "_keep_dense", False) or \
+                not _launchable(x):
             return None
         group = self.__dict__.get("_group")
         version = _version(x) if group is not None else None
         if version is not None and all(
-                m.group_size == self.group_size and m.out_features >= PROMPT_COLUMNS and
-                not m.__dict__.get("_keep_dense", False) for m in group[1:]):
+                m.group_size == G and m.out_features >= PROMPT_COLUMNS and
+                not m.__dict__.get("_keep_dense", False) for m in group[1:]) and \
+                _launch_pays(M, K, sum(m.out_features for m in group), G, len(group)):
             weights = [m._canonical() for m in group]
-            ys = ops.int4_gemm(rows, weights, self.group_size)
+            ys = ops.int4_gemm(rows, weights, G)
             if ys is not None:
                 stream = ops._stream_handle(x.device)
                 for m, ym, weight in zip(group[1:], ys[1:], weights[1:]):
                     m.__dict__["_handed"] = (x, version, ym, stream, _source_state(*weight))
                 return ys[0]
-        ys = ops.int4_gemm(rows, [self._canonical()], self.group_size)
+        if not _launch_pays(M, K, self.out_features, G):
+            return None
+        ys = ops.int4_gemm(rows, [self._canonical()], G)
         return None if ys is None else ys[0]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -381,8 +422,9 @@ class Int4GateUpSiLU(nn.Module):
     def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
         """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
         M = rows.shape[0]
-        if not (GEMM_ROWS < M <= PROMPT_ROWS or M >= FUSED_ROWS and self.in_features <= FUSED_K) or \
-                self.intermediate_size < PROMPT_COLUMNS or getattr(self, "_keep_dense", False) or not _launchable(x):
+        if M <= GEMM_ROWS or self.intermediate_size < PROMPT_COLUMNS or getattr(self, "_keep_dense", False) or \
+                not _launchable(x) or \
+                not _launch_pays(M, self.in_features, 2 * self.intermediate_size, self.group_size, fused=True):
             return None
         ys = ops.int4_gemm(rows, [self._canonical()], self.group_size, True)
         return None if ys is None else ys[0]
