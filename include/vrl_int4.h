@@ -125,13 +125,16 @@ typedef struct vrl_int4_problem {
     int32_t M, N, K, G;
     int32_t fused_gate_up; /* 0: y[M,N]; 1: rows are gate||up, y[M,N/2] with the SiLU epilogue */
     int32_t prepacked;     /* 1: qweight is a blob made by vrl_int4_prepack(); scales/qzeros unused */
-    int32_t reserved[2];   /* 0 */
+    void *product;         /* vrl_int4_gemm_bf16() with fused_gate_up: where gate||up itself is kept too, bf16 [M,N],
+                              or NULL; 0 everywhere else */
 } vrl_int4_problem;
 
 /*
  * The products of a prompt pass: y[M,N] = x[M,K] . dequant(W)^T (or the fused gate||up form) for any number of
  * activation rows, over the canonical operands, up to 8 problems in one launch (the q|k|v linears of a layer,
- * policy.py:640-672).  Every problem has prepacked = 0 and the same K, G and fused_gate_up.  Shapes that the
+ * policy.py:640-672).  Every problem has prepacked = 0 and the same K, G and fused_gate_up.  A fused problem with
+ * `product` set also stores x . dequant(W)^T before SiLU, rounded to bf16, for a caller that will need its gradient
+ * (the replay, policy.py:419-424); y is the same either way.  Shapes that the
  * launch has no build for return VRL_INT4_ELIMIT and nothing is enqueued (it needs K % 128 == 0, G a power of two
  * >= 32, and 512 bytes of LDS per group of a 128-row weight tile): rebuild the weight with
  * vrl_int4_dequant_bf16() and use a library product.  That is also the faster form of large products, from 512 to

@@ -72,6 +72,22 @@ def test_prompt_gemm_matches_dequantised_product(M, N, K, G, fused, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,G", [
+    (129, 2 * 77, 512, 32), (33, 2 * 5632, 2048, 128), (700, 2 * 2050, 512, 128), (1664, 2 * 5632, 256, 128),
+    (4100, 2 * 1700, 512, 64),
+])
+def test_fused_launch_keeps_the_product_beside_the_result(M, N, K, G):
+    gen, dev = torch.Generator().manual_seed(M), torch.device("cuda:0")
+    triple = _triple(gen, K, N, G, dev)
+    x = torch.randn(M, K, generator=gen).to(torch.bfloat16).to(dev)
+    products = []
+    y, = ops.int4_gemm(x, [triple], G, True, products)
+    assert torch.equal(y, ops.int4_gemm(x, [triple], G, True)[0])
+    ref, tol = _reference(x, triple, G, False)
+    assert products[0].shape == (M, N) and bool(((products[0].double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
 def test_prompt_gemm_leaves_other_operands_to_the_general_route():
     gen, dev = torch.Generator().manual_seed(3), torch.device("cuda:0")
     x = torch.randn(64, 360, generator=gen).to(torch.bfloat16).to(dev)
@@ -176,6 +192,7 @@ def test_prompt_gemm_rejects_bad_calls():
         for rec in table:
             rec.x = rec.qweight = rec.scales = rec.qzeros = rec.y = p
             rec.M, rec.N, rec.K, rec.G, rec.fused_gate_up, rec.prepacked = 64, 32, 256, 128, 0, 0
+            rec.product = None
         for name, value in fields.items():
             setattr(table[n - 1], name, value)
         return lib.vrl_int4_gemm_bf16(table, n, None)
@@ -186,6 +203,7 @@ def test_prompt_gemm_rejects_bad_calls():
     assert call(M=0) == 1001 and call(prepacked=1) == 1001
     assert call(2, K=512) == 1001 and call(2, G=64) == 1001 and call(2, fused_gate_up=1) == 1001
     assert call(N=33, fused_gate_up=1) == 1001
+    assert call(product=p) == 1001 and call(product=p + 8, fused_gate_up=1) == 1002
     assert call(K=264, G=8) == 1005 and call(K=192, G=64) == 1005 and call(K=384, G=96) == 1005
 
 

@@ -118,7 +118,7 @@ class Problem(ctypes.Structure):
         ("G", ctypes.c_int32),
         ("fused_gate_up", ctypes.c_int32),
         ("prepacked", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 2),
+        ("product", ctypes.c_void_p),
     ]
 
 

@@ -31,6 +31,7 @@ struct GemmRec {
     const uint16_t *scales;
     const uint32_t *qzeros;
     uint16_t *y;
+    uint16_t *product;   // fused records: [M, N] before SiLU, or null
     int32_t M, N;        // N: weight rows (gate||up: both halves)
     int32_t tile_begin;  // first tile of the record in the launch
     int32_t mtiles;
@@ -297,6 +298,18 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 || C::MB * C::NB >= 32 ? 
     // lane: row lc of each row block, columns 4 kq .. 4 kq + 3 of each column block
     constexpr int OB = FUSED ? C::NB / 2 : C::NB;
     const bool wide = (out_cols & 3) == 0;
+    auto store = [&](uint16_t *row, int col, const f32x4_t &v) {
+        const u32x2_t o = {pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3])};
+        uint16_t *at = row + col;
+        if (wide) {
+            if (col < out_cols) *reinterpret_cast<u32x2_t *>(at) = o;
+        } else {
+            if (col < out_cols) at[0] = (uint16_t)o[0];
+            if (col + 1 < out_cols) at[1] = (uint16_t)(o[0] >> 16);
+            if (col + 2 < out_cols) at[2] = (uint16_t)o[1];
+            if (col + 3 < out_cols) at[3] = (uint16_t)(o[1] >> 16);
+        }
+    };
 #pragma unroll
     for (int b = 0; b < OWN; ++b) {
         const int m = mt * C::BM + xrow0 + 16 * (b0 + b);
@@ -307,19 +320,15 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 || C::MB * C::NB >= 32 ? 
             f32x4_t v = acc[b][n];
             if constexpr (FUSED) {
                 const f32x4_t u = acc[b][n + OB];
+                if (p.product) {
+                    uint16_t *row = p.product + (long)m * p.N;
+                    store(row, col, v);
+                    store(row + out_cols, col, u);
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[i] = (v[i] / (1.0f + __expf(-v[i]))) * u[i];
             }
-            uint16_t *y = p.y + (long)m * out_cols + col;
-            const u32x2_t o = {pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3])};
-            if (wide) {
-                if (col < out_cols) *reinterpret_cast<u32x2_t *>(y) = o;
-            } else {
-                if (col < out_cols) y[0] = (uint16_t)o[0];
-                if (col + 1 < out_cols) y[1] = (uint16_t)(o[0] >> 16);
-                if (col + 2 < out_cols) y[2] = (uint16_t)o[1];
-                if (col + 3 < out_cols) y[3] = (uint16_t)(o[1] >> 16);
-            }
+            store(p.y + (long)m * out_cols, col, v);
         }
     }
 }
@@ -419,6 +428,8 @@ extern "C" int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_proble
         if (rc != VRL_INT4_OK) return rc;
         if (q.prepacked || q.K != q0.K || q.G != q0.G || (q.fused_gate_up != 0) != fused || (fused && q.N % 2 != 0))
             return VRL_INT4_ESHAPE;
+        if (q.product && !fused) return VRL_INT4_ESHAPE;
+        if (!aligned16(q.product)) return VRL_INT4_EALIGN;
         if (q.K % 128 != 0 || q.G % 32 != 0 || !pow2(q.G) || (long)q.N * q.K / 2 >= (1L << 32)) return VRL_INT4_ELIMIT;
         GemmRec &r = args.recs[i];
         r.x = static_cast<const uint16_t *>(q.x);
@@ -426,6 +437,7 @@ extern "C" int vrl_int4_gemm_bf16(const vrl_int4_problem *problems, int n_proble
         r.scales = static_cast<const uint16_t *>(q.scales);
         r.qzeros = static_cast<const uint32_t *>(q.qzeros);
         r.y = static_cast<uint16_t *>(q.y);
+        r.product = static_cast<uint16_t *>(q.product);
         r.M = q.M;
         r.N = q.N;
     }

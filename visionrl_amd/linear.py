@@ -6,12 +6,14 @@ The reference calls its decode linears as plain modules, ``module(x[..., K]) ->
 ``policy.py:138-160`` for ``gen_head``).  These modules keep that calling
 convention and route the arithmetic to the HIP library; the weights are frozen
 (no gradient flows into the packed tensors).  A call whose input carries a gradient
-(a train-time replay over the quantised base, e.g. under LoRA adapters) multiplies by
-the dequantised weight through the library GEMM, so the gradient reaches the input.
+(a train-time replay over the quantised base, e.g. under LoRA adapters) computes the same
+product, at prompt sizes bit for bit that of a call without one, and multiplies the gradient
+by the dequantised weight, so that it reaches the input.
 """
 
 from __future__ import annotations
 
+import functools
 import weakref
 
 import torch
@@ -35,6 +37,7 @@ PROMPT_COLUMNS = 512
 CUS = 256
 
 
+@functools.lru_cache(maxsize=1024)   # (sizes only; a hit is 0.4 us less on every call of a prompt)
 def _launch_pays(rows: int, K: int, columns: int, group_size: int, products: int = 1, fused: bool = False) -> bool:
     """Whether one ``ops.int4_gemm`` launch beats rebuilding the weight and a library product per weight.
 
@@ -107,6 +110,13 @@ def _source_state(*tensors):
     and shape of its data instead.  In-place writes to such a tensor go unnoticed: ``prepack_()`` again
     after editing int4 buffers that were created under ``torch.inference_mode``."""
     return tuple((weakref.ref(t), _version(t), (t.data_ptr(), tuple(t.shape))) for t in tensors)
+
+
+def _versions(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor):
+    try:
+        return a._version, b._version, c._version
+    except RuntimeError:      # an inference tensor among them
+        return _version(a), _version(b), _version(c)
 
 
 def _source_changed(state, *tensors) -> bool:
@@ -226,6 +236,9 @@ class Int4Linear(nn.Module):
         of this module computes all of them in one plan-free launch and hands each sibling its
         result, which the sibling returns when it is called with the very same tensor object
         next.  Needs ``prepack_()`` on every member; anything else falls back to one launch each.
+        Prompt-sized calls, with and without a gradient, share a launch the same way over the canonical
+        buffers, where that is the faster route and every member has ``PROMPT_COLUMNS`` outputs; a caller
+        that wants the leader's result alone pays for the siblings' too.
         """
         if len(others) + 1 > ops.DirectGemv.MAX_PROBLEMS:
             raise ValueError(f"at most {ops.DirectGemv.MAX_PROBLEMS} modules per group")
@@ -247,7 +260,9 @@ class Int4Linear(nn.Module):
         """Keep the dequantised bf16 weight between calls (2 bytes per weight beside the 0.56 of the int4
         buffers): prompt-sized calls and the train-time replay (``policy.py:419-424``: one forward per
         micro-batch) then multiply by the kept tensor instead of rebuilding it every call.  It is rebuilt
-        when the canonical buffers were written or replaced since; ``keep=False`` drops it."""
+        when the canonical buffers were written or replaced since; ``keep=False`` drops it.  These are library
+        products at every size: where a module without the copy takes the prompt launch its results differ by the
+        order of fp32 sums, and by the rounding of gate and up before SiLU."""
         self._keep_dense = bool(keep)
         self._dense = None
         return self
@@ -279,21 +294,38 @@ class Int4Linear(nn.Module):
             return None
         group = self.__dict__.get("_group")
         version = _version(x) if group is not None else None
-        if version is not None and all(
-                m.group_size == G and m.out_features >= PROMPT_COLUMNS and
-                not m.__dict__.get("_keep_dense", False) for m in group[1:]) and \
-                _launch_pays(M, K, sum(m.out_features for m in group), G, len(group)):
-            weights = [m._canonical() for m in group]
-            ys = ops.int4_gemm(rows, weights, G)
-            if ys is not None:
-                stream = ops._stream_handle(x.device)
-                for m, ym, weight in zip(group[1:], ys[1:], weights[1:]):
-                    m.__dict__["_handed"] = (x, version, ym, stream, _source_state(*weight))
-                return ys[0]
+        if version is not None:
+            columns = 0
+            for m in group:
+                if m.group_size != G or m.out_features < PROMPT_COLUMNS or m.__dict__.get("_keep_dense", False):
+                    break
+                columns += m.out_features
+            else:
+                if _launch_pays(M, K, columns, G, len(group)):
+                    weights = [m._canonical() for m in group]
+                    ys = ops.int4_gemm(rows, weights, G)
+                    if ys is not None:
+                        # (x by weak reference: with a gradient it would keep what led to it alive)
+                        call = weakref.ref(x), version, ops._stream_handle(x.device)
+                        for m, ym, weight in zip(group[1:], ys[1:], weights[1:]):
+                            m.__dict__["_handed"] = (call, ym, weight, _versions(*weight))
+                        return ys[0]
         if not _launch_pays(M, K, self.out_features, G):
             return None
         ys = ops.int4_gemm(rows, [self._canonical()], G)
         return None if ys is None else ys[0]
+
+    def _take(self, handed, x: torch.Tensor, grad: bool):
+        """The handed result if it is this call's: of this very tensor, unchanged since, on this stream."""
+        if len(handed) == 3:   # from a decode-sized launch
+            return handed[2] if not grad and handed[0] is x and handed[1] == _version(x) else None
+        (ref, version, stream), y, (qweight, scales, qzeros), versions = handed
+        if ref() is not x or version != _version(x) or stream != ops._stream_handle(x.device) or \
+                grad and not _launchable(x):
+            return None
+        mine = self._canonical()
+        return y if mine[0] is qweight and mine[1] is scales and mine[2] is qzeros and \
+            versions == _versions(*mine) else None
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         rows = _rows(x, self.in_features)
@@ -303,18 +335,20 @@ class Int4Linear(nn.Module):
         own = self.__dict__   # plain attributes: nn.Module's own lookups and assignments cost microseconds
         handed = own.get("_handed")
         if handed is not None:
+            handed = own.pop("_handed", None)   # (one of two threads gets it)
             own["_handed"] = None
         group = own.get("_group")
         if group is not None:   # a new call of the leader: whatever it handed over before is void
             for m in group[1:]:
                 m.__dict__["_handed"] = None
-        if _wants_grad(x):
-            y = F.linear(rows, self._dense_weight(x))
-        elif handed is not None and handed[0] is x and handed[1] == _version(x) and \
-                (len(handed) == 3 or (handed[3] == ops._stream_handle(x.device) and
-                                      not _source_changed(handed[4], *self._canonical()))):
-            y = handed[2]   # computed by the group leader's launch from this very tensor, unchanged since
-        else:  # eager decode: skip the operator dispatcher, it costs more than the kernel
+        grad = _wants_grad(x)
+        y = None if handed is None else self._take(handed, x, grad)   # computed by the group leader's launch
+        if grad:   # the same product as without a gradient, bit for bit, at every prompt size
+            weight = self._dense_weight(x)
+            if y is None and rows.shape[0] > GEMM_ROWS:
+                y = self._prompt_gemm(x, rows)
+            y = F.linear(rows, weight) if y is None else _Launched.apply(rows, [y], weight)
+        elif y is None:  # eager decode: skip the operator dispatcher, it costs more than the kernel
             packed = self._fresh_packed()
             M = rows.shape[0]
             if packed is not None and packed.blob.device == rows.device:
@@ -358,23 +392,43 @@ def _silu_mul_ops(gate_up: torch.Tensor) -> torch.Tensor:
     return F.silu(gate) * up
 
 
-class _SiLUMul(torch.autograd.Function):
-    """``silu(gate) * up`` with its gradient as one launch each; only the product itself is saved.  A backward
-    that is itself recorded, or watched by a transform, goes through the torch operators."""
+class _Launched(torch.autograd.Function):
+    """What a launch computed from ``rows`` (handed in as a list, or it would count as an input), with the gradient
+    of ``rows . weight^T``: that of ``F.linear``, whose node saves the weight too."""
 
     @staticmethod
-    def forward(ctx, gate_up):
+    def forward(ctx, rows, result, weight):
+        ctx.save_for_backward(weight)
+        return result[0]
+
+    @staticmethod
+    def backward(ctx, grad):
+        weight, = ctx.saved_tensors
+        if torch.is_autocast_enabled("cuda"):   # a backward called under it: the product's type is the forward's
+            with torch.autocast("cuda", enabled=False):
+                return grad @ weight, None, None
+        return grad @ weight, None, None
+
+
+class _SiLUMul(torch.autograd.Function):
+    """``silu(gate) * up`` with its gradient as one launch each; only the product itself is saved.  ``result``: a
+    list that holds the value where a launch has computed it with the product.  A backward that is itself recorded,
+    or watched by a transform, goes through the torch operators."""
+
+    @staticmethod
+    def forward(ctx, gate_up, result):
         ctx.save_for_backward(gate_up)
-        return ops.silu_mul(gate_up)
+        return result[0] if result else ops.silu_mul(gate_up)
 
     @staticmethod
     def backward(ctx, grad):
         gate_up, = ctx.saved_tensors
-        if torch.is_grad_enabled() or not (_launchable(grad) and _launchable(gate_up)):
+        if torch.is_grad_enabled() or gate_up.shape[-1] % 16 or not (_launchable(grad) and _launchable(gate_up)):
             recorded = torch.is_grad_enabled()
             with torch.enable_grad():
-                return torch.autograd.grad(_silu_mul_ops(gate_up), gate_up, grad, create_graph=recorded)[0]
-        return ops.silu_mul_backward(_aligned(gate_up), _aligned(grad))   # (a saved-tensor hook may have made a view)
+                return torch.autograd.grad(_silu_mul_ops(gate_up), gate_up, grad, create_graph=recorded)[0], None
+        # (a saved-tensor hook may have made a view)
+        return ops.silu_mul_backward(_aligned(gate_up), _aligned(grad)), None
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
@@ -388,7 +442,7 @@ def _silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     if not _launchable(gate_up) or gate_up.dtype != torch.bfloat16 or inter < PROMPT_COLUMNS or inter % 8 != 0 \
             or not 0 < gate_up.numel() < 2 ** 31 or not gate_up.is_contiguous() or gate_up.data_ptr() % 16 != 0:
         return _silu_mul_ops(gate_up)
-    return _SiLUMul.apply(gate_up) if _wants_grad(gate_up) else ops.silu_mul(gate_up)
+    return _SiLUMul.apply(gate_up, None) if _wants_grad(gate_up) else ops.silu_mul(gate_up)
 
 
 class Int4GateUpSiLU(nn.Module):
@@ -419,15 +473,18 @@ class Int4GateUpSiLU(nn.Module):
             self._call = ops.DirectCall([self._packed], fused=True)
         return self
 
-    def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor):
+    def _prompt_gemm(self, x: torch.Tensor, rows: torch.Tensor, grad: bool):
         """A prompt-sized call as one launch, or ``None`` where the general route is the better or only one."""
         M = rows.shape[0]
         if M <= GEMM_ROWS or self.intermediate_size < PROMPT_COLUMNS or getattr(self, "_keep_dense", False) or \
                 not _launchable(x) or \
                 not _launch_pays(M, self.in_features, 2 * self.intermediate_size, self.group_size, fused=True):
             return None
-        ys = ops.int4_gemm(rows, [self._canonical()], self.group_size, True)
-        return None if ys is None else ys[0]
+        products = [] if grad else None
+        ys = ops.int4_gemm(rows, [self._canonical()], self.group_size, True, products)
+        if ys is None or not grad:
+            return None if ys is None else ys[0]
+        return _SiLUMul.apply(_Launched.apply(rows, products, self._dense_weight(x)), ys)
 
     _canonical = Int4Linear._canonical
     packed_is_stale = Int4Linear.packed_is_stale
@@ -442,7 +499,7 @@ class Int4GateUpSiLU(nn.Module):
         if packed is not None and not grad and not torch.compiler.is_compiling() \
                 and rows.shape[0] <= self._direct_rows and packed.blob.device == rows.device:
             y = self._call(rows)[0]
-        elif not grad and not torch.compiler.is_compiling() and (launched := self._prompt_gemm(x, rows)) is not None:
+        elif not torch.compiler.is_compiling() and (launched := self._prompt_gemm(x, rows, grad)) is not None:
             y = launched
         elif (grad or rows.shape[0] > GEMM_ROWS) and not torch.compiler.is_compiling():
             y = _silu_mul(F.linear(rows, self._dense_weight(x)))   # prompt-sized call: one library GEMM

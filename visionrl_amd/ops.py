@@ -135,18 +135,21 @@ def int4_gemv_into(y: torch.Tensor, x: torch.Tensor, qweight: torch.Tensor, scal
     return y
 
 
-def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
+def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False, products: list | None = None):
     """Prompt-sized products of one input with several canonical weights in one launch, or ``None``.
 
     ``x`` is a contiguous bf16 ``[M, K]`` device tensor, ``weights`` a list of ``(qweight, scales, qzeros)``
-    triples of one group size (``fused``: gate||up triples, SiLU applied).  Returns one bf16 tensor per weight;
+    triples of one group size (``fused``: gate||up triples, SiLU applied; ``products``, an empty list, then receives
+    the bf16 ``[M, 2 I]`` product of each as well).  Returns one bf16 tensor per weight;
     ``None`` for operands the launch has no build for (an odd group size, a misaligned view, scales that do not
     fit its LDS), in which case nothing was enqueued and the caller takes its general route.  Another ``x`` is
     refused: the launch reads ``M * K`` bf16 values from its address.
     """
-    _require_rows("x", x)
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous()):
+        _require_rows("x", x)
+        _require_device("x", x)
     M, K = x.shape
-    dev, G = _require_device("x", x), int(group_size)
+    dev, index, G = x.device, x.get_device(), int(group_size)
     words, groups = K // 8, K // G
     zwords = (groups + 7) // 8
     table = (_lib.Problem * len(weights))()
@@ -156,13 +159,16 @@ def int4_gemm(x: torch.Tensor, weights, group_size: int, fused: bool = False):
         if qweight.dtype != torch.int32 or qzeros.dtype != torch.int32 or scales.dtype != torch.bfloat16 or \
                 qweight.shape != (N, words) or scales.shape != (N, groups) or qzeros.shape != (N, zwords) or \
                 not (qweight.is_contiguous() and scales.is_contiguous() and qzeros.is_contiguous()) or \
-                not (qweight.device == dev and scales.device == dev and qzeros.device == dev):
+                not qweight.get_device() == scales.get_device() == qzeros.get_device() == index:
             return None
         y = torch.empty((M, N // 2 if fused else N), dtype=torch.bfloat16, device=dev)
         rec.x, rec.qweight, rec.scales, rec.qzeros, rec.y = \
             xp, qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), y.data_ptr()
         rec.M, rec.N, rec.K, rec.G, rec.fused_gate_up = M, N, K, G, flag
         outs.append(y)
+        if products is not None:
+            products.append(torch.empty((M, N), dtype=torch.bfloat16, device=dev))
+            rec.product = products[-1].data_ptr()
     with _on(dev):
         rc = _lib.load().vrl_int4_gemm_bf16(table, len(outs), _stream_handle(dev))
     if rc >= 1000:
