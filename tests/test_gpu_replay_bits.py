@@ -136,3 +136,20 @@ def test_checkpointed_layers_repeat_their_results(reentrant):
     checkpoint(block, x, use_reentrant=reentrant).sum().backward()
     assert torch.equal(x.grad, plain)
     assert len(seen) >= 2 and all(torch.equal(a, b) for other in seen[1:] for a, b in zip(seen[0], other))
+
+
+def test_results_are_not_handed_across_a_capture(launches):
+    """A leader's captured launch has computed nothing yet when the sibling is called outside the graph."""
+    gen, (q, k, v, *_) = _layer(5)
+    x = _input(gen, 64, 512)
+    with torch.no_grad():
+        want = q(x), k(x), v(x)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(side):
+            with torch.cuda.graph(graph, stream=side):
+                q(x)
+            n = len(launches)
+            assert torch.equal(k(x), want[1]) and len(launches) == n + 1
+        torch.cuda.synchronize()

@@ -96,6 +96,9 @@ def _launchable(x: torch.Tensor) -> bool:
         and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
 
 
+_capturing = torch._C._cuda_isCurrentStreamCapturing   # (torch.cuda's own form costs twice as much)
+
+
 def _version(t: torch.Tensor):
     """The tensor's in-place modification counter, or ``None`` where torch keeps none (inference tensors)."""
     try:
@@ -306,7 +309,7 @@ class Int4Linear(nn.Module):
                     ys = ops.int4_gemm(rows, weights, G)
                     if ys is not None:
                         # (x by weak reference: with a gradient it would keep what led to it alive)
-                        call = weakref.ref(x), version, ops._stream_handle(x.device)
+                        call = weakref.ref(x), version, ops._stream_handle(x.device), _capturing()
                         for m, ym, weight in zip(group[1:], ys[1:], weights[1:]):
                             m.__dict__["_handed"] = (call, ym, weight, _versions(*weight))
                         return ys[0]
@@ -319,9 +322,9 @@ class Int4Linear(nn.Module):
         """The handed result if it is this call's: of this very tensor, unchanged since, on this stream."""
         if len(handed) == 3:   # from a decode-sized launch
             return handed[2] if not grad and handed[0] is x and handed[1] == _version(x) else None
-        (ref, version, stream), y, (qweight, scales, qzeros), versions = handed
+        (ref, version, stream, capturing), y, (qweight, scales, qzeros), versions = handed
         if ref() is not x or version != _version(x) or stream != ops._stream_handle(x.device) or \
-                grad and not _launchable(x):
+                capturing != _capturing() or grad and not _launchable(x):
             return None
         mine = self._canonical()
         return y if mine[0] is qweight and mine[1] is scales and mine[2] is qzeros and \
