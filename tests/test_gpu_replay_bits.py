@@ -153,3 +153,30 @@ def test_results_are_not_handed_across_a_capture(launches):
             n = len(launches)
             assert torch.equal(k(x), want[1]) and len(launches) == n + 1
         torch.cuda.synchronize()
+
+
+def test_a_default_device_changes_no_route(launches):
+    from torch.overrides import TorchFunctionMode
+
+    class Watching(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    gen, (q, k, v, o, mlp) = _layer(6)
+    x = _input(gen, 64, 512)
+    with torch.no_grad():
+        want = o(x), mlp(x)
+        n = len(launches)
+        for device in ("cpu", "cuda:0"):
+            with torch.device(device):
+                assert torch.equal(o(x), want[0]) and torch.equal(mlp(x), want[1])
+        assert len(launches) == n + 4
+        with torch.device("cpu"), Watching():              # another mode sees the torch operators, as before
+            o(x)
+        assert len(launches) == n + 4
+    with torch.device("cpu"):
+        xg = x.clone().requires_grad_()
+        y = mlp(xg)
+        assert torch.equal(y, want[1])
+        y.float().sum().backward()
+    assert xg.grad.device == x.device

@@ -19,6 +19,8 @@ import weakref
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import ops
 from .int4_format import check_packed, pack_nibbles, quantize_minmax
@@ -84,12 +86,19 @@ def _wants_grad(x: torch.Tensor) -> bool:
     return torch.is_grad_enabled() and x.requires_grad
 
 
+def _only_default_devices() -> bool:
+    """Whether the function modes in force are default devices (``torch.set_default_device``, ``with
+    torch.device(...)``): they give factory calls a device and watch nothing."""
+    return all(type(mode) is DeviceContext for mode in _get_current_function_mode_stack())
+
+
 def _launchable(x: torch.Tensor) -> bool:
     """Whether a prompt-sized call may leave the torch operators: nothing watches them (a trace, a dispatch mode,
     a functorch transform, forward-mode differentiation, an autocast to another type), and ``x`` is a plain
     tensor.  The general route goes through ``F.linear`` and serves all of those."""
     return type(x) in _PLAIN and x.is_cuda and not torch.jit.is_tracing() \
-        and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 \
+        and torch._C._len_torch_dispatch_stack() == 0 \
+        and (torch._C._len_torch_function_stack() == 0 or _only_default_devices()) \
         and torch._C._functorch.peek_interpreter_stack() is None \
         and not torch._C._functorch.is_legacy_batchedtensor(x) \
         and torch.autograd.forward_ad._current_level < 0 \
