@@ -23,16 +23,6 @@ def pytest_collection_modifyitems(config, items):
             item.add_marker(skip)
 
 
-@pytest.fixture(scope="module", autouse=True)
-def _collect_cycles():
-    """Module groups and graphs hold GPU tensors in cycles: what earlier tests left is freed before a module that
-    accounts for memory starts, not in the middle of it."""
-    import gc
-
-    gc.collect()
-    yield
-
-
 @pytest.fixture(scope="session")
 def c_oracle():
     """The C restatement, built on demand (gcc only; it is test infrastructure)."""

@@ -6,12 +6,21 @@ the fused form carries both operands' sums through ``silu(g) * u`` (|silu'| < 1.
 """
 
 import ctypes
+import gc
+
 import pytest
 import torch
 
 from visionrl_amd import _lib, ops
 from visionrl_amd import linear as linear_mod
 from visionrl_amd.linear import Int4GateUpSiLU, Int4Linear
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _groups_let_go():
+    """Grouped modules hold each other, and their GPU tensors, in cycles."""
+    yield
+    gc.collect()
 
 
 def _triple(gen, K, N, G, dev):
@@ -35,28 +44,67 @@ def _reference(x, triple, G, fused):
     return ref, eps + 2.0 ** -8 * ref.abs()
 
 
+# M, N, K, G, fused, n, and the tile whose build the launch takes for them at 256 CUs ("s": waves split K)
+CASES = [
+    (33, 64, 256, 128, False, 1, "32x64"),          # one row into the second tile
+    (64, 2048, 2048, 128, False, 1, "32x64"),
+    (65, 2050, 512, 32, False, 1, "32x64"),         # odd widths: narrow stores, a ragged last tile
+    (40, 17, 256, 64, False, 3, "32x64"),
+    (70, 128, 4096, 32, False, 1, "32x64"),         # the largest tables of scales
+    (500, 2048, 256, 128, False, 1, "64x64"),
+    (600, 1537, 512, 64, False, 1, "64x64"),
+    (300, 2048, 2048, 128, False, 3, "64x128"),
+    (500, 3001, 512, 32, False, 1, "64x128"),
+    (257, 2047, 256, 256, False, 3, "64x128"),
+    (200, 2 * 1000, 256, 128, True, 1, "64x128"),
+    (129, 2 * 77, 512, 32, True, 1, "64x128"),
+    (33, 2 * 5632, 2048, 128, True, 1, "64x128"),
+    (512, 3000, 512, 64, False, 2, "128x128s"),
+    (300, 1000, 384, 128, False, 1, "128x128s"),    # K not a multiple of 256: the tiles with shorter chunks
+    (130, 1000, 128, 128, False, 1, "128x128s"),    # one chunk
+    (48, 96, 128, 32, True, 1, "128x128s"),
+    (1664, 2048, 512, 128, False, 3, "128x128"),    # more tiles than CUs
+    (600, 2500, 5632, 32, False, 1, "128x128"),     # the other builds' tables do not fit
+    (2047, 2 * 1500, 256, 256, True, 1, "128x128"),
+    (4100, 2 * 1700, 512, 64, True, 1, "256x256"),  # ragged both ways
+    (4090, 3500, 256, 128, False, 1, "256x256"),
+    (511, 16000, 384, 32, False, 2, "256x256"),
+]
+
+
+def _build(M, N, K, G, fused, n, cus=256):
+    """The library's choice of tile, restated: rows and columns, chunk of K, waves, blocks of 16 x 16 per wave."""
+    builds = {"32x64": (32, 64, 256, 8, 2), "64x64": (64, 64, 256, 16, 4), "64x128": (64, 128, 256, 16, 8),
+              "128x128s": (128, 128, 128, 8, 16), "128x128": (128, 128, 64, 4, 0), "256x256": (256, 256, 64, 8, 0)}
+    widths = [N + 16 * i for i in range(n)]
+
+    def tiles(name):
+        bm, bn = builds[name][:2]
+        return sum(-(-M // bm) * -(-(w // 2 if fused else w) // (bn // 2 if fused else bn)) for w in widths)
+
+    def fits(name):     # two stages and the table of scales; where waves split K, their partial tiles over both
+        bm, bn, kc, waves, blocks = builds[name]
+        lds = 2 * (bm * kc * 2 + bn * kc // 2) + bn * (K // G) * 4
+        return K % kc == 0 and max(lds, waves * blocks * 1024) <= 160 * 1024
+
+    for name in ("32x64", "64x64", "64x128", "128x128s")[2 if fused else 0:]:
+        if fits(name) and tiles(name) <= cus:
+            return name
+    if fits("256x256") and tiles("256x256") * 100 >= -(-tiles("256x256") // cus) * cus * 85:
+        return "256x256"
+    return "128x128"
+
+
+def test_every_build_of_the_launch_has_a_case():
+    for *shape, build in CASES:
+        assert _build(*shape) == build, shape
+    reached = {(build, fused) for _, _, _, _, fused, _, build in CASES}
+    wide = {"64x128", "128x128s", "128x128", "256x256"}
+    assert reached == {(b, False) for b in wide | {"32x64", "64x64"}} | {(b, True) for b in wide}
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,G,fused,n", [
-    (33, 64, 256, 128, False, 1),       # 32x64 tiles, one row into the second
-    (64, 2048, 2048, 128, False, 1),
-    (65, 2050, 512, 32, False, 1),      # odd widths: narrow stores, a ragged last tile
-    (40, 17, 256, 64, False, 3),
-    (500, 2048, 256, 128, False, 1),    # 64x64 tiles
-    (512, 3000, 512, 64, False, 2),     # 64x128 and 128x128 tiles by tile count
-    (200, 2 * 1000, 256, 128, True, 1),
-    (129, 2 * 77, 512, 32, True, 1),
-    (33, 2 * 5632, 2048, 128, True, 1),
-    (300, 1000, 384, 128, False, 1),    # K not a multiple of 256: the tiles with shorter chunks
-    (130, 1000, 128, 128, False, 1),    # one chunk
-    (48, 96, 128, 32, True, 1),
-    (1664, 2048, 512, 128, False, 3),   # more tiles than CUs
-    (2047, 2 * 1500, 256, 256, True, 1),
-    (4100, 2 * 1700, 512, 64, True, 1), # 256x256 tiles, ragged both ways
-    (4090, 3500, 256, 128, False, 1),
-    (511, 16000, 384, 32, False, 2),
-    (70, 128, 4096, 32, False, 1),      # the largest tables of scales
-    (600, 2500, 5632, 32, False, 1),
-])
+@pytest.mark.parametrize("M,N,K,G,fused,n", [case[:6] for case in CASES])
 def test_prompt_gemm_matches_dequantised_product(M, N, K, G, fused, n):
     gen = torch.Generator().manual_seed(M + N + K)
     dev = torch.device("cuda:0")
@@ -101,6 +149,31 @@ def test_prompt_gemm_leaves_other_operands_to_the_general_route():
     big = _triple(gen, 16384, 40000, 32, dev)                                        # scales beyond LDS
     x = torch.randn(400, 16384, generator=gen).to(torch.bfloat16).to(dev)
     assert ops.int4_gemm(x, [big], 32) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [33, 600, 2048, 2049, 4095, 4096])
+def test_modules_match_float64_on_both_sides_of_every_line(rows):
+    """On the library's route gate and up are rounded to bf16 before SiLU: up to 2^-8 of each (eight significant bits,
+    so half a unit in the last place is 2^-8 of a value just above a power of two), through |silu'| < 1.1 and |silu|."""
+    gen, dev = torch.Generator().manual_seed(rows), torch.device("cuda:0")
+    bias = torch.randn(768, generator=gen).to(torch.bfloat16).to(dev)
+    triple = _triple(gen, 512, 768, 128, dev)
+    linear = Int4Linear.from_packed(*triple, 128, bias=bias)
+    halves = [_triple(gen, 512, 520, 64, dev) for _ in range(2)]
+    mlp = Int4GateUpSiLU(*(Int4Linear.from_packed(*t, 64) for t in halves))
+    x = torch.randn(1, rows, 512, generator=gen).to(torch.bfloat16).to(dev)
+    with torch.no_grad():
+        y, h = linear(x), mlp(x)
+    assert y.shape == (1, rows, 768) and h.shape == (1, rows, 520)
+    ref, tol = _reference(x[0], triple, 128, False)
+    ref = ref + bias.double()                              # the bias is added in bf16: a second rounding
+    assert bool(((y[0].double() - ref).abs() <= tol + 2.0 ** -8 * ref.abs() + 2.0 ** -8 * tol).all())
+    both = tuple(torch.cat(ts) for ts in zip(*halves))
+    ref, tol = _reference(x[0], both, 64, True)
+    g, u = _reference(x[0], both, 64, False)[0].chunk(2, 1)
+    tol = tol + 2.0 ** -8 * (1.1 * (g * u).abs() + torch.nn.functional.silu(g).abs() * u.abs()) * (1 + 2.0 ** -7)
+    assert bool(((h[0].double() - ref).abs() <= tol).all())
 
 
 @pytest.mark.gpu

@@ -4,6 +4,8 @@ The weight tile is bit-exact, so ``grad @ weight`` (the very call the node makes
 linear is looked at; the fused module's is float64, with three bf16 roundings in a row (2^-6).
 """
 
+import gc
+
 import pytest
 import torch
 from torch.utils.checkpoint import checkpoint
@@ -14,6 +16,13 @@ from visionrl_amd.linear import Int4GateUpSiLU, Int4Linear
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _groups_let_go():
+    """Grouped modules hold each other, and their GPU tensors, in cycles."""
+    yield
+    gc.collect()
 
 
 def _linear(gen, K, N, G=128, bias=False):

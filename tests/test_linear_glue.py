@@ -341,7 +341,7 @@ def test_grouped_siblings_hand_results_over_by_tensor_identity():
     other = x.clone() * 2
     assert torch.equal(k(other), alone[1](other))
     assert torch.equal(v(x), want[2])                    # v still takes what q handed it for x
-    # more rows than the plan-free launch takes: every module on its own
+    # more rows than the plan-free launch takes, and too narrow for the prompt launch: every module on its own
     big = torch.randn(40, 512, device=dev).to(torch.bfloat16)
     assert torch.equal(q(big), alone[0](big)) and k._handed is None
 
@@ -349,7 +349,8 @@ def test_grouped_siblings_hand_results_over_by_tensor_identity():
 @pytest.mark.gpu
 def test_prompt_sized_calls_go_through_the_library_gemm():
     """More than 32 rows (the prompt pass): bit-exact weight tile, then the library GEMM, for the plain
-    and the fused gate|up module, prepacked or not."""
+    and the fused gate|up module, prepacked or not (weights of fewer than 512 outputs; wider ones take the
+    prompt launch at most sizes, ``test_gpu_prompt_gemm``)."""
     import torch.nn.functional as F
 
     dev = "cuda:0"
@@ -380,7 +381,7 @@ def test_prompt_sized_calls_go_through_the_library_gemm():
 @pytest.mark.gpu
 def test_kept_dense_weight_serves_prompt_sized_calls_until_the_source_changes():
     """``keep_dense_()``: prompt-sized and gradient-carrying calls multiply by one kept bf16 tensor (the
-    same results, no dequantisation per call); a write to the canonical buffers makes the next call
+    same results at these widths, no dequantisation per call); a write to the canonical buffers makes the next call
     rebuild it; ``keep_dense_(False)`` drops it."""
     import torch.nn.functional as F
 
