@@ -320,7 +320,7 @@ class Int4Linear(nn.Module):
                         # (x by weak reference: with a gradient it would keep what led to it alive)
                         call = weakref.ref(x), version, ops._stream_handle(x.device), _capturing()
                         for m, ym, weight in zip(group[1:], ys[1:], weights[1:]):
-                            m.__dict__["_handed"] = (call, ym, weight, _versions(*weight))
+                            m.__dict__["_handed"] = (call, ym, [weakref.ref(t) for t in weight], _versions(*weight))
                         return ys[0]
         if not _launch_pays(M, K, self.out_features, G):
             return None
@@ -336,7 +336,7 @@ class Int4Linear(nn.Module):
                 capturing != _capturing() or grad and not _launchable(x):
             return None
         mine = self._canonical()
-        return y if mine[0] is qweight and mine[1] is scales and mine[2] is qzeros and \
+        return y if mine[0] is qweight() and mine[1] is scales() and mine[2] is qzeros() and \
             versions == _versions(*mine) else None
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
