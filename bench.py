@@ -495,8 +495,8 @@ def module_path(items, steps: int):
 
 def prompt_pass_linears(device, steps: int):
     """The linears of the prompt pass (vrl/models/families/janus_pro/policy.py:523, iteration 0: 2B x 256 rows)
-    through the int4 modules: one launch over the packed words per module up to 2048 rows (gate|up from 4096 on),
-    dequantised weight (bit-exact tile) and library GEMM otherwise; with ``keep_dense_()`` the bf16 tile is kept
+    through the int4 modules: one launch over the packed words per module where that is the faster route, dequantised
+    weight (bit-exact tile) and library GEMM otherwise; with ``keep_dense_()`` the bf16 tile is kept
     between calls.  Four layers' modules, milliseconds per
     24-layer pass (the measured four scaled by six), at 2 x 256 and 32 x 256 rows."""
     from visionrl_amd.linear import Int4GateUpSiLU, Int4Linear

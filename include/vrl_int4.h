@@ -20,7 +20,9 @@
  *   w[n,k] = bf16_rne( (float)(q[n,k] - z[n,k/G]) * (float)s[n,k/G] )   (bit-exact)
  *   y[m,n] = bf16_rne( sum_k (float)x[m,k] * w[n,k] )                   (fp32 accumulate,
  *                                                                        order unspecified)
- * Scales must be finite bf16 numbers; zero, negative and subnormal scales are allowed.
+ * Scales must be finite bf16 numbers; zero, negative and subnormal scales are allowed.  The products fold the
+ * zero-point into fp32 constants of up to 143 scales, so a scale of 2^120 or more in magnitude may give infinities
+ * or NaN there; the dequantised tile is exact for every finite scale.
  *
  * Every call only enqueues work on `hip_stream` (a hipStream_t, NULL = the
  * default stream) of the current device; it does not allocate, synchronise or

@@ -45,7 +45,7 @@ def test_abi_version_and_error_strings(lib):
 
 
 def test_problem_struct_matches_header():
-    # 5 pointers + 4 ints + flag + 3 reserved ints
+    # 5 pointers, 6 ints, a pointer that most calls leave null
     assert ctypes.sizeof(_lib.Problem) == 5 * 8 + 8 * 4
 
 

@@ -981,7 +981,9 @@ int vrl_int4_grouped_plan_build(const vrl_int4_problem *problems, int n_problems
         // more than a workgroup's share and the launch waits for it: then half as many tiles, which cost more
         // each (half the waves share a staging; three layers of 2048 x 5632 at 32 rows 42.7 against 32.0 us,
         // four at 24 rows 42.7 against 36.2; from a share of 5/8 of a piece on whole pieces are as good or
-        // better: 60.8 against 65.4 us for seven layers and the head at 24 rows).
+        // better: 60.8 against 65.4 us for seven layers and the head at 24 rows).  Both figures are from records of
+        // K = 5632; on layers of 1024 x 2816, 3072 x 8192 and 4096 x 11008 plans took 0.66 to 1.03 of the time they
+        // took with tile-by-tile ranges of whole pieces (the longest: four layers of 4096 and the head at 8 to 16 rows).
         int pass_cut = wpb;
         for (int i = 0; i < n_problems; ++i)
             if (in_passes(recs[i]) && wpb * tile_cost(recs[i]) > 1.6 * total_cost / (double)grid) pass_cut = wpb / 2;

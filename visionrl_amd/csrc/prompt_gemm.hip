@@ -1,6 +1,6 @@
 // Prompt-sized products over the canonical int4 operands: y[M,N] = x[M,K] . dequant(W)^T for more activation
 // rows than the GEMV launches take (the prompt pass, vrl/models/families/janus_pro/policy.py:640-672, and the
-// forward of a training replay, policy.py:419-424).
+// forward of a training replay, policy.py:419-424, which keeps gate||up itself beside the fused result).
 //
 // One launch covers up to GEMM_MAX problems (q|k|v of a layer; gate|up with the SiLU epilogue is one problem).
 // A workgroup owns BM activation rows x BN weight rows and walks K in chunks of KC.  Both operands reach LDS by
@@ -393,10 +393,16 @@ using Gemm256x256 = GemmCfg<1, 8, 1, 16, 2, 64, 2>;
 // The smallest tile whose launch is one round of workgroups: until the chip is full a launch takes as long as one
 // tile does, and a smaller tile is done sooner (K = 2048, one round: 7.7 / 9.5 / 14.0 / 21.0 us in the order
 // below; the waves split K, since a tile alone on its CU is bound by the latency of its own chain).  Beyond that
-// tiles whose waves split nothing: 256x256, every weight rebuilt once for 256 rows (1086 TFLOP/s for gate|up of
-// 8192 rows by 2048, against 975), where its rounds are at least 85 % full, 128x128 otherwise (gate|up of 1664
-// rows: 109 against 88 us; of 1280 rows: 62 against 76).  Measured at 48 to 8192 rows of q|k|v (3 x 2048),
-// o_proj, gate|up (11264) and down_proj (K = 5632): the choice is the best or within 5 % of it at every one.
+// tiles whose waves split nothing: 256x256, every weight rebuilt once for 256 rows (gate|up of 8192 rows by 2048:
+// 348 us alone, against 388; 373 to 395 between other work), where its rounds are at least 85 % full, 128x128
+// otherwise (gate|up of 1664 rows: 109 against 88 us; of 1280 rows: 62 against 76).  Measured at 48 to 8192 rows of
+// q|k|v (3 x 2048), o_proj, gate|up (11264) and down_proj (K = 5632): of these builds the choice is the best or within
+// 5 % of it at every one.  Not built: a 64 x 128 tile whose waves split K two ways, 7 % faster than the choice for
+// gate|up of 512 rows (36.6 against 39.3 us) and q|k|v of 1024 (38.1 against 40.8).
+//
+// From counters: the vector units are active in 43 to 72 % of the busy cycles of a CU, the matrix units in 11 (32x64)
+// to 55 % (256x256); the LDS in 17 to 35 %, of which 8 to 30 % are conflicts.  The large tile is bound by issuing to
+// the first two, the small ones by the latency of a tile's chain.
 template <bool FUSED>
 int dispatch_gemm(GemmArgs &args, hipStream_t stream) {
     const long cus = device_cu_count();

@@ -1,8 +1,8 @@
 // silu(gate) * up over the library product of a gate||up weight, and its gradient: the middle of LlamaMLP where
-// the product itself is the library's (prompts beyond the rows of vrl_int4_gemm_bf16, and the training replay,
-// policy.py:419-424).  Bound by memory: each value is read once and written once, 16 bytes per lane, where the
+// the product itself is the library's (prompts that vrl_int4_gemm_bf16 is not the faster form for), and in the
+// backward of every training replay (policy.py:419-424).  Bound by memory: each value is read once and written once, 16 bytes per lane, where the
 // separate tensor operations passed over halves and temporaries (1664 x 5632: 10.6 us, 5.3 TB/s, against
-// 14.6 + 11.8; its gradient 15.8 us, 7.1 TB/s, against 15.9 + 17.9 + 9.9 + 11.8).  All arithmetic in fp32, one
+// 14.6 + 11.8; its gradient 15.8 us, 5.9 TB/s, against 15.9 + 17.9 + 9.9 + 11.8).  All arithmetic in fp32, one
 // rounding per result.
 #include "host_checks.hpp"
 
