@@ -44,7 +44,7 @@ def _launch_pays(rows: int, K: int, columns: int, group_size: int, products: int
     """Whether one ``ops.int4_gemm`` launch beats rebuilding the weight and a library product per weight.
 
     Both routes were timed, queued back to back on the GPU, at 33 to 8192 rows, K of 1024 to 11008, up to 22016 weight
-    rows and groups of 32, 64 and 128.  The library's rate is 1.2 to 1.4 times the launch's once its products are
+    rows and groups of 32, 64 and 128.  The library's rate is 1.2 to 1.6 times the launch's once its products are
     large; what the launch saves is the pass that writes the weight, SiLU's pass and the launches of a group.  A group
     costs as much again for each halving of the group size below 128, in the table of scales of every tile: ``k``
     is the K of equal cost.
@@ -55,14 +55,15 @@ def _launch_pays(rows: int, K: int, columns: int, group_size: int, products: int
     if fused:
         # 2048 -> 2 x 5632: 44 against 52 us at 512 rows, 96 against 109 at 1792; 3072 -> 2 x 8192: 96 against 109 at
         # 1024, 165 against 155 at 1536; 4096 -> 2 x 11008: 83 against 102 at 256, 236 against 209 at 1024.  From
-        # FUSED_ROWS on a short K is faster again, for SiLU's pass (K = 2048: 193 against 192 us at 4096 rows, 373
-        # against 408 at 8192; K = 3072: 365 against 335 and 708 against 639).
+        # FUSED_ROWS on a short K is faster again on the whole, for SiLU's pass, where the library's time jumps with
+        # the rows (K = 2048: 0.69 to 1.19 of its time at twelve sizes up to 12288 rows, 0.97 in the mean, 373 against
+        # 408 us at 8192; K = 1024: 0.75 to 1.04, 0.88; K = 3072: 365 against 335 at 4096, 708 against 639 at 8192).
         return rows <= PROMPT_ROWS and work <= 48 << 30 or rows >= FUSED_ROWS and K <= 2048 and k <= 4096
     if rows > PROMPT_ROWS:
         return False
     tiles = lambda bm, bn: -(-rows // bm) * -(-columns // bn)
     if products > 1:
-        # q|k|v of 2048 / 3072 / 4096 outputs each: 61 / 108 / 207 us against 87 / 150 / 194 at 1664 rows (the last
+        # q|k|v of 2048 / 3072 / 4096 outputs each: 61 / 96 / 207 us against 87 / 136 / 194 at 1664 rows (the last
         # stays with the library), 26 / 64 / 84 against 63 / 93 / 120 at 512.  Beyond 80 groups only one workgroup
         # fits a CU and more than a round of them is slow (groups of 32, K = 4096: 56 against 98 us at 256 rows, one
         # round; 144 against 117 at 512).
