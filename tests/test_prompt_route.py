@@ -17,6 +17,8 @@ QKV, GATE_UP = dict(products=3), dict(fused=True)
     (256, 4096, 3 * 4096, 32, QKV, True),          # 56, 98
     (512, 4096, 3 * 4096, 32, QKV, False),         # 144, 117
     (512, 3072, 3 * 3072, 32, QKV, False),         # 109, 89
+    (256, 11008, 3 * 1024, 64, QKV, True),         # 46, 99: one round of 64 x 64 tiles
+    (512, 11008, 3 * 1024, 64, QKV, False),        # 147, 124: the tables of the builds of one round do not fit
     (2048, 2048, 2048, 128, {}, True),             # 26, 30
     (1024, 5632, 2048, 128, {}, True),             # 38, 46
     (1152, 5632, 2048, 128, {}, False),            # 58, 51

@@ -61,29 +61,29 @@ def _launch_pays(rows: int, K: int, columns: int, group_size: int, products: int
         return rows <= PROMPT_ROWS and work <= 48 << 30 or rows >= FUSED_ROWS and K <= 2048 and k <= 4096
     if rows > PROMPT_ROWS:
         return False
+    # one round of workgroups: of the builds that split K, as far as their tables of scales fit the LDS
     tiles = lambda bm, bn: -(-rows // bm) * -(-columns // bn)
+    small = any(groups <= most and tiles(bm, bn) <= CUS for bm, bn, most in ((32, 64, 448), (64, 64, 320), (64, 128, 128)))
+    wide = groups <= 160 and tiles(128, 128) <= CUS
     if products > 1:
         # q|k|v of 2048 / 3072 / 4096 outputs each: 61 / 96 / 207 us against 87 / 136 / 194 at 1664 rows (the last
         # stays with the library), 26 / 64 / 84 against 63 / 93 / 120 at 512.  Beyond 80 groups only one workgroup
         # fits a CU and more than a round of them is slow (groups of 32, K = 4096: 56 against 98 us at 256 rows, one
         # round; 144 against 117 at 512).
-        return work < 72 << 30 if groups <= 80 else tiles(128, 128) <= CUS
-    # One weight: worth it while its tiles are one round of workgroups of the builds that split K (5632 -> 2048: 38
-    # against 46 us at 1024 rows, 58 against 51 at 1152; 11008 -> 4096: 67 against 85 at 512, 110 against 94 at 768),
-    # as far as their tables fit.  Beyond that with two of: one round of 128 x 128 tiles, a short K, few rows
-    # (2048 -> 2048: 26 against 30 us at 2048 rows; 4096 -> 16384: 48 against 76 at 256; 2048 -> 16384: 48 against 54
-    # at 512; 4096 -> 4096: 45 against 42 at 768, where only the first holds).
-    for bm, bn, most in ((32, 64, 448), (64, 64, 320), (64, 128, 128)):
-        if groups <= most and tiles(bm, bn) <= CUS:
-            return True
-    return (groups <= 160 and tiles(128, 128) <= CUS) + (k <= 3072) + (rows <= 512) >= 2
+        return work < 72 << 30 if groups <= 80 else small or wide
+    # One weight: worth it while its tiles are one round up to 64 x 128 (5632 -> 2048: 38 against 46 us at 1024 rows,
+    # 58 against 51 at 1152; 11008 -> 4096: 67 against 85 at 512, 110 against 94 at 768).  Beyond that with two of: one
+    # round of 128 x 128 tiles, a short K, few rows (2048 -> 2048: 26 against 30 us at 2048 rows; 4096 -> 16384: 48
+    # against 76 at 256; 2048 -> 16384: 48 against 54 at 512; 4096 -> 4096: 45 against 42 at 768, where only the first
+    # holds).
+    return small or wide + (k <= 3072) + (rows <= 512) >= 2
 
 
 _PLAIN = (torch.Tensor, nn.Parameter)
 
 
 def _wants_grad(x: torch.Tensor) -> bool:
-    """The HIP launches are not recorded by autograd: such calls take the dequant + GEMM route."""
+    """Whether autograd records the call: the HIP launches are not recorded by themselves."""
     return torch.is_grad_enabled() and x.requires_grad
 
 
