@@ -189,3 +189,23 @@ def test_a_default_device_changes_no_route(launches):
         assert torch.equal(y, want[1])
         y.float().sum().backward()
     assert xg.grad.device == x.device
+
+
+@pytest.mark.parametrize("rows", [64, 600])
+def test_a_kept_dense_weight_means_library_products(rows, launches):
+    """With and without a gradient, at widths where a module without the copy takes the launch."""
+    gen, (q, k, v, o, mlp) = _layer(7)
+    x = _input(gen, rows, 512)
+    with torch.no_grad():
+        o(x), mlp(x)
+        assert launches == [1, 1]
+        o.keep_dense_(), mlp.keep_dense_()
+        dense = torch.nn.functional.linear(x, o.dequantize())
+        fused = ops.silu_mul(torch.nn.functional.linear(x, ops.int4_dequant(*mlp._canonical(), 128)))
+        assert torch.equal(o(x), dense) and torch.equal(mlp(x), fused)
+        k.keep_dense_()                                    # one of a group: every member on its own
+        q(x), v(x)
+        assert torch.equal(k(x), torch.nn.functional.linear(x, k.dequantize()))
+    assert launches == [1, 1, 1, 1]
+    xg = x.clone().requires_grad_()
+    assert torch.equal(o(xg), dense) and torch.equal(mlp(xg), fused) and launches == [1, 1, 1, 1]
