@@ -231,6 +231,51 @@ typedef struct vrl_step_call {
 
 int vrl_decode_run_calls(const vrl_step_call *calls, int n_calls, int *failed_at, void *hip_stream);
 
+/*
+ * A whole decode step of a Llama trunk in one launch (decode_trunk.hip): for one new token per row, every layer's
+ * norm, q|k|v, rotary + cache append + attention, o_proj + residual, norm, gate|up + SiLU, down_proj + residual,
+ * and the model's norm.  Results are those of the entry points above called one after another, bit for bit.  The
+ * launch is cooperative, one workgroup per compute unit, and may be captured into a graph.
+ *   layers    n_layers records in DEVICE memory, 16-byte aligned; weights prepacked (vrl_int4_prepack, G = 128),
+ *             gate_up one blob of 2 * inter rows, norms bf16 [hidden], caches as for vrl_rope_attn_decode_bf16
+ *   x         bf16 [M, hidden]: the new tokens' embeddings (read only)
+ *   mask, cos, sin, position  as for vrl_rope_attn_decode_bf16; position_per_row: int64 [M], one slot per row.
+ *             A row whose position lies outside [0, L_max) appends nothing and attends to nothing.
+ *   split_from  filled slots from which the attention's order of sums is that of vrl_rope_attn_decode_split_bf16
+ *             with this split_from (its ranges); 0: that of vrl_rope_attn_decode_bf16.  Order only, not work.
+ *   normed    bf16 [M, hidden] or NULL: norm(h) under `norm`, `eps`;  h_out  bf16 [M, hidden] or NULL: h itself
+ *   workspace vrl_decode_trunk_workspace_bytes() bytes of device memory, 256-byte aligned, zero before the first
+ *             launch that uses it and left to the launches from then on.  Launches that share one must be ordered.
+ *   wait_limit  0, or how often a wave looks for a result of another workgroup in vain before it takes NaN for it
+ *             and waits no more (default 2^22): every wait ends, and a launch that gave up has NaN in its output.
+ *             Its workspace has to be zeroed before the next launch.
+ * vrl_decode_trunk_workspace_bytes returns 0 where the launch does not apply (the other fields may then be NULL).
+ * It applies to M <= 4, hidden 2048, head_dim 128, group_size 128, L_max <= 8192, n_heads * 128 a multiple of 256
+ * up to 8192, inter a multiple of 256 up to 8192, where the launches above would add up the norms in one of the
+ * orders that were built, on a device of at least 128 compute units with cooperative launches.
+ */
+typedef struct vrl_trunk_layer {
+    const void *q, *k, *v, *o, *gate_up, *down;   /* prepacked blobs */
+    const void *norm1, *norm2;
+    void *k_cache, *v_cache;
+    float eps1, eps2, scaling;
+    int32_t reserved;
+} vrl_trunk_layer;
+
+typedef struct vrl_trunk {
+    const vrl_trunk_layer *layers;
+    const void *x, *mask, *cos, *sin, *norm;
+    const int64_t *position;
+    void *normed, *h_out, *workspace;
+    size_t workspace_bytes;
+    int32_t n_layers, M, hidden, inter, n_heads, n_kv_heads, head_dim, group_size, L_max, position_per_row, split_from;
+    float eps;
+    uint32_t wait_limit;
+} vrl_trunk;
+
+size_t vrl_decode_trunk_workspace_bytes(const vrl_trunk *trunk);
+int vrl_decode_trunk_bf16(const vrl_trunk *trunk, void *hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

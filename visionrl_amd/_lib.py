@@ -49,6 +49,8 @@ SYMBOLS = (
     "vrl_int4_gemv_prepacked_lora_up_bf16",
     "vrl_decode_run_calls",
     "vrl_int4_gemv_prepacked_norm_lora_bf16",
+    "vrl_decode_trunk_workspace_bytes",
+    "vrl_decode_trunk_bf16",
 )
 
 
@@ -203,6 +205,25 @@ class AttnLora(ctypes.Structure):
     ]
 
 
+class TrunkLayer(ctypes.Structure):
+    """Mirror of ``vrl_trunk_layer``: a record of the array in device memory."""
+
+    _fields_ = [(name, ctypes.c_void_p) for name in ("q", "k", "v", "o", "gate_up", "down", "norm1", "norm2",
+                                                     "k_cache", "v_cache")] + \
+        [("eps1", ctypes.c_float), ("eps2", ctypes.c_float), ("scaling", ctypes.c_float), ("reserved", ctypes.c_int32)]
+
+
+class Trunk(ctypes.Structure):
+    """Mirror of ``vrl_trunk``."""
+
+    _fields_ = [(name, ctypes.c_void_p) for name in ("layers", "x", "mask", "cos", "sin", "norm", "position", "normed",
+                                                     "h_out", "workspace")] + \
+        [("workspace_bytes", ctypes.c_size_t)] + \
+        [(name, ctypes.c_int32) for name in ("n_layers", "M", "hidden", "inter", "n_heads", "n_kv_heads", "head_dim",
+                                             "group_size", "L_max", "position_per_row", "split_from")] + \
+        [("eps", ctypes.c_float), ("wait_limit", ctypes.c_uint32)]
+
+
 class PlanInfo(ctypes.Structure):
     """Mirror of ``vrl_int4_plan_info``."""
 
@@ -295,6 +316,10 @@ def _bind(lib):
                                                            ctypes.POINTER(LoraAdapter), ci, vp, vp]
     lib.vrl_decode_run_calls.argtypes = [ctypes.POINTER(StepCall), ci, ctypes.POINTER(ctypes.c_int), vp]
     lib.vrl_decode_run_calls.restype = ci
+    lib.vrl_decode_trunk_workspace_bytes.restype = ctypes.c_size_t
+    lib.vrl_decode_trunk_workspace_bytes.argtypes = [ctypes.POINTER(Trunk)]
+    lib.vrl_decode_trunk_bf16.restype = ci
+    lib.vrl_decode_trunk_bf16.argtypes = [ctypes.POINTER(Trunk), vp]
     lib.vrl_rope_attn_decode_split_workspace_bytes.argtypes = [ci, ci, ci]
     lib.vrl_rope_attn_decode_split_bf16.restype = ci
     lib.vrl_rope_attn_decode_split_bf16.argtypes = [vp, vp, vp, ci, ci, vp, vp, vp, vp, vp, vp, vp,

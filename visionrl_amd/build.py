@@ -22,7 +22,7 @@ LIB_NAME = "libvrl_int4.so"
 LIB_PATH = os.path.join(CSRC, LIB_NAME)
 BENCH_LIB_PATH = os.path.join(CSRC, "libvrl_bench.so")
 SOURCES = ["int4_gemv.hip", "cfg_sample.hip", "decode_layer.hip", "head_sample.hip", "prompt_gemm.hip",
-           "silu_mul.hip"]
+           "silu_mul.hip", "decode_trunk.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
 
 HIPCC_FLAGS = [

@@ -18,6 +18,10 @@ slot of the new token held in device memory, and every buffer preallocated, so t
 step can be recorded as one HIP graph.  Arithmetic follows the library's roundings (each tensor
 op in fp32, rounded to bf16); the attention keeps its probabilities in fp32.
 
+Where rows are few enough for the launch boundaries to be most of that (up to 4 rows of 2048 values,
+no adapters), the whole list is one launch with the same bits: workgroups that stay for the step and
+hand their results to each other through memory (``vrl_decode_trunk_bf16``).
+
 Needs a trunk whose projections were swapped for prepacked :class:`Int4Linear` modules with the
 fused MLP (``apply_int4_to_policy`` defaults).  Attention projections may carry one active LoRA
 adapter each (the reference's default, ``policy.py:81-88``, ``:298-324``): their layer then takes
@@ -414,6 +418,55 @@ class NativeDecodeTrunk:
                 self._calls_short[at] = call
             self._table_short = _lib.step_calls(self._calls_short)
         self._failed_at = ctypes.c_int(-1)
+        self._trunk = self._one_launch(trunk, cache, cur, mask, slot, H, Hkv, D)
+
+    def _one_launch(self, trunk, cache, cur, mask, slot, H: int, Hkv: int, D: int):
+        """The step as one launch: arguments of ``vrl_decode_trunk_bf16`` for its default and its short form, or
+        ``None`` where the list is what runs (adapters, more rows or other shapes than the launch takes)."""
+        records = (_lib.TrunkLayer * len(trunk.layers))()
+        inter = None
+        for i, (record, layer) in enumerate(zip(records, trunk.layers)):
+            attn, mlp = layer.self_attn, layer.mlp
+            proj = [_projection(getattr(attn, n), n) for n in ("q_proj", "k_proj", "v_proj", "o_proj")]
+            weights = [w for w, _ in proj] + [mlp.gate_up._packed, mlp.down_proj._packed]
+            inter = weights[5].K if inter is None else inter
+            shapes = [(H * D, self.hidden), (Hkv * D, self.hidden), (Hkv * D, self.hidden), (self.hidden, H * D),
+                      (2 * inter, self.hidden), (self.hidden, inter)]
+            if any(adapter is not None for _, adapter in proj) or [(w.N, w.K) for w in weights] != shapes or \
+                    any(w.group_size != 128 for w in weights):
+                return None
+            norms = layer.input_layernorm, layer.post_attention_layernorm
+            for name, t in zip(("q", "k", "v", "o", "gate_up", "down", "norm1", "norm2", "k_cache", "v_cache"),
+                               (*(w.blob for w in weights), *(n.weight.data for n in norms), cache.layers[i].keys,
+                                cache.layers[i].values)):
+                self._keep.append(t)
+                setattr(record, name, t.data_ptr())
+            record.eps1, record.eps2 = (float(n.variance_epsilon) for n in norms)
+            record.scaling = float(attn.scaling)
+        desc = _lib.Trunk(n_layers=len(records), M=self.rows, hidden=self.hidden, inter=inter, n_heads=H,
+                          n_kv_heads=Hkv, head_dim=D, group_size=128, L_max=self.max_len,
+                          position_per_row=int(slot.numel() != 1),
+                          split_from=self._split_from if self._split_ws is not None else 0)
+        lib = _lib.load()
+        with ops._on(self.device):
+            nbytes = lib.vrl_decode_trunk_workspace_bytes(ctypes.byref(desc))
+        if nbytes == 0:
+            return None
+        table = torch.frombuffer(bytearray(records), dtype=torch.uint8).to(self.device)
+        workspace = torch.zeros(nbytes, dtype=torch.uint8, device=self.device)
+        norm = trunk.norm.weight.data
+        self._keep += [table, workspace, norm]
+        for name, t in zip(("layers", "x", "mask", "cos", "sin", "norm", "position", "workspace"),
+                           (table, cur, mask, self.cos, self.sin, norm, slot, workspace)):
+            setattr(desc, name, t.data_ptr())
+        desc.workspace_bytes, desc.eps = nbytes, float(trunk.norm.variance_epsilon)
+        if self.normed is not None:
+            desc.normed = self.normed.data_ptr()
+        else:
+            desc.h_out = self.final[0].data_ptr()
+        short = _lib.Trunk.from_buffer_copy(desc)
+        short.split_from = 0
+        return desc, short
 
     def short_form(self, cached_slots: int) -> bool:
         """Whether :meth:`run` has a launch list of its own for a step that finds ``cached_slots`` filled slots
@@ -427,6 +480,11 @@ class NativeDecodeTrunk:
         form begins at; the results are those of the default list either way, up to the order of fp32 sums)."""
         stream = ops._stream_handle(self.device)
         short = short and self._table_short is not None
+        if self._trunk is not None:
+            with ops._on(self.device):
+                rc = _lib.load().vrl_decode_trunk_bf16(ctypes.byref(self._trunk[short]), stream)
+            _lib.check(rc, "vrl_decode_trunk_bf16")
+            return self.normed
         table, calls = (self._table_short, self._calls_short) if short else (self._table, self._calls)
         with ops._on(self.device):
             rc = _lib.load().vrl_decode_run_calls(table, len(table), ctypes.byref(self._failed_at), stream)
