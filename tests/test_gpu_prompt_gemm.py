@@ -46,19 +46,19 @@ def _reference(x, triple, G, fused):
 
 # M, N, K, G, fused, n, and the tile whose build the launch takes for them at 256 CUs ("s": waves split K)
 CASES = [
-    (33, 64, 256, 128, False, 1, "32x64"),          # one row into the second tile
-    (64, 2048, 2048, 128, False, 1, "32x64"),
-    (65, 2050, 512, 32, False, 1, "32x64"),         # odd widths: narrow stores, a ragged last tile
-    (40, 17, 256, 64, False, 3, "32x64"),
-    (70, 128, 4096, 32, False, 1, "32x64"),         # the largest tables of scales
+    (33, 64, 256, 128, False, 1, "32x64k"),          # one row into the second tile
+    (64, 2048, 2048, 128, False, 1, "32x32"),
+    (65, 2050, 512, 32, False, 1, "32x32"),         # odd widths: narrow stores, a ragged last tile
+    (40, 17, 256, 64, False, 3, "32x64k"),
+    (70, 128, 4096, 32, False, 1, "32x32"),         # the largest tables of scales
     (500, 2048, 256, 128, False, 1, "64x64"),
     (600, 1537, 512, 64, False, 1, "64x64"),
     (300, 2048, 2048, 128, False, 3, "64x128"),
     (500, 3001, 512, 32, False, 1, "64x128"),
     (257, 2047, 256, 256, False, 3, "64x128"),
-    (200, 2 * 1000, 256, 128, True, 1, "64x128"),
-    (129, 2 * 77, 512, 32, True, 1, "64x128"),
-    (33, 2 * 5632, 2048, 128, True, 1, "64x128"),
+    (200, 2 * 1000, 256, 128, True, 1, "64x64"),
+    (129, 2 * 77, 512, 32, True, 1, "32x64"),
+    (33, 2 * 5632, 2048, 128, True, 1, "64x64"),
     (512, 3000, 512, 64, False, 2, "128x128s"),
     (300, 1000, 384, 128, False, 1, "128x128s"),    # K not a multiple of 256: the tiles with shorter chunks
     (130, 1000, 128, 128, False, 1, "128x128s"),    # one chunk
@@ -66,6 +66,14 @@ CASES = [
     (1664, 2048, 512, 128, False, 3, "128x128"),    # more tiles than CUs
     (600, 2500, 5632, 32, False, 1, "128x128"),     # the other builds' tables do not fit
     (2047, 2 * 1500, 256, 256, True, 1, "128x128"),
+    (160, 2047, 1024, 128, False, 1, "32x64"),
+    (150, 1000, 512, 64, False, 3, "32x64"),        # one chunk
+    (129, 2 * 4001, 256, 128, True, 1, "64x128"),
+    (40, 100, 11264, 32, False, 1, "32x32"),        # tables that leave room for two chunks only
+    (160, 2048, 5632, 32, False, 1, "32x64"),
+    (45, 2 * 100, 5632, 32, True, 1, "32x64"),
+    (512, 2048, 5632, 32, False, 1, "64x64"),
+    (64, 2 * 5632, 5632, 32, True, 1, "64x64"),
     (4100, 2 * 1700, 512, 64, True, 1, "256x256"),  # ragged both ways
     (4090, 3500, 256, 128, False, 1, "256x256"),
     (511, 16000, 384, 32, False, 2, "256x256"),
@@ -74,7 +82,8 @@ CASES = [
 
 def _build(M, N, K, G, fused, n, cus=256):
     """The library's choice of tile, restated: rows and columns, chunk of K, waves, blocks of 16 x 16 per wave."""
-    builds = {"32x64": (32, 64, 256, 8, 2), "64x64": (64, 64, 256, 16, 4), "64x128": (64, 128, 256, 16, 8),
+    builds = {"32x32": (32, 32, 512, 16, 2), "32x64": (32, 64, 512, 16, 4), "32x64k": (32, 64, 256, 8, 2),
+              "64x64": (64, 64, 256, 8, 8) if fused else (64, 64, 256, 16, 4), "64x128": (64, 128, 256, 16, 8),
               "128x128s": (128, 128, 128, 8, 16), "128x128": (128, 128, 64, 4, 0), "256x256": (256, 256, 64, 8, 0)}
     widths = [N + 16 * i for i in range(n)]
 
@@ -82,12 +91,12 @@ def _build(M, N, K, G, fused, n, cus=256):
         bm, bn = builds[name][:2]
         return sum(-(-M // bm) * -(-(w // 2 if fused else w) // (bn // 2 if fused else bn)) for w in widths)
 
-    def fits(name):     # two stages and the table of scales; where waves split K, their partial tiles over both
+    def fits(name):     # two chunks at least and the table of scales; where waves split K, their partial tiles over both
         bm, bn, kc, waves, blocks = builds[name]
         lds = 2 * (bm * kc * 2 + bn * kc // 2) + bn * (K // G) * 4
         return K % kc == 0 and max(lds, waves * blocks * 1024) <= 160 * 1024
 
-    for name in ("32x64", "64x64", "64x128", "128x128s")[2 if fused else 0:]:
+    for name in (["32x64"] if fused else ["32x32", "32x64", "32x64k"]) + ["64x64", "64x128", "128x128s"]:
         if fits(name) and tiles(name) <= cus:
             return name
     if fits("256x256") and tiles("256x256") * 100 >= -(-tiles("256x256") // cus) * cus * 85:
@@ -99,8 +108,8 @@ def test_every_build_of_the_launch_has_a_case():
     for *shape, build in CASES:
         assert _build(*shape) == build, shape
     reached = {(build, fused) for _, _, _, _, fused, _, build in CASES}
-    wide = {"64x128", "128x128s", "128x128", "256x256"}
-    assert reached == {(b, False) for b in wide | {"32x64", "64x64"}} | {(b, True) for b in wide}
+    both = {"32x64", "64x64", "64x128", "128x128s", "128x128", "256x256"}
+    assert reached == {(b, False) for b in both | {"32x32", "32x64k"}} | {(b, True) for b in both}
 
 
 @pytest.mark.gpu
@@ -117,6 +126,43 @@ def test_prompt_gemm_matches_dequantised_product(M, N, K, G, fused, n):
         ref, tol = _reference(x, t, G, fused)
         assert y.shape == ref.shape and torch.equal(y, y2)
         assert bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,N,G,tile", [(256, 300, 32, "32x64k"), (256, 2000, 32, "64x64"), (512, 800, 128, "32x64"), (512, 4000, 128, "64x128"), (384, 2000, 64, "128x128s"),
+                                        (2048, 9000, 128, "128x128"), (7680, 4500, 32, "128x128")])
+@pytest.mark.parametrize("largest", [116, 123])   # scales below 2^117 take the plain rebuild, a larger one the other
+def test_prompt_gemm_weights_over_the_range_of_scales(K, N, G, tile, largest):
+    """Rows with a single one give the weights themselves: the bits of the dequantised tile, at scales of every exponent
+    (15 * 1.98 * 2^123 is still one that a bf16 holds).  K = 7680 in groups of 32: the table fills LDS, the other form."""
+    gen = torch.Generator().manual_seed(K + N + largest)
+    dev, M = torch.device("cuda:0"), 512
+    assert _build(M, N, K, G, False, 1) == tile
+    qw, _, qz = _triple(gen, K, N, G, dev)
+    exponents = torch.randint(-126, 101, (N, K // G), generator=gen)
+    exponents[N // 2:N // 2 + 3] = largest
+    scales = torch.ldexp((1 + 0.98 * torch.rand(N, K // G, generator=gen)) * (1 - 2 * torch.randint(0, 2, (N, K // G), generator=gen)),
+                         exponents).to(torch.bfloat16).to(dev)
+    at = torch.randint(0, K, (M,), generator=gen)
+    x = torch.zeros(M, K, dtype=torch.bfloat16)
+    x[torch.arange(M), at] = 1
+    (y,) = ops.int4_gemm(x.to(dev), [(qw, scales, qz)], G, False)
+    assert torch.equal(y, ops.int4_dequant(qw, scales, qz, G)[:, at.to(dev)].T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_prompt_gemm_scales_that_are_no_numbers(bad):
+    """They make their own output column no number, and no other."""
+    gen = torch.Generator().manual_seed(11)
+    dev, K, N = torch.device("cuda:0"), 512, 700
+    qw, scales, qz = _triple(gen, K, N, 128, dev)
+    x = torch.randn(100, K, generator=gen).to(torch.bfloat16).to(dev)
+    (clean,) = ops.int4_gemm(x, [(qw, scales, qz)], 128, False)
+    scales[333, 1] = bad
+    (y,) = ops.int4_gemm(x, [(qw, scales, qz)], 128, False)
+    keep = torch.arange(N, device=dev) != 333
+    assert bool(y[:, 333].isnan().all()) and torch.equal(y[:, keep], clean[:, keep])
 
 
 @pytest.mark.gpu

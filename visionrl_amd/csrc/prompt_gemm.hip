@@ -15,6 +15,7 @@
 // permute the global addresses instead of the LDS side, which they fill in lane order.  Scales and zero-points of
 // all of K are laid down once per workgroup as one word each.
 #include <atomic>
+#include <type_traits>
 
 #include "canonical.hpp"
 #include "host_checks.hpp"
@@ -39,43 +40,76 @@ struct GemmRec {
 struct GemmArgs {
     GemmRec recs[GEMM_MAX];
     int32_t n, K, gshift, tiles;   // every record shares K and the group size 1 << gshift
+    int32_t wave_flags;            // there is LDS behind the table for a word per wave
 };
 
-// One packed word -> eight exactly rounded bf16 weights in k order.  float(q) by the byte converter, then
-// fma(q, s, -z s): both products are exact (4 by 8 bits), so the sum is the exact (q - z) s and the conversion
-// is the one rounding of the contract.  23 plain instructions that can be issued between MFMAs, pair by pair,
-// against 19 of the GEMV kernels' asm block, which cannot be split.
-struct ScaleZero { float s, zs; };
+// One packed word -> eight exactly rounded bf16 weights in k order, in instructions that can be issued between MFMAs, pair by
+// pair: (q - z) s as fma(q', s', c) with an exact product and an exact c, so that the conversion is the one rounding of the
+// contract.  Two forms.  Plain: a nibble under the exponent of 1024 is the half-precision value 1024 + q, or 1024 + 16 q where
+// it sits four bits further up, which the mixed fma takes as it is: 17 instructions.
+// Its c, -(1024 + z) s, is finite for
+// scales below 2^117; a workgroup that meets a larger one (an infinity, a NaN) takes the wide form for all of its tile, the
+// byte converter's float(q) and c = -z s: 23 instructions, the only form before
+// (prompt of 512 rows, four layers: 414 -> 399 us from this alone).
+struct ScaleZero { float s, c, s16, c16; };
+struct Nibbles { uint32_t h[4]; };
+struct Masks { uint32_t low, high, bias; };
+constexpr uint32_t WIDE_SCALE = 0x7A00u;   // bf16 bits of 2^117
 
-__device__ __forceinline__ ScaleZero scale_zero(uint32_t meta) {   // (scale bits << 16) | zero
-    const float s = bf16_bits_to_f32(meta >> 16);
-    return {s, -s * (float)(meta & 0xFFu)};
+__device__ __forceinline__ float half_of(uint32_t v, int i) {
+    typedef __attribute__((ext_vector_type(2))) _Float16 half2_t;
+    return (float)__builtin_bit_cast(half2_t, v)[i];
 }
 
-struct Nibbles { uint32_t even, odd; };
+template <bool WIDE>
+__device__ __forceinline__ ScaleZero scale_zero(uint32_t meta) {   // (scale bits << 16) | half-precision 1024 + zero
+    const float s = bf16_bits_to_f32(meta >> 16);
+    if constexpr (WIDE) return {s, -s * (float)(meta & 0xFFu), 0.0f, 0.0f};
+    const float c = -half_of(meta, 0) * s;
+    return {s, c, s * 0.0625f, __builtin_fmaf(960.0f, s, c)};
+}
 
-__device__ __forceinline__ Nibbles nibbles(uint32_t v) {
-    Nibbles b{v & 0x0F0F0F0Fu, (v >> 4) & 0x0F0F0F0Fu};
-    asm("" : "+v"(b.even), "+v"(b.odd));   // or the compiler takes every nibble out by itself: 28 instructions
+template <bool WIDE>
+__device__ __forceinline__ Nibbles nibbles(uint32_t v, const Masks &m) {
+    if constexpr (WIDE) {
+        Nibbles b{{v & 0x0F0F0F0Fu, (v >> 4) & 0x0F0F0F0Fu, 0u, 0u}};
+        asm("" : "+v"(b.h[0]), "+v"(b.h[1]));   // or the compiler takes every nibble out by itself: 28 instructions
+        return b;
+    }
+    const uint32_t w = v >> 8;
+    Nibbles b{{(v & m.low) | m.bias, (v & m.high) | m.bias, (w & m.low) | m.bias, (w & m.high) | m.bias}};
+    asm("" : "+v"(b.h[0]), "+v"(b.h[1]), "+v"(b.h[2]), "+v"(b.h[3]));   // or half of the and-ors come apart again
     return b;
 }
 
+template <bool WIDE>
 __device__ __forceinline__ uint32_t dequant_pair(const Nibbles &b, int i, const ScaleZero &c) {
-    return pack_bf16_rne(__builtin_fmaf((float)((b.even >> (8 * i)) & 0xFFu), c.s, c.zs),
-                         __builtin_fmaf((float)((b.odd >> (8 * i)) & 0xFFu), c.s, c.zs));
+    if constexpr (WIDE)
+        return pack_bf16_rne(__builtin_fmaf((float)((b.h[0] >> (8 * i)) & 0xFFu), c.s, c.c),
+                             __builtin_fmaf((float)((b.h[1] >> (8 * i)) & 0xFFu), c.s, c.c));
+    return pack_bf16_rne(__builtin_fmaf(half_of(b.h[i % 2 * 2], i / 2), c.s, c.c),
+                         __builtin_fmaf(half_of(b.h[i % 2 * 2 + 1], i / 2), c.s16, c.c16));
 }
 
-// 16 bytes per lane from global memory to LDS at `lds` + 16 * lane; counted by vmcnt, touches no register.
-__device__ __forceinline__ void dma16(uint8_t *lds, const uint8_t *g) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(uintptr_t)g,
-                                     (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
+// 16 bytes per lane from global memory (base + off, 32 bits) to LDS at `lds` + 16 * lane; counted by vmcnt, touches no
+// register.  In assembly: the compiler takes the builtin for an access of both counters and from then on waits for every
+// outstanding LDS read where it needs the first, once per MFMA step.  What orders these loads against the LDS reads are the
+// waits and barriers of the kernel, as with the builtin.  (m0 is not allocated; nothing else here uses it.)
+__device__ __forceinline__ void dma16(uint8_t *lds, const uint8_t *base, uint32_t off) {
+    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base));
 }
 
 // WM x WN x WK waves share a tile: WM and WN split its rows and columns, WK the k of every chunk (their partial
 // tiles meet in LDS at the end).  A wave owns MB x NB blocks of 16 x 16.  S chunks of KC k are in LDS at a time.
-template <int WM_, int WN_, int WK_, int MB_, int NB_, int KC_, int S_>
+// AHEAD: a chunk's barrier stands inside the last MFMA step of the chunk before it, whose remaining products cover the
+// round trip for the next words and activations and the rebuild of the first weights; otherwise at the chunk's start.
+// Tiles of 128 rows and more have the products for that: 1664 rows, K = 2048, gate|up 88.6 -> 82.2 us, q|k|v 54.7 -> 50.3,
+// down_proj 51.0 -> 46.0, of which the plain rebuild and precise waits give 5.2, 3.0 and 2.4.  With 64 rows it costs 5 %.
+template <int WM_, int WN_, int WK_, int MB_, int NB_, int KC_, int S_, bool AHEAD_>
 struct GemmCfg {
     static constexpr int WM = WM_, WN = WN_, WK = WK_, MB = MB_, NB = NB_, KC = KC_, S = S_;
+    static constexpr bool AHEAD = AHEAD_;
     static constexpr int WAVES = WM * WN * WK, THREADS = WAVES * WAVE;
     static constexpr int BM = 16 * MB * WM, BN = 16 * NB * WN;
     static constexpr int T = KC / 32 / WK;                // MFMA steps per wave and chunk = packed words a lane reads per row
@@ -87,7 +121,7 @@ struct GemmCfg {
     static constexpr int STAGE = X_BYTES + W_BYTES;
     static_assert(X_BYTES % (1024 * WAVES) == 0 && (WAVES % W_UNITS == 0 || W_UNITS % WAVES == 0), "whole direct loads");
     static_assert(T == 2 || T == 4, "a lane's words are one 8- or 16-byte read, inside one group of 32 k");
-    static_assert(MB % WK == 0, "the waves that split K finish a share of the row blocks each");
+    static_assert(MB % WK == 0 || WK % MB == 0, "the waves that split K finish a share of the row blocks each, or none");
     static constexpr size_t PARTIAL = WK > 1 ? (size_t)WAVES * MB * NB * 1024 : 0;   // over the stages, once they are done
     static constexpr size_t lds(int groups) {
         const size_t loop = (size_t)S * STAGE + (size_t)BN * groups * 4;
@@ -108,7 +142,7 @@ __device__ __forceinline__ int activation_swizzle(int r) {
 }
 template <int P>
 __device__ __forceinline__ int weight_swizzle(int r) {
-    return P == 2 ? r >> 3 & 1 : P == 4 ? -(r >> 2) & 3 : r >> 1 & 7;
+    return P == 2 ? r >> 3 & 1 : P == 4 ? -(r >> 2) & 3 : P == 8 ? r >> 1 & 7 : r & 15;
 }
 
 // The weight row behind local row r of column tile nt.  Fused records: a wave's first NB/2 blocks of 16 rows are
@@ -176,21 +210,30 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 || C::MB * C::NB >= 32 ? 
         uint8_t *xl = smem + slot * C::STAGE + wave * (C::X_LOADS * 1024);
         uint8_t *wl = smem + slot * C::STAGE + C::X_BYTES + wave * C::W_LOADS % C::W_UNITS * 1024;
 #pragma unroll
-        for (int i = 0; i < C::X_LOADS; ++i) dma16(xl + i * 1024, xc + xsrc[i]);
+        for (int i = 0; i < C::X_LOADS; ++i) dma16(xl + i * 1024, xc, xsrc[i]);
 #pragma unroll
-        for (int i = 0; i < C::W_LOADS; ++i) dma16(wl + i * 1024, wc + wsrc[i]);
+        for (int i = 0; i < C::W_LOADS; ++i) dma16(wl + i * 1024, wc, wsrc[i]);
     };
 
     // scales and zero-points of the tile's rows, (scale bits << 16) | zero, group-major
+    bool wide_scales = args.wave_flags == 0;
     for (int idx = tid; idx < C::BN * groups; idx += C::THREADS) {
         const int r = idx / groups, g = idx - r * groups;
         const long row = weight_row<C, FUSED>(r, nt, p.N);
         const uint32_t sb = as_global(p.scales)[row * groups + g];
         const uint32_t z = ((gptr_cu32)(uintptr_t)p.qzeros)[row * zwords + (g >> 3)] >> (4 * (g & 7)) & 0xFu;
-        table[g * C::BN + r] = (sb << 16) | z;
+        table[g * C::BN + r] = (sb << 16) | (0x6400u + z);
+        wide_scales |= (sb & 0x7FFFu) >= WIDE_SCALE;
     }
 #pragma unroll
-    for (int s = 0; s < C::S - 1; ++s) issue(s, s);
+    for (int s = 0; s < C::S - !C::AHEAD; ++s) issue(s, s);
+    if (args.wave_flags) {   // (the barrier leaves the direct loads in flight)
+        uint32_t *const flags = table + C::BN * groups;
+        const bool any = __ballot(wide_scales) != 0;
+        if (lane == 0) flags[wave] = any;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        wide_scales = __ballot(flags[lane % C::WAVES] != 0) != 0;
+    }
 
     f32x4_t acc[C::MB][C::NB];
 #pragma unroll
@@ -204,75 +247,116 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 || C::MB * C::NB >= 32 ? 
     const int wbyte = 16 * C::T * wk + 4 * C::T * kq;
     const int woff = wrow0 * (C::KC / 2) + (((wbyte >> 4) ^ weight_swizzle<C::WP>(lc)) << 4) + (wbyte & 15);
     const int xoff = xrow0 * (C::KC * 2);
-    int slot = 0;
-    for (int c = 0; c < chunks; ++c) {
-        // chunk c has arrived for every wave, and every wave is done with the slot that is filled next
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"((C::S - 2) * (C::X_LOADS + C::W_LOADS)) : "memory");
-        const uint8_t *xs = smem + slot * C::STAGE + xoff;
-        const uint8_t *ws = smem + slot * C::STAGE + C::X_BYTES + woff;
+    Masks masks{0x000F000Fu, 0x00F000F0u, 0x64006400u};
+    asm volatile("" : "+s"(masks.low), "+s"(masks.high));   // one scalar register and no literal per and-or
+    asm volatile("" : "+v"(masks.bias));
+    auto walk = [&](auto form) {
+        constexpr bool WIDE = decltype(form)::value;
         uint32_t w[C::NB][C::T];
         ScaleZero sz[C::NB];
-        const int g = (c * C::KC + 32 * C::T * wk + 8 * C::T * kq) >> args.gshift;
-#pragma unroll
-        for (int n = 0; n < C::NB; ++n) {
-            typedef __attribute__((ext_vector_type(C::T))) uint32_t words_t;
-            const words_t v = *reinterpret_cast<const words_t *>(ws + n * (16 * C::KC / 2));
-#pragma unroll
-            for (int t = 0; t < C::T; ++t) w[n][t] = v[t];
-            sz[n] = scale_zero(table[g * C::BN + wrow0 + 16 * n]);
-        }
-        auto fetch = [&](int t, int b) {
-            return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t *>(
-                xs + b * (16 * C::KC * 2) + (((xpiece + t) ^ xswz) << 4)));
-        };
         bf16x8_t xb[C::MB];
-#pragma unroll
-        for (int b = 0; b < C::MB; ++b) xb[b] = fetch(0, b);
-        issue(c + C::S - 1, slot == 0 ? C::S - 1 : slot - 1);
-        // Row block by row block: its MFMAs, the request for its next activations, a share of the next step's
-        // weights.  The scheduler is kept to this order: by its own it requests activations right before they are
-        // used and rebuilds weights in one piece (a 128x128 tile of K = 5632 alone on its CU: 70.9 against 58.4 us,
-        // a 64x128 one 31.4 against 29.8; the smallest tile has nothing to gain, 15.4 against 16.6).
         u32x4_t wa[C::NB];
+        auto words = [&](int chunk, int slot) {
+            const uint8_t *ws = smem + slot * C::STAGE + C::X_BYTES + woff;
+            const int g = (min(chunk, chunks - 1) * C::KC + 32 * C::T * wk + 8 * C::T * kq) >> args.gshift;
 #pragma unroll
-        for (int n = 0; n < C::NB; ++n) {
-            const Nibbles q = nibbles(w[n][0]);
+            for (int n = 0; n < C::NB; ++n) {
+                typedef __attribute__((ext_vector_type(C::T))) uint32_t words_t;
+                const words_t v = *reinterpret_cast<const words_t *>(ws + n * (16 * C::KC / 2));
 #pragma unroll
-            for (int i = 0; i < 4; ++i) wa[n][i] = dequant_pair(q, i, sz[n]);
-        }
-#pragma unroll
-        for (int t = 0; t < C::T; ++t) {
-            const bool last = t == C::T - 1;
-            constexpr int PAIRS = 4 * C::NB;
-            Nibbles q[C::NB];
-            u32x4_t next[C::NB];
-#pragma unroll
-            for (int b = 0; b < C::MB; ++b) {
-#pragma unroll
-                for (int n = 0; n < C::NB; ++n)
-                    acc[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wa[n]), xb[b],
-                                                                        acc[b][n], 0, 0, 0);
-                if (!last) {
-                    xb[b] = fetch(t + 1, b);
-#pragma unroll
-                    for (int pair = b * PAIRS / C::MB; pair < (b + 1) * PAIRS / C::MB; ++pair) {
-                        const int n = pair / 4, i = pair % 4;
-                        if (i == 0) q[n] = nibbles(w[n][last ? 0 : t + 1]);
-                        next[n][i] = dequant_pair(q[n], i, sz[n]);
-                    }
-                }
-                if constexpr (C::MB > 2) __builtin_amdgcn_sched_barrier(0);
+                for (int t = 0; t < C::T; ++t) w[n][t] = v[t];
+                sz[n] = scale_zero<WIDE>(table[g * C::BN + wrow0 + 16 * n]);
             }
-            if (!last)
+        };
+        auto fetch = [&](int slot, int t, int b) {
+            return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t *>(
+                smem + slot * C::STAGE + xoff + b * (16 * C::KC * 2) + (((xpiece + t) ^ xswz) << 4)));
+        };
+        auto first_step = [&](int chunk, int slot) {
+            words(chunk, slot);
 #pragma unroll
-                for (int n = 0; n < C::NB; ++n) wa[n] = next[n];
+            for (int b = 0; b < C::MB; ++b) xb[b] = fetch(slot, 0, b);
+            if (!C::AHEAD) issue(chunk + C::S - 1, slot == 0 ? C::S - 1 : slot - 1);
+#pragma unroll
+            for (int n = 0; n < C::NB; ++n) {
+                const Nibbles q = nibbles<WIDE>(w[n][0], masks);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) wa[n][i] = dequant_pair<WIDE>(q, i, sz[n]);
+            }
+        };
+        // the next chunk has arrived for every wave, and every wave is done with the slot that is filled next
+        auto arrive = [&]() {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"((C::S - 2) * (C::X_LOADS + C::W_LOADS)) : "memory");
+        };
+        if (C::AHEAD) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"((C::S - 1) * (C::X_LOADS + C::W_LOADS)) : "memory");
+            first_step(0, 0);
         }
-        slot = slot + 1 == C::S ? 0 : slot + 1;
-    }
+        int slot = 0;
+        for (int c = 0; c < chunks; ++c) {
+            if (!C::AHEAD) {
+                arrive();
+                first_step(c, slot);
+            }
+            const int following = slot + 1 == C::S ? 0 : slot + 1;
+            // Row block by row block: its MFMAs, the request for its next activations, a share of the next step's
+            // weights.  The scheduler is kept to this order: by its own it requests activations right before they are
+            // used and rebuilds weights in one piece.
+#pragma unroll
+            for (int t = 0; t < C::T; ++t) {
+                const bool last = t == C::T - 1;
+                constexpr int PAIRS = 4 * C::NB;
+                constexpr int HOLD = C::MB >= 4 ? C::MB / 4 : 1;             // row blocks ahead of the chunk's barrier
+                constexpr int AFTER = C::MB >= 4 ? HOLD + C::MB / 4 : HOLD;  // and ahead of the next words' use
+                const int from = last ? AFTER : 0;
+                Nibbles q[C::NB];
+                u32x4_t next[C::NB];
+#pragma unroll
+                for (int b = 0; b < C::MB; ++b) {
+#pragma unroll
+                    for (int n = 0; n < C::NB; ++n)
+                        acc[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wa[n]), xb[b],
+                                                                            acc[b][n], 0, 0, 0);
+                    // (the next activations take the registers of those just used)
+                    if constexpr (C::MB > 2) __builtin_amdgcn_sched_barrier(2 | 4);   // vector and scalar arithmetic may cross
+                    if (!last) {
+                        xb[b] = fetch(slot, t + 1, b);
+                    } else if (C::AHEAD && b == HOLD - 1) {
+                        // All of chunk c is in registers, for every wave, and all of chunk c + 1 has arrived: the rest of
+                        // this step's products cover the round trip for its first words and their rebuild.
+                        arrive();
+                        words(c + 1, following);
+                        issue(c + C::S, slot);
+#pragma unroll
+                        for (int e = 0; e < HOLD; ++e) xb[e] = fetch(following, 0, e);
+                    } else if (C::AHEAD && b >= HOLD) {
+                        xb[b] = fetch(following, 0, b);
+                    }
+                    if (!last || C::AHEAD) {
+#pragma unroll
+                        for (int pair = max(b - from, 0) * PAIRS / (C::MB - from); pair < max(b + 1 - from, 0) * PAIRS / (C::MB - from); ++pair) {
+                            const int n = pair / 4, i = pair % 4;
+                            if (i == 0) q[n] = nibbles<WIDE>(w[n][last ? 0 : t + 1], masks);
+                            next[n][i] = dequant_pair<WIDE>(q[n], i, sz[n]);
+                        }
+                    }
+                    if constexpr (C::MB > 2) __builtin_amdgcn_sched_barrier(0);
+                }
+                if (!last || C::AHEAD)
+#pragma unroll
+                    for (int n = 0; n < C::NB; ++n) wa[n] = next[n];
+            }
+            slot = following;
+        }
+    };
+    if (wide_scales)   // workgroup-uniform
+        walk(std::true_type{});
+    else
+        walk(std::false_type{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the repeats must not land in another workgroup's LDS
 
     int b0 = 0;
-    constexpr int OWN = C::MB / C::WK;   // row blocks a wave finishes
+    constexpr int OWN = C::MB > C::WK ? C::MB / C::WK : 1;   // row blocks a wave finishes
     if constexpr (C::WK > 1) {
         // partial tiles meet in LDS: wave wk finishes blocks wk * OWN ...
         __syncthreads();
@@ -284,6 +368,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES >= 8 || C::MB * C::NB >= 32 ? 
 #pragma unroll
             for (int n = 0; n < C::NB; ++n) red[(wk * step + base + b * C::NB + n) * WAVE + lane] = acc[b][n];
         __syncthreads();
+        if (b0 >= C::MB) return;
 #pragma unroll
         for (int b = 0; b < OWN; ++b)
 #pragma unroll
@@ -360,7 +445,9 @@ int launch_gemm(GemmArgs &args, hipStream_t stream) {
     const long tiles = gemm_tiles<C, FUSED>(args);
     if (tiles > (1L << 24)) return VRL_INT4_ESHAPE;
     if (!gemm_fits<C>(args)) return VRL_INT4_ELIMIT;
-    const size_t lds = C::lds(args.K >> args.gshift);
+    size_t lds = C::lds(args.K >> args.gshift);
+    args.wave_flags = lds + C::WAVES * sizeof(uint32_t) <= GEMM_LDS_CAP;
+    if (args.wave_flags) lds += C::WAVES * sizeof(uint32_t);
     auto kernel = &gemm_int4_kernel<C, FUSED>;
     if (lds > 64 * 1024) {   // once per build and device, at the largest size a launch may ask for
         static std::atomic<uint64_t> raised{0};
@@ -383,32 +470,52 @@ bool gemm_one_round(GemmArgs &args, long cus) {
     return gemm_fits<C>(args) && gemm_tiles<C, FUSED>(args) <= cus;
 }
 
-using Gemm32x64 = GemmCfg<1, 4, 2, 2, 1, 256, 2>;
-using Gemm64x64 = GemmCfg<1, 4, 4, 4, 1, 256, 2>;
-using Gemm64x128 = GemmCfg<1, 4, 4, 4, 2, 256, 2>;
-using Gemm128x128Split = GemmCfg<1, 4, 2, 8, 2, 128, 2>;
-using Gemm128x128 = GemmCfg<1, 4, 1, 8, 2, 64, 2>;
-using Gemm256x256 = GemmCfg<1, 8, 1, 16, 2, 64, 2>;
+template <int S> using Gemm32x32 = GemmCfg<1, 2, 8, 2, 1, 512, S, false>;
+template <int S> using Gemm32x64 = GemmCfg<1, 2, 8, 2, 2, 512, S, false>;
+template <int S> using Gemm32x64Short = GemmCfg<1, 4, 2, 2, 1, 256, S, false>;   // K no multiple of 512
+template <int S> using Gemm64x64 = GemmCfg<1, 4, 4, 4, 1, 256, S, false>;
+template <int S> using Gemm64x64Fused = GemmCfg<1, 2, 4, 4, 2, 256, S, false>;
+using Gemm64x128 = GemmCfg<1, 4, 4, 4, 2, 256, 2, false>;
+using Gemm128x128Split = GemmCfg<1, 4, 2, 8, 2, 128, 2, true>;
+using Gemm128x128 = GemmCfg<1, 4, 1, 8, 2, 64, 2, true>;
+using Gemm256x256 = GemmCfg<1, 8, 1, 16, 2, 64, 2, true>;
+
+// The launch over a tile whose launch is one round, with three chunks in LDS, or two where the table leaves room for no more.
+template <template <int> class C, bool FUSED>
+bool launch_one_round(GemmArgs &args, long cus, hipStream_t stream, int &rc) {
+    if (gemm_one_round<C<3>, FUSED>(args, cus))
+        rc = launch_gemm<C<3>, FUSED>(args, stream);
+    else if (gemm_one_round<C<2>, FUSED>(args, cus))
+        rc = launch_gemm<C<2>, FUSED>(args, stream);
+    else
+        return false;
+    return true;
+}
 
 // The smallest tile whose launch is one round of workgroups: until the chip is full a launch takes as long as one
-// tile does, and a smaller tile is done sooner (K = 2048, one round: 7.7 / 9.5 / 14.0 / 21.0 us in the order
-// below; the waves split K, since a tile alone on its CU is bound by the latency of its own chain).  Beyond that
-// tiles whose waves split nothing: 256x256, every weight rebuilt once for 256 rows (gate|up of 8192 rows by 2048:
-// 348 us alone, against 388; 373 to 395 between other work), where its rounds are at least 85 % full, 128x128
-// otherwise (gate|up of 1664 rows: 109 against 88 us; of 1280 rows: 62 against 76).  Measured at 48 to 8192 rows of
-// q|k|v (3 x 2048), o_proj, gate|up (11264) and down_proj (K = 5632): of these builds the choice is the best or within
-// 5 % of it at every one.  Not built: a 64 x 128 tile whose waves split K two ways, 7 % faster than the choice for
-// gate|up of 512 rows (36.6 against 39.3 us) and q|k|v of 1024 (38.1 against 40.8).
+// tile does, and a smaller tile is done sooner (K = 2048, one round: 6.7 / 8.2 / 9.9 / 15.2 / 21.7 us in the order
+// below without the short and the fused ones; the waves split K, since a tile alone on its CU is bound by the latency of its own chain).
+// The more k a chunk of these has, the fewer trips: down_proj (K = 5632, N = 2048) at 40 rows in chunks of 512 on 32x32
+// tiles takes 10.5 us, in chunks of 256 on 32x64 ones 16.0; at 160 rows 32x64 in chunks of 512 takes 14.4 against 17.0.  With
+// a third chunk in LDS 64x64 takes 18.8 against 21.9 us (512 rows, K = 5632).  Gate|up of up to 64 rows takes 11.0 us on
+// 64x64 tiles of eight waves against 15.1 on 64x128.  Beyond one round tiles whose waves split nothing: 256x256, every
+// weight rebuilt once for 256 rows, where its rounds are at least 85 % full (gate|up of 8192 rows by 2048: 339 us),
+// 128x128 otherwise.  Not faster: a third chunk for 64x128 or the 128x128 ones, four or five for 32x64, 64x64 tiles with
+// their waves two by two (512 rows, K = 5632: 24.9 us), AHEAD for the tiles above 128x128.
 //
-// From counters: the vector units are active in 43 to 72 % of the busy cycles of a CU, the matrix units in 11 (32x64)
-// to 55 % (256x256); the LDS in 17 to 35 %, of which 8 to 30 % are conflicts.  The large tile is bound by issuing to
-// the first two, the small ones by the latency of a tile's chain.
+// The large tile is bound by issuing to the vector and matrix units, the small ones by the latency of a tile's chain.
 template <bool FUSED>
 int dispatch_gemm(GemmArgs &args, hipStream_t stream) {
     const long cus = device_cu_count();
-    if constexpr (!FUSED) {   // a wave of these holds one block of columns, a fused one needs gate and up
-        if (gemm_one_round<Gemm32x64, false>(args, cus)) return launch_gemm<Gemm32x64, false>(args, stream);
-        if (gemm_one_round<Gemm64x64, false>(args, cus)) return launch_gemm<Gemm64x64, false>(args, stream);
+    int rc;
+    if constexpr (!FUSED) {   // a wave of all but the second holds one block of columns, a fused one needs gate and up
+        if (launch_one_round<Gemm32x32, false>(args, cus, stream, rc)) return rc;
+        if (launch_one_round<Gemm32x64, false>(args, cus, stream, rc)) return rc;
+        if (launch_one_round<Gemm32x64Short, false>(args, cus, stream, rc)) return rc;
+        if (launch_one_round<Gemm64x64, false>(args, cus, stream, rc)) return rc;
+    } else {
+        if (launch_one_round<Gemm32x64, true>(args, cus, stream, rc)) return rc;
+        if (launch_one_round<Gemm64x64Fused, true>(args, cus, stream, rc)) return rc;
     }
     if (gemm_one_round<Gemm64x128, FUSED>(args, cus)) return launch_gemm<Gemm64x128, FUSED>(args, stream);
     if (gemm_one_round<Gemm128x128Split, FUSED>(args, cus)) return launch_gemm<Gemm128x128Split, FUSED>(args, stream);
