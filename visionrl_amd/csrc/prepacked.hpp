@@ -105,8 +105,34 @@ constexpr int PP_ZERO_ROW = 2;  // DevProblem::prepacked bit
 
 // natural-order staging of x[:, k0:k1) (k beyond K reads as zero), plus a row of zeros at
 // row M if the record asks for one
+// Up to 16 rows a wave takes 512 k of a row at a time, straight into LDS: all of a workgroup's requests are on their way at
+// once and no instruction divides by the row length (a step of 24 layers of 2048 with adapters at 16 rows 1345 -> 1318 us, 30
+// layers of 4096 at 8 rows 1875 -> 1860).  With more rows a workgroup's loads are bound by their rate, and the direct ones
+// are the slower (the head's call at 32 rows 17.1 against 18.1 us; a step at 32 rows 1639 against 1645).
+constexpr int STAGE_DIRECT_ROWS = 16;
 __device__ __forceinline__ void stage_x_natural(const DevProblem &p, int k0, int k1, uint16_t *xs,
                                                 int xstride, int nthreads) {
+    if (p.M <= STAGE_DIRECT_ROWS) {
+        const int pieces = (k1 - k0) / PP_SC, nwaves = nthreads / WAVE;
+        const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int rows = p.M + ((p.prepacked & PP_ZERO_ROW) ? 1 : 0);
+        for (int m = 0, j = wave;; j += nwaves) {
+            for (; j >= pieces && m < rows; j -= pieces) ++m;
+            if (m >= rows) break;
+            const int k = k0 + j * PP_SC;
+            uint16_t *const at = xs + m * xstride + j * PP_SC;
+            const uint16_t *const from = p.x + (long)m * p.K + k;
+            if (m < p.M && k + PP_SC <= p.K) {   // wave-uniform
+                dma16(reinterpret_cast<uint8_t *>(at), reinterpret_cast<const uint8_t *>(from), lane * 16);
+            } else {
+                u32x4_t d = {0u, 0u, 0u, 0u};
+                if (m < p.M && k + lane * 8 < p.K) d = *as_global(reinterpret_cast<const u32x4_t *>(from + lane * 8));
+                *reinterpret_cast<u32x4_t *>(at + lane * 8) = d;
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the compiler does not see the direct loads
+        return;
+    }
     const int words_per_row = (k1 - k0) >> 3;
     const int total = (p.M + ((p.prepacked & PP_ZERO_ROW) ? 1 : 0)) * words_per_row;
     for (int idx = threadIdx.x; idx < total; idx += nthreads) {

@@ -45,12 +45,11 @@ struct GemmArgs {
 
 // One packed word -> eight exactly rounded bf16 weights in k order, in instructions that can be issued between MFMAs, pair by
 // pair: (q - z) s as fma(q', s', c) with an exact product and an exact c, so that the conversion is the one rounding of the
-// contract.  Two forms.  Plain: a nibble under the exponent of 1024 is the half-precision value 1024 + q, or 1024 + 16 q where
-// it sits four bits further up, which the mixed fma takes as it is: 17 instructions.
-// Its c, -(1024 + z) s, is finite for
-// scales below 2^117; a workgroup that meets a larger one (an infinity, a NaN) takes the wide form for all of its tile, the
-// byte converter's float(q) and c = -z s: 23 instructions, the only form before
-// (prompt of 512 rows, four layers: 414 -> 399 us from this alone).
+// contract.  Two forms.  Plain, 17 instructions: a nibble under the exponent of 1024 is the half-precision value 1024 + q, or
+// 1024 + 16 q where it sits four bits further up, which the mixed fma takes as it is.  Its c, -(1024 + z) s, is finite for
+// scales below 2^117; a workgroup that meets a larger one (an infinity, a NaN) takes the wide form for all of its tile:
+// the byte converter's float(q) and c = -z s, 23 instructions.  A prompt of 512 rows, four layers: 414 us with the wide form
+// everywhere, 399 with the plain one.
 struct ScaleZero { float s, c, s16, c16; };
 struct Nibbles { uint32_t h[4]; };
 struct Masks { uint32_t low, high, bias; };
@@ -89,15 +88,6 @@ __device__ __forceinline__ uint32_t dequant_pair(const Nibbles &b, int i, const 
                              __builtin_fmaf((float)((b.h[1] >> (8 * i)) & 0xFFu), c.s, c.c));
     return pack_bf16_rne(__builtin_fmaf(half_of(b.h[i % 2 * 2], i / 2), c.s, c.c),
                          __builtin_fmaf(half_of(b.h[i % 2 * 2 + 1], i / 2), c.s16, c.c16));
-}
-
-// 16 bytes per lane from global memory (base + off, 32 bits) to LDS at `lds` + 16 * lane; counted by vmcnt, touches no
-// register.  In assembly: the compiler takes the builtin for an access of both counters and from then on waits for every
-// outstanding LDS read where it needs the first, once per MFMA step.  What orders these loads against the LDS reads are the
-// waits and barriers of the kernel, as with the builtin.  (m0 is not allocated; nothing else here uses it.)
-__device__ __forceinline__ void dma16(uint8_t *lds, const uint8_t *base, uint32_t off) {
-    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base));
 }
 
 // WM x WN x WK waves share a tile: WM and WN split its rows and columns, WK the k of every chunk (their partial
