@@ -44,7 +44,8 @@ def _launch_pays(rows: int, K: int, columns: int, group_size: int, products: int
     """Whether one ``ops.int4_gemm`` launch beats rebuilding the weight and a library product per weight.
 
     Both routes were timed, queued back to back on the GPU, at 33 to 8192 rows, K of 1024 to 11008, up to 22016 weight
-    rows and groups of 32, 64 and 128.  The library's rate is 1.2 to 1.6 times the launch's once its products are
+    rows and groups of 32, 64 and 128, with a launch that took 3 to 40 % longer than today's: the lines below are on the
+    safe side of it.  The library's rate is 1.2 to 1.6 times the launch's once its products are
     large; what the launch saves is the pass that writes the weight, SiLU's pass and the launches of a group.  A group
     costs as much again for each halving of the group size below 128, in the table of scales of every tile: ``k``
     is the K of equal cost.
