@@ -235,7 +235,9 @@ int vrl_decode_run_calls(const vrl_step_call *calls, int n_calls, int *failed_at
  * A whole decode step of a Llama trunk in one launch (decode_trunk.hip): for one new token per row, every layer's
  * norm, q|k|v, rotary + cache append + attention, o_proj + residual, norm, gate|up + SiLU, down_proj + residual,
  * and the model's norm.  Results are those of the entry points above called one after another, bit for bit.  The
- * launch is cooperative, one workgroup per compute unit, and may be captured into a graph.
+ * launch is cooperative, one workgroup per compute unit, and may be captured into a graph.  Where something else
+ * keeps compute units for itself (a kernel of another stream, graph or process), the workgroups that have started
+ * share the work after a while: the same results, later.
  *   layers    n_layers records in DEVICE memory, 16-byte aligned; weights prepacked (vrl_int4_prepack, G = 128),
  *             gate_up one blob of 2 * inter rows, norms bf16 [hidden], caches as for vrl_rope_attn_decode_bf16
  *   x         bf16 [M, hidden]: the new tokens' embeddings (read only)
@@ -249,6 +251,7 @@ int vrl_decode_run_calls(const vrl_step_call *calls, int n_calls, int *failed_at
  *   wait_limit  0, or how often a wave looks for a result of another workgroup in vain before it takes NaN for it
  *             and waits no more (default 2^22): every wait ends, and a launch that gave up has NaN in its output.
  *             Its workspace has to be zeroed before the next launch.
+ *   max_workgroups  0, or how many workgroups take part at most (the others end at once)
  * vrl_decode_trunk_workspace_bytes returns 0 where the launch does not apply (the other fields may then be NULL).
  * It applies to M <= 4, hidden 2048, head_dim 128, group_size 128, L_max <= 8192, n_heads * 128 a multiple of 256
  * up to 8192, inter a multiple of 256 up to 8192, where the launches above would add up the norms in one of the
@@ -270,7 +273,7 @@ typedef struct vrl_trunk {
     size_t workspace_bytes;
     int32_t n_layers, M, hidden, inter, n_heads, n_kv_heads, head_dim, group_size, L_max, position_per_row, split_from;
     float eps;
-    uint32_t wait_limit;
+    uint32_t wait_limit, max_workgroups;
 } vrl_trunk;
 
 size_t vrl_decode_trunk_workspace_bytes(const vrl_trunk *trunk);

@@ -181,6 +181,90 @@ def test_steps_on_several_streams():
     assert all(torch.equal(s.native.normed, w) for s, w in zip(steps, want))
 
 
+@pytest.mark.parametrize("workgroups", [1, 3, 100, 255])
+@pytest.mark.parametrize("kwargs", [
+    dict(rows=1, slot=(330,)), dict(rows=2, slot=(900,), kv_heads=4), dict(rows=3, slot=(0,), inter=5376),
+    dict(rows=4, slot=(511, 900, 40, 2000)), dict(rows=4, slot=(800,), heads=12, kv_heads=4),
+    dict(rows=2, slot=(130,), inter=8192, final_norm=False),
+])
+def test_a_part_of_the_chip_has_the_bits_of_the_list(workgroups, kwargs):
+    """The parts of every product dealt out to fewer workgroups than they are laid out for."""
+    print("decode trunk team:", workgroups, kwargs, flush=True)
+    step = Step(**kwargs)
+    for desc in step.one:
+        desc.max_workgroups = workgroups
+    slots = kwargs["slot"] if len(kwargs["slot"]) > 1 else kwargs["slot"] * kwargs["rows"]
+    inside = [m for m, slot in enumerate(slots) if slot < 1024]
+    want, want_cache = step.run(False)
+    for _ in range(2):
+        got, cache = step.run(True)
+        assert torch.equal(got[inside].view(torch.int16), want[inside].view(torch.int16))
+        assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(cache, want_cache))
+
+
+@pytest.mark.parametrize("layers,heads,kv_heads", [(1, 8, 2), (1, 8, 8), (2, 8, 2)])
+def test_workgroups_without_a_part_behind_the_last_exchange(layers, heads, kv_heads):
+    """One row and few heads: some workgroups have gate|up tiles only, and in the last layer nobody needs to have
+    seen them before the first ones end."""
+    print("decode trunk few heads:", layers, heads, kv_heads, flush=True)
+    step = Step(1, layers=layers, heads=heads, kv_heads=kv_heads, length=320, slot=(200,), final_norm=False)
+    step.check()
+
+
+def test_a_kernel_that_keeps_a_compute_unit():
+    """A step beside a kernel that stays on the chip for long: neither waits for it nor gives anything up."""
+    print("decode trunk: beside a kernel", flush=True)
+    step = Step(2, layers=4)
+    want, want_cache = step.run(False)
+    side = torch.cuda.Stream()
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    start.record()
+    torch.cuda._sleep(10_000_000)
+    end.record()
+    torch.cuda.synchronize()
+    cycles = int(10_000_000 * 300 / start.elapsed_time(end))   # 0.3 s
+    before = [t.clone() for t in step.cache]
+    busy, done = torch.cuda.Event(), torch.cuda.Event()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(cycles)
+        busy.record()
+    got = step.native.run()
+    done.record()
+    done.synchronize()
+    assert not busy.query()
+    assert torch.equal(got, want)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(step.cache, want_cache))
+    for t, b in zip(step.cache, before):
+        t.copy_(b)
+    got, _ = step.run(True)
+    assert torch.equal(got, want)
+
+
+def test_recorded_steps_on_several_streams():
+    """Replays of steps with workspaces of their own, in flight together and beside an eager one."""
+    print("decode trunk: recorded steps", flush=True)
+    steps = [Step(2, seed=s, layers=4) for s in (1, 2, 3)]
+    want = [s.run(False)[0] for s in steps]
+    graphs = []
+    for s in steps[:2]:
+        s.native.run()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            s.native.run()
+        graphs.append(graph)
+    streams = [torch.cuda.Stream() for _ in steps]
+    torch.cuda.synchronize()
+    for _ in range(10):
+        for launch, stream in zip((graphs[0].replay, graphs[1].replay, steps[2].native.run), streams):
+            with torch.cuda.stream(stream):
+                launch()
+    torch.cuda.synchronize()
+    assert all(torch.equal(s.native.normed, w) for s, w in zip(steps, want))
+
+
 def test_every_wait_ends():
     """One look per wave: nothing is waited for, the launch ends and its output says so; over a cleared workspace
     the next step is right again."""

@@ -221,7 +221,7 @@ class Trunk(ctypes.Structure):
         [("workspace_bytes", ctypes.c_size_t)] + \
         [(name, ctypes.c_int32) for name in ("n_layers", "M", "hidden", "inter", "n_heads", "n_kv_heads", "head_dim",
                                              "group_size", "L_max", "position_per_row", "split_from")] + \
-        [("eps", ctypes.c_float), ("wait_limit", ctypes.c_uint32)]
+        [("eps", ctypes.c_float), ("wait_limit", ctypes.c_uint32), ("max_workgroups", ctypes.c_uint32)]
 
 
 class PlanInfo(ctypes.Structure):

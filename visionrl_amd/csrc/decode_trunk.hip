@@ -24,10 +24,19 @@
 // only if it has a part in the next one, every part of which is waited for before the one after it begins, and so on
 // around the layer.
 //
-// Waiting.  Every workgroup is resident (one per compute unit, launched cooperatively: the runtime refuses a grid that does
-// not fit and runs such launches one after another, from whichever stream or graph), so every wait ends.  It is bounded all
-// the same: a wave gives up after `budget` unsuccessful looks in total, takes NaN for what did not come, hands NaN on and
-// never waits again, so the launch ends and its output says so.
+// Who takes part.  The work is laid out for one workgroup per compute unit, all of them there at once, and a workgroup takes
+// every register of its compute unit: a single wave of anything else (a collective that waits for a late rank, another
+// process, a step from another graph) keeps one of them out, for as long as it likes.  So nothing waits for a workgroup that
+// has not started.  Each takes a ticket, and the team is fixed once, by one compare-and-swap: by the last to arrive, or by one
+// that has waited for the others as long as the step would take those that are there (TEAM_TICKS).  Members are running by
+// then and stay, so what one waits for comes; a workgroup that starts later finds itself left out and ends.  With everyone
+// there each has its own part of every product.  Otherwise the parts are dealt out to the members, product by product:
+// the same sums and bits, without the work ahead of its input (24 layers at 2 rows: 515 us with all 256, 838 with 255 or 128
+// of them, 6.0 ms with 16; the launch list takes 766).  The team is looked up behind the first product, before anything is
+// handed out, so that the tickets cost next to nothing.
+//
+// Waits are bounded all the same: a wave gives up after `budget` unsuccessful looks in total, takes NaN for what did not
+// come, hands NaN on and never waits again, so the launch ends and its output says so.
 //
 // The order of sums is the launch list's, bit for bit: products by super-chunks of 512 k added up in order, norms and
 // attention as in stage_x_norm and rope_attn_decode_kernel.  A policy may take either form for the same step (partial
@@ -50,6 +59,16 @@ constexpr int HEAD_DIM = 128;
 constexpr int STATE = HEAD_DIM + 2;         // words of a softmax state: output, maximum, sum
 constexpr uint32_t NOT_COME = 0x7FC07FC0u; // NaN as two bf16 values and as a float
 constexpr uint32_t TRUNK_BUDGET = 1u << 22; // looks of about a microsecond each
+// How long a workgroup waits for the others to start, in ticks of 10 ns: what a layer takes one workgroup alone (3.9 ms at 2
+// rows), divided by those that are there, and never less than the launch itself may need to bring all of them up.
+constexpr uint32_t TEAM_TICKS = 400000, TEAM_TICKS_LEAST = 10000;
+
+// The first 256 bytes of the workspace.
+struct TrunkState {
+    uint64_t team;       // number of a launch's first layer << 32 | workgroups that take part in it
+    uint32_t number;     // of the last exchange; the last workgroup to arrive counts it up
+    uint32_t arrived;    // tickets taken; the last workgroup to arrive puts it back
+};
 
 struct TrunkArgs {
     const vrl_trunk_layer *layers;
@@ -57,10 +76,11 @@ struct TrunkArgs {
     const uint8_t *mask;
     const long long *position;
     uint16_t *normed, *h_out;
-    uint32_t *counter;              // the number of the last exchange
+    TrunkState *state;
     uint64_t *e_qkv, *e_part, *e_attn, *e_mid, *e_act, *e_out;
     float eps;
     uint32_t budget;
+    int32_t grid, most;                   // workgroups, and how many of them may take part
     int32_t n_layers, position_stride, M, A, KV, I, heads, kv_heads, L_max;
     int32_t nsc_a, nsc_i;                 // super-chunks of A and I
     int32_t split_from, split_build;      // filled slots from which a pair's slots are divided in ranges; whether they ever are
@@ -202,19 +222,25 @@ struct TrunkCfg {
     static constexpr size_t STAGE_BYTES = ((ALL > OWN ? ALL : OWN) + 15) / 16 * 16;
     static constexpr int PART = TW * MW * 16;   // floats
     static constexpr size_t ATTN_BYTES = (size_t)TW * HEAD_DIM * 4 + 5 * 64 * 4 + 2 * TW * 4;
-    static constexpr size_t LDS = STAGE_BYTES + 2 * PART * 4 + ATTN_BYTES + TW * 4;
+    static constexpr size_t LDS = STAGE_BYTES + 2 * PART * 4 + ATTN_BYTES + TW * 4 + 16;
 };
 
 // A lane's words of a part of a row, and of the norm's weight for its share of them
 template <int MW, int P>
 struct Rows { uint32_t h[4 * (H / 512 / P)], w[MW]; };
 
+typedef __attribute__((address_space(3))) uint8_t *lds_ptr;
 template <class C>
-__global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
+__device__ void share_out(arg_ptr args, lds_ptr smem);
+
+// The step.  SHARED false: every workgroup is there and works on its own part of each product; the kernel.  SHARED true:
+// the team is not the whole grid; a function that the kernel calls for the rest of its life, so that neither form's
+// registers are the other's (in one function a step of 24 layers took 537 us in place of 511).
+template <class C, bool SHARED>
+__device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uint8_t *smem) {
     constexpr int MW = C::MW, splits = C::SPLITS;
-    extern __shared__ __align__(16) uint8_t smem[];
     int tid = threadIdx.x, lane, wave, lc, kq;
-    int wg = blockIdx.x, G = gridDim.x;
+    int wg = blockIdx.x, G = a.grid;
     int M = a.M, A = a.A, KV = a.KV, I = a.I, heads = a.heads;
     uint16_t *const xs = reinterpret_cast<uint16_t *>(smem);
     float *const parts = reinterpret_cast<float *>(smem + C::STAGE_BYTES);
@@ -222,12 +248,13 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
     uint32_t *const qs = reinterpret_cast<uint32_t *>(pacc + TW * HEAD_DIM), *const ks = qs + 64, *const vs = ks + 64,
              *const turn = vs + 64;
     float *const pm = reinterpret_cast<float *>(turn + 128), *const pl = pm + TW, *const red = pl + TW;
+    uint32_t *const joined = reinterpret_cast<uint32_t *>(red + TW);
     uint32_t budget = a.budget;
-    const uint32_t first = *a.counter;   // exchange e of layer l is number first + 8 + 8 l + e
+    uint32_t number = 0;   // exchange e of a layer is number + e; known from the first product on
 
     // Arguments used once a layer, or once, are read again where they are used.
     auto again = [&]() {
-        arg_ptr p = (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+        arg_ptr p = args;
         asm volatile("" : "+s"(p));
         return p;
     };
@@ -249,9 +276,14 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
 
     // ---- which units of a product are this wave's: unit u counts super-chunks, then gate and up, then tiles
     auto slots_of = [&](int at, int tiles) { return at < tiles ? (tiles - 1 - at) / G + 1 : 0; };
-    const int slots_qkv = slots_of(wg, (A + 2 * KV) >> 4), slots_i = slots_of(wg, I >> 4);
-    // the tiles of o_proj and down_proj begin at the other end of the grid, where workgroups have fewer of the others
-    const bool has_h = G - 1 - wg < H / 16;   // (one at most)
+    int slots_qkv, slots_i;
+    bool has_h;
+    auto place_tiles = [&]() {
+        slots_qkv = slots_of(wg, (A + 2 * KV) >> 4), slots_i = slots_of(wg, I >> 4);
+        // the tiles of o_proj and down_proj begin at the other end of the grid, where workgroups have fewer of the others
+        has_h = G - 1 - wg < H / 16;   // (one at most)
+    };
+    place_tiles();
     // (a unit: a super-chunk of a tile; never more than sixteen)
     auto units_of = [&](Phase ph) {
         return ph == P_QKV ? slots_qkv * NSC : ph == P_GATE_UP ? slots_i * 2 * NSC : has_h ? (ph == P_O ? a.nsc_a : a.nsc_i) : 0;
@@ -372,7 +404,8 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
 #pragma unroll
         for (uint32_t &v : x.w) v = __builtin_nondeterministic_value(v);
     };
-    auto take_rows = [&](auto P, Rows<MW, P> &x, const void *weight, const uint64_t *words, uint32_t number) {
+    // (`plain`: the rows themselves, in place of words)
+    auto take_rows = [&](auto P, Rows<MW, P> &x, const void *weight, const uint64_t *words, uint32_t number, const uint16_t *plain = nullptr) {
         constexpr int EIGHTS = H / 512 / P;
 #pragma unroll
         for (int j = 0; j < GROUPS; ++j) {
@@ -381,6 +414,15 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
             x.w[2 * j] = w[0], x.w[2 * j + 1] = w[1];
         }
         const int row = min(part_of(P) / P, M - 1), at = row_at(P) / 2;
+        if (plain) {
+#pragma unroll
+            for (int i = 0; i < 2 * EIGHTS; ++i) {
+                const u32x2_t v = *(const __attribute__((address_space(1))) u32x2_t *)(uintptr_t)(
+                    plain + 2 * (row * ROW_WORDS + i / 2 * 256 + i % 2 * 2 + at));
+                x.h[2 * i] = v[0], x.h[2 * i + 1] = v[1];
+            }
+            return;
+        }
         await_pairs<2 * EIGHTS>(x.h, number, budget, words, M * ROW_WORDS, [&](int) { return at; },
                                 [&](int i) { return row * ROW_WORDS + i / 2 * 256 + i % 2 * 2; });
     };
@@ -428,35 +470,41 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
     // sixteen lanes visit the slots of wave w, group g: 64 u + 4 w + g, four at a time; groups, then waves.  The
     // workgroups of a pair take its waves' slots each (`lead`: the first of them), and all waves' states meet through
     // memory; or, from `split_from` filled slots on, a contiguous range of slots as in its split form (`ranges`).
-    const int pair = wg / splits, split = wg % splits;
-    const bool attends = pair < M * heads;
-    int am = attends ? pair / heads : 0, ah = attends ? pair % heads : 0;
-    const int group = heads / a.kv_heads;
-    const bool appends = attends && split == 0 && ah % group == 0;
-    int akv = ah / group;
-    int p = -1, j_lo = 0, j_hi = 0, lead = 0, my_waves = 0;
-    bool ranges = false, own_slot = false;
+    int pair, split, am, ah, akv, p, j_lo, j_hi, lead, my_waves;
+    bool attends, appends, ranges, own_slot;
+    auto place_pair = [&]() {
+        const arg_ptr t = again();   // (or these arguments are kept in registers from layer to layer)
+        const int group = heads / t->kv_heads;
+        pair = wg / splits, split = wg % splits;
+        attends = pair < M * heads;
+        am = attends ? pair / heads : 0, ah = attends ? pair % heads : 0;
+        appends = attends && split == 0 && ah % group == 0;
+        akv = ah / group;
+        p = -1, j_lo = 0, j_hi = 0, lead = 0, my_waves = 0;
+        ranges = own_slot = false;
+        if (attends) {
+            const uint8_t *mrow = t->mask + (long)am * t->L_max;
+            const long long p64 = t->position[(long)am * t->position_stride];
+            const int at = __builtin_amdgcn_readfirstlane(p64 >= 0 && p64 < t->L_max ? (int)p64 : -1);
+            if (at >= 0) {   // else the row is left alone: nothing appended, nothing attended
+                p = at;
+                ranges = p >= t->split_from;
+                const int share = ((p + splits - 1) / splits + 63) / 64 * 64;
+                j_lo = ranges ? min(p, split * share) : 0;
+                j_hi = ranges ? min(p, j_lo + share) : p;
+                if (wave == 0) {   // (read by this wave alone)
+                    turn[lane] = ((gptr_cu32)(uintptr_t)(t->cos + (long)p * HEAD_DIM))[lane];
+                    turn[64 + lane] = ((gptr_cu32)(uintptr_t)(t->sin + (long)p * HEAD_DIM))[lane];
+                }
+                own_slot = (split == 0 || !ranges) && mrow[p] != 0;
+            }
+            my_waves = ranges ? TW : TW / splits;
+            lead = ranges ? 0 : split * my_waves;
+        }
+    };
+    place_pair();
     uint32_t live = 0;
     constexpr int BATCH = 4, AT_ONCE = 2 * BATCH;   // slots of a group per step of the running softmax; requested at once
-    if (attends) {
-        const uint8_t *mrow = a.mask + (long)am * a.L_max;
-        const long long p64 = a.position[(long)am * a.position_stride];
-        const int at = __builtin_amdgcn_readfirstlane(p64 >= 0 && p64 < a.L_max ? (int)p64 : -1);
-        if (at >= 0) {   // else the row is left alone: nothing appended, nothing attended
-            p = at;
-            ranges = p >= a.split_from;
-            const int share = ((p + splits - 1) / splits + 63) / 64 * 64;
-            j_lo = ranges ? min(p, split * share) : 0;
-            j_hi = ranges ? min(p, j_lo + share) : p;
-            if (wave == 0) {   // (read by this wave alone)
-                turn[lane] = ((gptr_cu32)(uintptr_t)(a.cos + (long)p * HEAD_DIM))[lane];
-                turn[64 + lane] = ((gptr_cu32)(uintptr_t)(a.sin + (long)p * HEAD_DIM))[lane];
-            }
-            own_slot = (split == 0 || !ranges) && mrow[p] != 0;
-        }
-        my_waves = ranges ? TW : TW / splits;
-        lead = ranges ? 0 : split * my_waves;
-    }
     auto slot_of = [&](int j0, int u) { return j0 + u * (4 * TW) + (lead + wave) * 4 + kq; };   // j0: the first of the trip
     auto counts = [&](int j0) {   // which of the trip's slots count, a bit each
         const uint8_t *mrow = again()->mask + (long)am * a.L_max;
@@ -486,267 +534,214 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
     };
 
     // The residual stream at (row, column pair) of this workgroup's o_proj and down_proj tiles, kept by the threads that
-    // finish them.  The input rows begin it, and are handed to the first layer like a layer's output.
+    // finish them.  The input rows begin it.
     uint32_t stream = 0;
     auto stream_word = [&]() { return tile_row() * ROW_WORDS + (G - 1 - wg) * 8 + (lane & 7); };
-    if (has_h && wave == 0 && stores()) {
-        stream = ((gptr_cu32)(uintptr_t)a.cur)[stream_word()];
-        put_word(a.e_out + stream_word(), stream, first + 6);
-    }
-    load(P_QKV, 0);
-    for (int l = 0; l < a.n_layers; ++l) {
-        const layer_ptr L = (layer_ptr)(uintptr_t)a.layers + l;
-        const uint32_t number = first + 8u + 8u * l;
-        forget();
-        opaque(am), opaque(ah), opaque(akv);
-        // -------------------------------------------------------------- norm, q|k|v
-        {
-            Rows<MW, C::P1> x;
-            Built built;
-            undefined(x);
-            build_ahead(P_QKV, built);
-            if (slots_qkv) take_rows(P1, x, L->norm1, a.e_out, number - 2);   // the sixth exchange of the layer before
-            load(P_O, l);
-            if (slots_qkv) {
-                normalise(P1, x, L->eps1);
-                multiply_staged(P_QKV, built);
+    auto begin_stream = [&]() {
+        if (has_h && wave == 0 && stores()) stream = ((gptr_cu32)(uintptr_t)again()->cur)[stream_word()];
+    };
+
+    // ---- the parts of a layer that both forms of the step go through
+    auto publish_qkv = [&]() {
+        if (!slots_qkv) return;
+        lds_barrier();
+        if (wave < slots_qkv) {
+            const float2 s = tile_sum(0, wave * NSC, NSC);
+            if (stores())
+                put_word(a.e_qkv + tile_row() * ((A + 2 * KV) >> 1) + (wg + wave * G) * 8 + (lane & 7),
+                         pack_bf16_rne(s.x, s.y), number + 1);
+        }
+    };
+    // wave 0: the new token's query, key (both rotated) and value into LDS, the latter two into the caches
+    auto receive_token = [&](layer_ptr L, bool append) __attribute__((always_inline)) {
+        // lanes 0..15 the query's dimensions 4 i ... and 64 + 4 i ..., 16..31 the key's, 32..47 the value's (48..63 too)
+        const int part = kq, row_words = (A + 2 * KV) >> 1;
+        const int at = (part == 0 ? ah * 64 : (part == 1 ? A >> 1 : (A + KV) >> 1) + akv * 64) + 2 * lc;
+        uint32_t x[4];
+        await_pairs<2>(x, number + 1, budget, a.e_qkv, M * row_words, [&](int) { return at; },
+                       [&](int i) { return am * row_words + 32 * i; });
+        if (part < 2) {   // bf16(bf16(x cos) + bf16(rotate_half(x) sin))
+            auto round = [](float v) { return low_bf16(pack_bf16_rne(v, 0.0f)); };
+            const u32x2_t c0 = *reinterpret_cast<const u32x2_t *>(turn + 2 * lc), c1 = *reinterpret_cast<const u32x2_t *>(turn + 32 + 2 * lc);
+            const u32x2_t s0 = *reinterpret_cast<const u32x2_t *>(turn + 64 + 2 * lc), s1 = *reinterpret_cast<const u32x2_t *>(turn + 96 + 2 * lc);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float a0 = low_bf16(x[e]), a1 = high_bf16(x[e]), b0 = low_bf16(x[2 + e]), b1 = high_bf16(x[2 + e]);
+                x[e] = pack_bf16_rne(round(a0 * low_bf16(c0[e])) + round(-b0 * low_bf16(s0[e])),
+                                     round(a1 * high_bf16(c0[e])) + round(-b1 * high_bf16(s0[e])));
+                x[2 + e] = pack_bf16_rne(round(b0 * low_bf16(c1[e])) + round(a0 * low_bf16(s1[e])),
+                                         round(b1 * high_bf16(c1[e])) + round(a1 * high_bf16(s1[e])));
             }
         }
-        auto publish_qkv = [&]() {
-            if (!slots_qkv) return;
-            lds_barrier();
-            if (wave < slots_qkv) {
-                const float2 s = tile_sum(0, wave * NSC, NSC);
-                if (stores())
-                    put_word(a.e_qkv + tile_row() * ((A + 2 * KV) >> 1) + (wg + wave * G) * 8 + (lane & 7),
-                             pack_bf16_rne(s.x, s.y), number + 1);
+        uint32_t *out = qs + min(part, 2) * 64 + 2 * lc;   // qs, ks, vs
+        *reinterpret_cast<u32x2_t *>(out) = u32x2_t{x[0], x[1]};
+        *reinterpret_cast<u32x2_t *>(out + 32) = u32x2_t{x[2], x[3]};
+        if (append && appends && p >= 0 && part > 0) {
+            gptr_w to = (gptr_w)(uintptr_t)(static_cast<uint16_t *>(part == 1 ? L->k_cache : L->v_cache) + cache_base() +
+                                            (long)p * HEAD_DIM) + 2 * lc;
+            to[0] = x[0], to[1] = x[1], to[32] = x[2], to[33] = x[3];
+        }
+    };
+    // the softmax states of this workgroup's waves over its slots (`kv`: the first of them, requested)
+    auto score_slots = [&](layer_ptr L, Slots &kv) __attribute__((always_inline)) {
+        const float scaling = L->scaling;
+        const u32x4_t q4 = *reinterpret_cast<const u32x4_t *>(qs + lc * 4);
+        float mx = -INFINITY, sum = 0.0f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        uint32_t now = live;
+        for (int j0 = j_lo; j0 + (lead + wave) * 4 < j_hi; j0 += AT_ONCE * 4 * TW) {   // wave-uniform
+            if (j0 > j_lo) {
+                request(kv, L, j0);
+                now = counts(j0);
             }
-        };
-        // -------------------------------------------------------------- rotary, append, attention
-        // Two branches with the same barriers: the waves that attend rebuild o_proj's weights afterwards, the others
-        // meanwhile, and neither's registers hold both the weights and the keys and values.
-        Built built_o;
-        if (wave >= my_waves) {
-            publish_qkv();
-            build_ahead(P_O, built_o);
-            if (attends) {
-                lds_barrier();
-                if (ranges) lds_barrier();
-            }
-        } else {
-            Slots kv;
-            request(kv, L, j_lo);
-            publish_qkv();
-            if (wave == 0) {
-                // lanes 0..15 the query's dimensions 4 i ... and 64 + 4 i ..., 16..31 the key's, 32..47 the value's (48..63 too)
-                const int part = kq, row_words = (A + 2 * KV) >> 1;
-                const int at = (part == 0 ? ah * 64 : (part == 1 ? A >> 1 : (A + KV) >> 1) + akv * 64) + 2 * lc;
-                uint32_t x[4];
-                await_pairs<2>(x, number + 1, budget, a.e_qkv, M * row_words, [&](int) { return at; },
-                               [&](int i) { return am * row_words + 32 * i; });
-                if (part < 2) {   // bf16(bf16(x cos) + bf16(rotate_half(x) sin))
-                    auto round = [](float v) { return low_bf16(pack_bf16_rne(v, 0.0f)); };
-                    const u32x2_t c0 = *reinterpret_cast<const u32x2_t *>(turn + 2 * lc), c1 = *reinterpret_cast<const u32x2_t *>(turn + 32 + 2 * lc);
-                    const u32x2_t s0 = *reinterpret_cast<const u32x2_t *>(turn + 64 + 2 * lc), s1 = *reinterpret_cast<const u32x2_t *>(turn + 96 + 2 * lc);
 #pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const float a0 = low_bf16(x[e]), a1 = high_bf16(x[e]), b0 = low_bf16(x[2 + e]), b1 = high_bf16(x[2 + e]);
-                        x[e] = pack_bf16_rne(round(a0 * low_bf16(c0[e])) + round(-b0 * low_bf16(s0[e])),
-                                             round(a1 * high_bf16(c0[e])) + round(-b1 * high_bf16(s0[e])));
-                        x[2 + e] = pack_bf16_rne(round(b0 * low_bf16(c1[e])) + round(a0 * low_bf16(s1[e])),
-                                                 round(b1 * high_bf16(c1[e])) + round(a1 * high_bf16(s1[e])));
-                    }
+            for (int b = 0; b < AT_ONCE; b += BATCH) {
+                if (slot_of(j0, b) - kq >= j_hi) break;   // wave-uniform: nothing in the rest
+                float dot[BATCH] = {0.f, 0.f, 0.f, 0.f}, sc[BATCH], m2 = mx;
+                dot4(dot, q4, kv.k + b);
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u) {
+                    dot[u] = row16_sum(dot[u]);   // the sixteen lanes that share the slot
+                    sc[u] = now >> (b + u) & 1 ? dot[u] * scaling : -INFINITY;
+                    m2 = fmaxf(m2, sc[u]);
                 }
-                uint32_t *out = (part == 0 ? qs : part == 1 ? ks : vs) + 2 * lc;
-                *reinterpret_cast<u32x2_t *>(out) = u32x2_t{x[0], x[1]};
-                *reinterpret_cast<u32x2_t *>(out + 32) = u32x2_t{x[2], x[3]};
-                if (appends && p >= 0 && part > 0) {
-                    gptr_w to = (gptr_w)(uintptr_t)(static_cast<uint16_t *>(part == 1 ? L->k_cache : L->v_cache) + cache_base() +
-                                                    (long)p * HEAD_DIM) + 2 * lc;
-                    to[0] = x[0], to[1] = x[1], to[32] = x[2], to[33] = x[3];
-                }
-            }
-            lds_barrier();
-            {
-                const float scaling = L->scaling;
-                const u32x4_t q4 = *reinterpret_cast<const u32x4_t *>(qs + lc * 4);
-                float mx = -INFINITY, sum = 0.0f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                uint32_t now = live;
-                for (int j0 = j_lo; j0 + (lead + wave) * 4 < j_hi; j0 += AT_ONCE * 4 * TW) {   // wave-uniform
-                    if (j0 > j_lo) {
-                        request(kv, L, j0);
-                        now = counts(j0);
-                    }
+                const float ref = m2 == -INFINITY ? 0.0f : m2, c0 = __expf(mx - ref);
+                mx = m2;
 #pragma unroll
-                    for (int b = 0; b < AT_ONCE; b += BATCH) {
-                        if (slot_of(j0, b) - kq >= j_hi) break;   // wave-uniform: nothing in the rest
-                        float dot[BATCH] = {0.f, 0.f, 0.f, 0.f}, sc[BATCH], m2 = mx;
-                        dot4(dot, q4, kv.k + b);
-#pragma unroll
-                        for (int u = 0; u < BATCH; ++u) {
-                            dot[u] = row16_sum(dot[u]);   // the sixteen lanes that share the slot
-                            sc[u] = now >> (b + u) & 1 ? dot[u] * scaling : -INFINITY;
-                            m2 = fmaxf(m2, sc[u]);
-                        }
-                        const float ref = m2 == -INFINITY ? 0.0f : m2, c0 = __expf(mx - ref);
-                        mx = m2;
-#pragma unroll
-                        for (int u = 0; u < BATCH; ++u) {
-                            const float w = __expf(sc[u] - ref);
-                            sum = u ? sum + w : __builtin_fmaf(sum, c0, w);
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) {
-                                const float v = e & 1 ? high_bf16(kv.v[b + u][e >> 1]) : low_bf16(kv.v[b + u][e >> 1]);
-                                acc[e] = u ? __builtin_fmaf(w, v, acc[e]) : __builtin_fmaf(acc[e], c0, w * v);
-                            }
-                        }
-                    }
-                }
-                // the wave's four groups, 0 with 1 and 2 with 3, then both; what group 0 holds then counts
-#pragma unroll
-                for (int step = 0; step < 2; ++step) {
-                    float m1 = mx, m2 = mx, l1 = sum, l2 = sum;
-                    step ? swap_32(m1, m2) : swap_16(m1, m2);
-                    step ? swap_32(l1, l2) : swap_16(l1, l2);
-                    mx = fmaxf(m1, m2);
-                    const float ref = mx == -INFINITY ? 0.0f : mx, c1 = __expf(m1 - ref), c2 = __expf(m2 - ref);
-                    sum = __builtin_fmaf(l1, c1, l2 * c2);
+                for (int u = 0; u < BATCH; ++u) {
+                    const float w = __expf(sc[u] - ref);
+                    sum = u ? sum + w : __builtin_fmaf(sum, c0, w);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        float a1 = acc[e], a2 = acc[e];
-                        step ? swap_32(a1, a2) : swap_16(a1, a2);
-                        // (which product is rounded: as each build of rope_attn_decode_kernel came out of the compiler)
-                        acc[e] = e < 5 || a.split_build ? __builtin_fmaf(a2, c2, a1 * c1) : __builtin_fmaf(a1, c1, a2 * c2);
+                        const float v = e & 1 ? high_bf16(kv.v[b + u][e >> 1]) : low_bf16(kv.v[b + u][e >> 1]);
+                        acc[e] = u ? __builtin_fmaf(w, v, acc[e]) : __builtin_fmaf(acc[e], c0, w * v);
                     }
                 }
-                if (ranges) {
-                    if (kq == 0) {
-                        *reinterpret_cast<f32x4_t *>(pacc + wave * HEAD_DIM + lc * 8) = f32x4_t{acc[0], acc[1], acc[2], acc[3]};
-                        *reinterpret_cast<f32x4_t *>(pacc + wave * HEAD_DIM + lc * 8 + 4) = f32x4_t{acc[4], acc[5], acc[6], acc[7]};
-                    }
-                    if (lane == 0) pm[wave] = mx, pl[wave] = sum;
-                } else if (kq == 0) {
-                    uint64_t *state = a.e_part + (long)(pair * STATES + lead + wave) * STATE;
+            }
+        }
+        // the wave's four groups, 0 with 1 and 2 with 3, then both; what group 0 holds then counts
 #pragma unroll
-                    for (int e = 0; e < 8; e += 2)
-                        put_pair(state, STATE, lc * 8 + e, __builtin_bit_cast(uint32_t, acc[e]), __builtin_bit_cast(uint32_t, acc[e + 1]), number + 2);
-                    if (lane == 0)
-                        put_pair(state, STATE, HEAD_DIM, __builtin_bit_cast(uint32_t, mx), __builtin_bit_cast(uint32_t, sum), number + 2);
-                }
-            }
-            if (ranges) lds_barrier();
-            if (wave == 0) {
-                // n states in LDS (pacc, pm, pl) joined in order for columns col, col + 1, the token's own slot first
-                float o0 = 0.0f, o1 = 0.0f, total, top;
-                float own = -INFINITY;   // the new token's own slot, where this workgroup counts it
-                if (own_slot) {
-                    const uint16_t *q = reinterpret_cast<const uint16_t *>(qs), *k = reinterpret_cast<const uint16_t *>(ks);
-                    const float dot = bf16_bits_to_f32(q[lane]) * bf16_bits_to_f32(k[lane]);
-                    own = wave_sum(__builtin_fmaf(bf16_bits_to_f32(q[lane + 64]), bf16_bits_to_f32(k[lane + 64]), dot)) * L->scaling;
-                }
-                auto join_states = [&](int n, int col, float own) {
-                    const float m_w = lc < n ? pm[lc] : -INFINITY, l_w = lc < n ? pl[lc] : 0.0f;   // lane w of sixteen: state w
-                    top = fmaxf(own, row16_max(m_w));
-                    const float ref = top == -INFINITY ? 0.0f : top, c_w = __expf(m_w - ref), c_own = __expf(own - ref);
-                    const float v0 = low_bf16(vs[col >> 1]), v1 = high_bf16(vs[col >> 1]);
-                    total = c_own;
+        for (int step = 0; step < 2; ++step) {
+            float m1 = mx, m2 = mx, l1 = sum, l2 = sum;
+            step ? swap_32(m1, m2) : swap_16(m1, m2);
+            step ? swap_32(l1, l2) : swap_16(l1, l2);
+            mx = fmaxf(m1, m2);
+            const float ref = mx == -INFINITY ? 0.0f : mx, c1 = __expf(m1 - ref), c2 = __expf(m2 - ref);
+            sum = __builtin_fmaf(l1, c1, l2 * c2);
 #pragma unroll
-                    for (int w = 0; w < TW; ++w)
-                        if (w < n) {   // uniform
-                            const float2 v = *reinterpret_cast<const float2 *>(pacc + w * HEAD_DIM + col);
-                            const float c = lane_of(c_w, w);
-                            o0 = w ? __builtin_fmaf(c, v.x, o0) : __builtin_fmaf(c_own, v0, c * v.x);
-                            o1 = w ? __builtin_fmaf(c, v.y, o1) : __builtin_fmaf(c_own, v1, c * v.y);
-                            total = __builtin_fmaf(c, lane_of(l_w, w), total);
-                        }
-                };
-                int col = 2 * lane;
-                if (ranges) join_states(TW, col, own);
-                {
-                    const int n = ranges ? splits : TW;   // states of the pair
-                    uint64_t *states = a.e_part + (long)pair * STATES * STATE;
-                    if (ranges) {
-                        put_pair(states, STATES * STATE, split * STATE + col, __builtin_bit_cast(uint32_t, o0), __builtin_bit_cast(uint32_t, o1), number + 2);
-                        if (lane == 0)
-                            put_pair(states, STATES * STATE, split * STATE + HEAD_DIM, __builtin_bit_cast(uint32_t, top), __builtin_bit_cast(uint32_t, total), number + 2);
-                    }
-                    // this workgroup's share of the columns: lane, load -> (state, column pair); last (maximum, sum)
-                    constexpr int PAIRS = (HEAD_DIM / 2) / splits, PER_LOAD = WAVE / PAIRS, LOADS = STATES / PER_LOAD;
-                    const int z = lane / PAIRS, c = lane % PAIRS, col0 = split * (HEAD_DIM / splits);
-                    uint32_t st[2 * LOADS + 2];
-                    await_pairs<1 + LOADS>(st, number + 2, budget, states, STATES * STATE, [&](int i) {   // (past n: repeats)
-                        return i == 0 ? min(lc, n - 1) * STATE + HEAD_DIM : min(z + (i - 1) * PER_LOAD, n - 1) * STATE + col0 + 2 * c;
-                    }, [](int) { return 0; });
-                    wave_fence();   // (what the join above read)
-                    pm[lc] = __builtin_bit_cast(float, st[0]), pl[lc] = __builtin_bit_cast(float, st[1]);
+            for (int e = 0; e < 8; ++e) {
+                float a1 = acc[e], a2 = acc[e];
+                step ? swap_32(a1, a2) : swap_16(a1, a2);
+                // (which product is rounded: as each build of rope_attn_decode_kernel came out of the compiler)
+                acc[e] = e < 5 || a.split_build ? __builtin_fmaf(a2, c2, a1 * c1) : __builtin_fmaf(a1, c1, a2 * c2);
+            }
+        }
+        if (ranges) {
+            if (kq == 0) {
+                *reinterpret_cast<f32x4_t *>(pacc + wave * HEAD_DIM + lc * 8) = f32x4_t{acc[0], acc[1], acc[2], acc[3]};
+                *reinterpret_cast<f32x4_t *>(pacc + wave * HEAD_DIM + lc * 8 + 4) = f32x4_t{acc[4], acc[5], acc[6], acc[7]};
+            }
+            if (lane == 0) pm[wave] = mx, pl[wave] = sum;
+        } else if (kq == 0) {
+            uint64_t *state = a.e_part + (long)(pair * STATES + lead + wave) * STATE;
 #pragma unroll
-                    for (int i = 0; i < LOADS; ++i)
-                        *reinterpret_cast<float2 *>(pacc + min(z + i * PER_LOAD, n - 1) * HEAD_DIM + col0 + 2 * c) =
-                            float2{__builtin_bit_cast(float, st[2 + 2 * i]), __builtin_bit_cast(float, st[3 + 2 * i])};
-                    wave_fence();
-                    col = col0 + 2 * c;
-                    join_states(n, col, ranges ? -INFINITY : own);
+            for (int e = 0; e < 8; e += 2)
+                put_pair(state, STATE, lc * 8 + e, __builtin_bit_cast(uint32_t, acc[e]), __builtin_bit_cast(uint32_t, acc[e + 1]), number + 2);
+            if (lane == 0)
+                put_pair(state, STATE, HEAD_DIM, __builtin_bit_cast(uint32_t, mx), __builtin_bit_cast(uint32_t, sum), number + 2);
+        }
+    };
+    // wave 0: the states of this workgroup's waves joined into one and handed on (`ranges` only), and the pair's states
+    // joined for this workgroup's share of the columns
+    struct Joined { float o0, o1, total, top; };
+    auto own_score = [&](layer_ptr L) __attribute__((always_inline)) {
+        float own = -INFINITY;   // the new token's own slot, where this workgroup counts it
+        if (own_slot) {
+            const uint16_t *q = reinterpret_cast<const uint16_t *>(qs), *k = reinterpret_cast<const uint16_t *>(ks);
+            const float dot = bf16_bits_to_f32(q[lane]) * bf16_bits_to_f32(k[lane]);
+            own = wave_sum(__builtin_fmaf(bf16_bits_to_f32(q[lane + 64]), bf16_bits_to_f32(k[lane + 64]), dot)) * L->scaling;
+        }
+        return own;
+    };
+    // n states in LDS (pacc, pm, pl) joined in order for columns col, col + 1, the token's own slot first
+    auto join_states = [&](int n, int col, float own) {
+        float o0 = 0.0f, o1 = 0.0f, total, top;
+            const float m_w = lc < n ? pm[lc] : -INFINITY, l_w = lc < n ? pl[lc] : 0.0f;   // lane w of sixteen: state w
+            top = fmaxf(own, row16_max(m_w));
+            const float ref = top == -INFINITY ? 0.0f : top, c_w = __expf(m_w - ref), c_own = __expf(own - ref);
+            const float v0 = low_bf16(vs[col >> 1]), v1 = high_bf16(vs[col >> 1]);
+            total = c_own;
+#pragma unroll
+            for (int w = 0; w < TW; ++w)
+                if (w < n) {   // uniform
+                    const float2 v = *reinterpret_cast<const float2 *>(pacc + w * HEAD_DIM + col);
+                    const float c = lane_of(c_w, w);
+                    o0 = w ? __builtin_fmaf(c, v.x, o0) : __builtin_fmaf(c_own, v0, c * v.x);
+                    o1 = w ? __builtin_fmaf(c, v.y, o1) : __builtin_fmaf(c_own, v1, c * v.y);
+                    total = __builtin_fmaf(c, lane_of(l_w, w), total);
                 }
-                // every slot masked: zeros (not where they stand for a query that did not come: then 0 / 0)
-                if (top == -INFINITY && budget) o0 = o1 = 0.0f, total = 1.0f;
-                if (lane < (HEAD_DIM / 2) / splits)
-                    put_word(a.e_attn + am * (A >> 1) + ((ah * HEAD_DIM + col) >> 1), pack_bf16_rne(o0 / total, o1 / total), number + 3);
+        return Joined{o0, o1, total, top};
+    };
+    auto leave_state = [&](float own) __attribute__((always_inline)) {
+        const int col = 2 * lane;
+        const Joined s = join_states(TW, col, own);
+        uint64_t *states = a.e_part + (long)pair * STATES * STATE;
+        put_pair(states, STATES * STATE, split * STATE + col, __builtin_bit_cast(uint32_t, s.o0), __builtin_bit_cast(uint32_t, s.o1), number + 2);
+        if (lane == 0)
+            put_pair(states, STATES * STATE, split * STATE + HEAD_DIM, __builtin_bit_cast(uint32_t, s.top), __builtin_bit_cast(uint32_t, s.total), number + 2);
+    };
+    auto join_pair = [&](float own) __attribute__((always_inline)) {
+        const int n = ranges ? splits : TW;   // states of the pair
+        const uint64_t *states = a.e_part + (long)pair * STATES * STATE;
+        // this workgroup's share of the columns: lane, load -> (state, column pair); last (maximum, sum)
+        constexpr int PAIRS = (HEAD_DIM / 2) / splits, PER_LOAD = WAVE / PAIRS, LOADS = STATES / PER_LOAD;
+        const int z = lane / PAIRS, c = lane % PAIRS, col0 = split * (HEAD_DIM / splits);
+        uint32_t st[2 * LOADS + 2];
+        await_pairs<1 + LOADS>(st, number + 2, budget, states, STATES * STATE, [&](int i) {   // (past n: repeats)
+            return i == 0 ? min(lc, n - 1) * STATE + HEAD_DIM : min(z + (i - 1) * PER_LOAD, n - 1) * STATE + col0 + 2 * c;
+        }, [](int) { return 0; });
+        wave_fence();   // (what was read there before)
+        pm[lc] = __builtin_bit_cast(float, st[0]), pl[lc] = __builtin_bit_cast(float, st[1]);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            *reinterpret_cast<float2 *>(pacc + min(z + i * PER_LOAD, n - 1) * HEAD_DIM + col0 + 2 * c) =
+                float2{__builtin_bit_cast(float, st[2 + 2 * i]), __builtin_bit_cast(float, st[3 + 2 * i])};
+        wave_fence();
+        const int col = col0 + 2 * c;
+        Joined s = join_states(n, col, ranges ? -INFINITY : own);
+        // every slot masked: zeros (not where they stand for a query that did not come: then 0 / 0)
+        if (s.top == -INFINITY && budget) s.o0 = s.o1 = 0.0f, s.total = 1.0f;
+        if (lane < (HEAD_DIM / 2) / splits)
+            put_word(a.e_attn + am * (A >> 1) + ((ah * HEAD_DIM + col) >> 1), pack_bf16_rne(s.o0 / s.total, s.o1 / s.total), number + 3);
+    };
+    auto join = [&](int nsc, uint64_t *words, uint32_t n, uint16_t *h_out) {
+        lds_barrier();
+        if (wave == 0) {
+            const float2 s = tile_sum(1, 0, nsc);
+            const uint32_t y = pack_bf16_rne(s.x, s.y);
+            stream = pack_bf16_rne(low_bf16(stream) + low_bf16(y), high_bf16(stream) + high_bf16(y));
+            if (stores()) {
+                put_word(words + stream_word(), stream, n);
+                if (h_out) ((gptr_w)(uintptr_t)h_out)[stream_word()] = stream;
             }
-            build_ahead(P_O, built_o);
         }
-        // -------------------------------------------------------------- o_proj, joined with the residual stream
-        auto join = [&](int nsc, uint64_t *words, uint32_t n, uint16_t *h_out) {
-            lds_barrier();
-            if (wave == 0) {
-                const float2 s = tile_sum(1, 0, nsc);
-                const uint32_t y = pack_bf16_rne(s.x, s.y);
-                stream = pack_bf16_rne(low_bf16(stream) + low_bf16(y), high_bf16(stream) + high_bf16(y));
-                if (stores()) {
-                    put_word(words + stream_word(), stream, n);
-                    if (h_out) ((gptr_w)(uintptr_t)h_out)[stream_word()] = stream;
-                }
-            }
-        };
-        own_product(P_O, built_o, a.e_attn, A, number + 3, P_GATE_UP, l);
-        if (has_h) join(a.nsc_a, a.e_mid, number + 4, nullptr);
-        // -------------------------------------------------------------- norm, gate|up, SiLU
-        {
-            Rows<MW, C::P2> x;
-            Built built;
-            undefined(x);
-            build_ahead(P_GATE_UP, built);
-            if (slots_i) take_rows(P2, x, L->norm2, a.e_mid, number + 4);
-            load(P_DOWN, l);
-            if (slots_i) {
-                normalise(P2, x, L->eps2);
-                multiply_staged(P_GATE_UP, built);
-            }
+    };
+    auto publish_act = [&]() {
+        lds_barrier();
+        if (wave < slots_i) {
+            const float2 g = tile_sum(0, 2 * wave * NSC, NSC), u = tile_sum(0, (2 * wave + 1) * NSC, NSC);
+            const float x = g.x / (1.0f + __expf(-g.x)) * u.x, y = g.y / (1.0f + __expf(-g.y)) * u.y;
+            if (stores())
+                put_word(a.e_act + tile_row() * (I >> 1) + (wg + wave * G) * 8 + (lane & 7), pack_bf16_rne(x, y), number + 5);
         }
-        if (slots_i) {
-            lds_barrier();
-            if (wave < slots_i) {
-                const float2 g = tile_sum(0, 2 * wave * NSC, NSC), u = tile_sum(0, (2 * wave + 1) * NSC, NSC);
-                const float x = g.x / (1.0f + __expf(-g.x)) * u.x, y = g.y / (1.0f + __expf(-g.y)) * u.y;
-                if (stores())
-                    put_word(a.e_act + tile_row() * (I >> 1) + (wg + wave * G) * 8 + (lane & 7), pack_bf16_rne(x, y), number + 5);
-            }
-        }
-        // -------------------------------------------------------------- down_proj, joined with the residual stream
-        {
-            Built built;
-            build_ahead(P_DOWN, built);
-            own_product(P_DOWN, built, a.e_act, I, number + 5, P_QKV, l + 1);
-            if (has_h) join(a.nsc_i, a.e_out, number + 6, l + 1 == a.n_layers ? again()->h_out : nullptr);
-        }
-    }
-    // ---- the model's norm, a workgroup per row
-    const arg_ptr t = again();
-    if (t->normed && wg < M) {
+    };
+    // the model's norm, a workgroup per row
+    const auto last_norm = [&](int row) __attribute__((always_inline)) {
+        const arg_ptr t = again();
         // add_rmsnorm_kernel's order of sums: four waves, eight neighbouring values of every 2048 per lane
         uint32_t x[4];
         if (wave < 4) {
-            await_pairs<2>(x, first + 8u * t->n_layers + 6u, budget, a.e_out, M * ROW_WORDS,
-                                    [&](int) { return 4 * tid; }, [&](int i) { return wg * ROW_WORDS + i * 2; });
+            await_pairs<2>(x, number + 6, budget, a.e_out, M * ROW_WORDS,
+                                    [&](int) { return 4 * tid; }, [&](int i) { return row * ROW_WORDS + i * 2; });
             float ss = 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -766,14 +761,244 @@ __global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
                 const uint32_t n = pack_bf16_rne(low_bf16(x[e]) * r, high_bf16(x[e]) * r);
                 y[e] = pack_bf16_rne(low_bf16(w[e]) * low_bf16(n), high_bf16(w[e]) * high_bf16(n));
             }
-            ((__attribute__((address_space(1))) u32x4_t *)(uintptr_t)t->normed)[wg * (H / 8) + tid] = y;
+            ((__attribute__((address_space(1))) u32x4_t *)(uintptr_t)t->normed)[row * (H / 8) + tid] = y;
+        }
+    };
+
+    // ---- who takes part (wave TW - 1 sees to it): a ticket once this launch's number is known ...
+    struct Ticket { uint32_t first, rank; };
+    auto arrive = [&](Ticket &mine) {
+        TrunkState *const state = again()->state;
+        if (lane == 0) {
+            mine.first = __hip_atomic_load(&state->number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(mine.first)::"memory");   // read before the ticket: the last one counts it up
+            mine.rank = __hip_atomic_fetch_add(&state->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    };
+    // ... and the team: whoever offers first.  Afterwards all threads know the number; returns the team's size.
+    auto settle = [&](const Ticket &mine) {
+        if (wave == TW - 1 && lane == 0) {
+            const arg_ptr t = again();
+            TrunkState *const state = t->state;
+            const uint32_t first = mine.first, all = G, most = t->most;
+            uint64_t seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (mine.rank + 1 == all) {   // every workgroup has read the number: the next launch's, and a new count
+                __hip_atomic_store(&state->number, first + 8u + 8u * t->n_layers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&state->arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            uint32_t offer = mine.rank + 1 == most ? most : 0u;
+            const uint64_t since = __builtin_readsteadycounter();
+            while ((uint32_t)(seen >> 32) != first + 8u) {
+                if (offer) {
+                    const uint64_t team = (uint64_t)(first + 8u) << 32 | offer;
+                    if (__hip_atomic_compare_exchange_strong(&state->team, &seen, team, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT))
+                        seen = team;
+                    continue;
+                }
+                const uint32_t count = __hip_atomic_load(&state->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t here = count == 0u ? most : min(count, most);   // (0: put back, all have arrived)
+                const uint64_t waited = __builtin_readsteadycounter() - since;
+                if (waited >= TEAM_TICKS_LEAST && waited * here >= (uint64_t)t->n_layers * TEAM_TICKS) offer = here;
+                seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            joined[0] = first + 8u, joined[1] = mine.rank, joined[2] = (uint32_t)seen;
+        }
+        lds_barrier();
+        number = __builtin_amdgcn_readfirstlane(joined[0]);
+        return (int)__builtin_amdgcn_readfirstlane(joined[2]);
+    };
+
+    // ---- the team is not the whole grid: every product's parts are dealt out to its members, one after the other
+    if constexpr (SHARED) {
+        number = __builtin_amdgcn_readfirstlane(joined[0]);
+        const int rank = __builtin_amdgcn_readfirstlane(joined[1]), team = __builtin_amdgcn_readfirstlane(joined[2]);
+        if (rank >= team) return;   // left out
+        auto deal = [&](int parts, auto work) __attribute__((always_inline)) {
+            for (int part = rank; part < parts; part += team) {
+                forget();
+                wg = part;
+                work();
+                lds_barrier();   // LDS is free for the next part
+            }
+        };
+        const uint64_t *h_words = nullptr;   // the residual stream where the product before left it
+        auto take_stream = [&](uint32_t n) {   // wave 0
+            if (!h_words) return begin_stream();
+            uint64_t w;
+            for (;;) {
+                w = stores() ? __hip_atomic_load(h_words + stream_word(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (uint64_t)n << 32;
+                if (__builtin_amdgcn_ballot_w64((uint32_t)(w >> 32) != n) == 0 || budget == 0) break;
+                --budget;
+            }
+            stream = (uint32_t)(w >> 32) == n ? (uint32_t)w : NOT_COME;
+        };
+        for (int l = 0; l < a.n_layers; ++l, number += 8) {
+            const layer_ptr L = (layer_ptr)(uintptr_t)a.layers + l;
+            deal(G, [&]() {
+                place_tiles();
+                if (!slots_qkv) return;
+                Rows<MW, C::P1> x;
+                Built built;
+                undefined(x);
+                load(P_QKV, l);
+                build_ahead(P_QKV, built);
+                take_rows(P1, x, L->norm1, a.e_out, number - 2, l == 0 ? again()->cur : nullptr);
+                normalise(P1, x, L->eps1);
+                multiply_staged(P_QKV, built);
+                publish_qkv();
+            });
+            deal(M * heads * splits, [&]() {
+                place_pair();
+                Slots kv;
+                live = wave < my_waves ? counts(j_lo) : 0u;
+                if (wave < my_waves) request(kv, L, j_lo);
+                if (wave == 0) receive_token(L, true);
+                lds_barrier();
+                if (wave < my_waves) score_slots(L, kv);
+                if (!ranges) return;
+                lds_barrier();
+                if (wave == 0) leave_state(own_score(L));
+            });
+            deal(M * heads * splits, [&]() {
+                place_pair();
+                if (wave != 0) return;
+                wave_fence();
+                receive_token(L, false);
+                wave_fence();
+                join_pair(own_score(L));
+            });
+            deal(G, [&]() {
+                place_tiles();
+                Built built;
+                load(P_O, l);
+                build_ahead(P_O, built);
+                own_product(P_O, built, a.e_attn, A, number + 3, P_QKV, a.n_layers);
+                if (!has_h) return;
+                if (wave == 0) take_stream(number - 2);
+                join(a.nsc_a, a.e_mid, number + 4, nullptr);
+            });
+            h_words = a.e_mid;
+            deal(G, [&]() {
+                place_tiles();
+                if (!slots_i) return;
+                Rows<MW, C::P2> x;
+                Built built;
+                undefined(x);
+                load(P_GATE_UP, l);
+                build_ahead(P_GATE_UP, built);
+                take_rows(P2, x, L->norm2, a.e_mid, number + 4);
+                normalise(P2, x, L->eps2);
+                multiply_staged(P_GATE_UP, built);
+                publish_act();
+            });
+            deal(G, [&]() {
+                place_tiles();
+                Built built;
+                load(P_DOWN, l);
+                build_ahead(P_DOWN, built);
+                own_product(P_DOWN, built, a.e_act, I, number + 5, P_QKV, a.n_layers);
+                if (!has_h) return;
+                if (wave == 0) take_stream(number + 4);
+                join(a.nsc_i, a.e_out, number + 6, l + 1 == a.n_layers ? again()->h_out : nullptr);
+            });
+            h_words = a.e_out;
+        }
+        number -= 8;
+        if (again()->normed) deal(M, [&]() { last_norm(wg); });
+        return;
+    }
+
+    // ---- everyone is there
+    begin_stream();
+    load(P_QKV, 0);
+    for (int l = 0; l < a.n_layers; ++l) {
+        const layer_ptr L = (layer_ptr)(uintptr_t)a.layers + l;
+        forget();
+        opaque(am), opaque(ah), opaque(akv);
+        // -------------------------------------------------------------- norm, q|k|v
+        Ticket ticket{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u)};   // (the first layer's)
+        {
+            Rows<MW, C::P1> x;
+            Built built;
+            undefined(x);
+            build_ahead(P_QKV, built);
+            if (l == 0 && wave == TW - 1) arrive(ticket);
+            number += 8;
+            if (slots_qkv) take_rows(P1, x, L->norm1, a.e_out, number - 2, l == 0 ? again()->cur : nullptr);   // the sixth exchange of the layer before
+            load(P_O, l);
+            if (slots_qkv) {
+                normalise(P1, x, L->eps1);
+                multiply_staged(P_QKV, built);
+            }
+        }
+        if (l == 0) {
+            const int team = settle(ticket);
+            if (__builtin_expect(team != G, 0)) return share_out<C>(args, (lds_ptr)smem);
+        }
+        // -------------------------------------------------------------- rotary, append, attention
+        // Two branches with the same barriers: the waves that attend rebuild o_proj's weights afterwards, the others
+        // meanwhile, and neither's registers hold both the weights and the keys and values.
+        Built built_o;
+        if (wave >= my_waves) {
+            publish_qkv();
+            build_ahead(P_O, built_o);
+            if (attends) lds_barrier();   // (with ranges every wave attends)
+        } else {
+            Slots kv;
+            request(kv, L, j_lo);
+            publish_qkv();
+            if (wave == 0) receive_token(L, true);
+            lds_barrier();
+            score_slots(L, kv);
+            if (ranges) lds_barrier();
+            if (wave == 0) {
+                const float own = own_score(L);
+                if (ranges) leave_state(own);
+                join_pair(own);
+            }
+            build_ahead(P_O, built_o);
+        }
+        // -------------------------------------------------------------- o_proj, joined with the residual stream
+        own_product(P_O, built_o, a.e_attn, A, number + 3, P_GATE_UP, l);
+        if (has_h) join(a.nsc_a, a.e_mid, number + 4, nullptr);
+        // -------------------------------------------------------------- norm, gate|up, SiLU
+        {
+            Rows<MW, C::P2> x;
+            Built built;
+            undefined(x);
+            build_ahead(P_GATE_UP, built);
+            if (slots_i) take_rows(P2, x, L->norm2, a.e_mid, number + 4);
+            load(P_DOWN, l);
+            if (slots_i) {
+                normalise(P2, x, L->eps2);
+                multiply_staged(P_GATE_UP, built);
+            }
+        }
+        if (slots_i) publish_act();
+        // -------------------------------------------------------------- down_proj, joined with the residual stream
+        {
+            Built built;
+            build_ahead(P_DOWN, built);
+            own_product(P_DOWN, built, a.e_act, I, number + 5, P_QKV, l + 1);
+            if (has_h) join(a.nsc_i, a.e_out, number + 6, l + 1 == a.n_layers ? again()->h_out : nullptr);
         }
     }
-    // Every workgroup with a part in the step has read the counter: what this one has seen goes back to all of them.
-    if (wg == 0) {
-        lds_barrier();
-        if (tid == 0) *t->counter = first + 8u + 8u * t->n_layers;
-    }
+    if (again()->normed && wg < M) last_norm(wg);
+}
+
+template <class C>
+__device__ __attribute__((noinline)) void share_out(arg_ptr args, lds_ptr smem) {
+    const uint64_t at = (uint64_t)(uintptr_t)args;   // (uniform; not known to be, where it arrives)
+    args = (arg_ptr)(uintptr_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 |
+                                (uint32_t)__builtin_amdgcn_readfirstlane((int)at));
+    trunk_step<C, true>(*(const TrunkArgs *)args, args, (uint8_t *)smem);
+}
+
+template <class C>
+__global__ __launch_bounds__(TT) void decode_trunk_kernel(TrunkArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    trunk_step<C, false>(a, (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr(), smem);
 }
 
 // ---------------------------------------------------------------- host side
@@ -835,7 +1060,7 @@ bool trunk_plan(const vrl_trunk &t, TrunkPlan &plan) {
                              (size_t)t.M * t.n_heads * STATES * STATE,
                              (size_t)t.M * A / 2, (size_t)t.M * t.hidden / 2, (size_t)t.M * t.inter / 2,
                              (size_t)t.M * t.hidden / 2};
-    plan.bytes = 256;   // the counter
+    plan.bytes = 256;   // TrunkState
     for (int i = 0; i < 6; ++i) {
         plan.words[i] = words[i];
         plan.bytes += (words[i] * 8 + 255) / 256 * 256;
@@ -907,12 +1132,14 @@ extern "C" int vrl_decode_trunk_bf16(const vrl_trunk *trunk, void *hip_stream) {
     a.kv_heads = t.n_kv_heads;
     a.L_max = t.L_max;
     a.budget = t.wait_limit ? t.wait_limit : TRUNK_BUDGET;
+    a.grid = plan.grid;
+    a.most = t.max_workgroups ? (int)std::min(t.max_workgroups, (uint32_t)plan.grid) : plan.grid;
     a.nsc_a = pp_nsc(a.A);
     a.nsc_i = pp_nsc(a.I);
     a.split_build = t.split_from > 0;
     a.split_from = a.split_build ? t.split_from : INT32_MAX;
     uint8_t *ws = static_cast<uint8_t *>(t.workspace);
-    a.counter = reinterpret_cast<uint32_t *>(ws);
+    a.state = reinterpret_cast<TrunkState *>(ws);
     uint64_t **const at[6] = {&a.e_qkv, &a.e_part, &a.e_attn, &a.e_mid, &a.e_act, &a.e_out};
     size_t offset = 256;
     for (int i = 0; i < 6; ++i) {
