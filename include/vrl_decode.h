@@ -249,8 +249,9 @@ int vrl_decode_run_calls(const vrl_step_call *calls, int n_calls, int *failed_at
  *   workspace vrl_decode_trunk_workspace_bytes() bytes of device memory, 256-byte aligned, zero before the first
  *             launch that uses it and left to the launches from then on.  Launches that share one must be ordered.
  *   wait_limit  0, or how often a wave looks for a result of another workgroup in vain before it takes NaN for it
- *             and waits no more (default 2^22): every wait ends, and a launch that gave up has NaN in its output.
- *             Its workspace has to be zeroed before the next launch.
+ *             and waits no more (default 2^22, seconds; every workgroup waited for is running): every wait ends, and
+ *             a launch that gave up has NaN in its output and in the cache slot of the new token.  Later launches over
+ *             its workspace write NaN as their output and nothing else, until it is zeroed.
  *   max_workgroups  0, or how many workgroups take part at most (the others end at once)
  * vrl_decode_trunk_workspace_bytes returns 0 where the launch does not apply (the other fields may then be NULL).
  * It applies to M <= 4, hidden 2048, head_dim 128, group_size 128, L_max <= 8192, n_heads * 128 a multiple of 256

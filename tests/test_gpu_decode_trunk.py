@@ -292,6 +292,26 @@ def test_other_steps_keep_the_list(kwargs):
     assert torch.isfinite(step.run(False)[0]).all()
 
 
+@pytest.mark.parametrize("final_norm", [True, False])
+def test_a_workspace_that_was_given_up_on_says_so(final_norm):
+    """Steps over it touch no cache and have NaN in every value, until it is zeroed."""
+    print("decode trunk: given up", final_norm, flush=True)
+    step = Step(3, final_norm=final_norm)
+    want, want_cache = step.run(False)
+    for desc in step.one:
+        desc.wait_limit = 1
+    assert step.run(True)[0].isnan().any()
+    for desc in step.one:
+        desc.wait_limit = 0
+    for _ in range(2):
+        got, cache = step.run(True)
+        assert got.isnan().all() and all(torch.equal(a, b) for a, b in zip(cache, step.cache))
+    (workspace,) = [t for t in step.native._keep if torch.is_tensor(t) and t.data_ptr() == step.one[0].workspace]
+    workspace.zero_()
+    got, cache = step.run(True)
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(cache, want_cache))
+
+
 def test_refusals():
     """Checks of the entry point, before any launch."""
     print("decode trunk: refusals", flush=True)

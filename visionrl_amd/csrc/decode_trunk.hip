@@ -36,7 +36,8 @@
 // handed out, so that the tickets cost next to nothing.
 //
 // Waits are bounded all the same: a wave gives up after `budget` unsuccessful looks in total, takes NaN for what did not
-// come, hands NaN on and never waits again, so the launch ends and its output says so.
+// come, hands NaN on and never waits again, so the launch ends and its output says so.  What it left behind in the workspace
+// is not to be built on: it marks it, and later launches over it only write NaN, until it is zeroed.
 //
 // The order of sums is the launch list's, bit for bit: products by super-chunks of 512 k added up in order, norms and
 // attention as in stage_x_norm and rope_attn_decode_kernel.  A policy may take either form for the same step (partial
@@ -68,6 +69,7 @@ struct TrunkState {
     uint64_t team;       // number of a launch's first layer << 32 | workgroups that take part in it
     uint32_t number;     // of the last exchange; the last workgroup to arrive counts it up
     uint32_t arrived;    // tickets taken; the last workgroup to arrive puts it back
+    uint32_t gave_up;    // a wait over this workspace was given up
 };
 
 struct TrunkArgs {
@@ -766,16 +768,18 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
     };
 
     // ---- who takes part (wave TW - 1 sees to it): a ticket once this launch's number is known ...
-    struct Ticket { uint32_t first, rank; };
+    struct Ticket { uint32_t first, gave_up, rank; };
     auto arrive = [&](Ticket &mine) {
         TrunkState *const state = again()->state;
         if (lane == 0) {
             mine.first = __hip_atomic_load(&state->number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            mine.gave_up = __hip_atomic_load(&state->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("s_waitcnt vmcnt(0)" : "+v"(mine.first)::"memory");   // read before the ticket: the last one counts it up
             mine.rank = __hip_atomic_fetch_add(&state->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
-    // ... and the team: whoever offers first.  Afterwards all threads know the number; returns the team's size.
+    // ... and the team: whoever offers first.  Afterwards all threads know the number; returns the team's size, 0: the
+    // workspace is marked (by an earlier launch, so all workgroups find the same).
     auto settle = [&](const Ticket &mine) {
         if (wave == TW - 1 && lane == 0) {
             const arg_ptr t = again();
@@ -788,7 +792,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
             }
             uint32_t offer = mine.rank + 1 == most ? most : 0u;
             const uint64_t since = __builtin_readsteadycounter();
-            while ((uint32_t)(seen >> 32) != first + 8u) {
+            while (!mine.gave_up && (uint32_t)(seen >> 32) != first + 8u) {
                 if (offer) {
                     const uint64_t team = (uint64_t)(first + 8u) << 32 | offer;
                     if (__hip_atomic_compare_exchange_strong(&state->team, &seen, team, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -802,17 +806,28 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
                 if (waited >= TEAM_TICKS_LEAST && waited * here >= (uint64_t)t->n_layers * TEAM_TICKS) offer = here;
                 seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            joined[0] = first + 8u, joined[1] = mine.rank, joined[2] = (uint32_t)seen;
+            joined[0] = first + 8u, joined[1] = mine.rank, joined[2] = mine.gave_up ? 0u : (uint32_t)seen;
         }
         lds_barrier();
         number = __builtin_amdgcn_readfirstlane(joined[0]);
         return (int)__builtin_amdgcn_readfirstlane(joined[2]);
     };
 
+    auto mark = [&]() {
+        if (budget == 0 && lane == 0)
+            __hip_atomic_store(&again()->state->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+
     // ---- the team is not the whole grid: every product's parts are dealt out to its members, one after the other
     if constexpr (SHARED) {
         number = __builtin_amdgcn_readfirstlane(joined[0]);
         const int rank = __builtin_amdgcn_readfirstlane(joined[1]), team = __builtin_amdgcn_readfirstlane(joined[2]);
+        static_assert(TT == ROW_WORDS, "a word each");
+        if (team == 0 && rank < M) {
+            const arg_ptr t = again();
+            for (gptr_w out : {(gptr_w)(uintptr_t)t->normed, (gptr_w)(uintptr_t)t->h_out})
+                if (out) out[rank * ROW_WORDS + tid] = NOT_COME;
+        }
         if (rank >= team) return;   // left out
         auto deal = [&](int parts, auto work) __attribute__((always_inline)) {
             for (int part = rank; part < parts; part += team) {
@@ -906,6 +921,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         }
         number -= 8;
         if (again()->normed) deal(M, [&]() { last_norm(wg); });
+        mark();
         return;
     }
 
@@ -917,13 +933,14 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         forget();
         opaque(am), opaque(ah), opaque(akv);
         // -------------------------------------------------------------- norm, q|k|v
-        Ticket ticket{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u)};   // (the first layer's)
+        Ticket ticket{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u),
+                      __builtin_nondeterministic_value(0u)};   // (the first layer's)
         {
             Rows<MW, C::P1> x;
             Built built;
             undefined(x);
             build_ahead(P_QKV, built);
-            if (l == 0 && wave == TW - 1) arrive(ticket);
+            if (__builtin_expect(l == 0 && wave == TW - 1, 0)) arrive(ticket);
             number += 8;
             if (slots_qkv) take_rows(P1, x, L->norm1, a.e_out, number - 2, l == 0 ? again()->cur : nullptr);   // the sixth exchange of the layer before
             load(P_O, l);
@@ -932,7 +949,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
                 multiply_staged(P_QKV, built);
             }
         }
-        if (l == 0) {
+        if (__builtin_expect(l == 0, 0)) {
             const int team = settle(ticket);
             if (__builtin_expect(team != G, 0)) return share_out<C>(args, (lds_ptr)smem);
         }
@@ -985,6 +1002,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         }
     }
     if (again()->normed && wg < M) last_norm(wg);
+    mark();
 }
 
 template <class C>
