@@ -33,7 +33,7 @@ class Step:
     """A trunk of random int4 layers over a random cache, its step as one launch and as the list."""
 
     def __init__(self, rows, layers=2, heads=16, kv_heads=16, inter=5632, length=1024, slot=(330,), padded=True,
-                 final_norm=True, seed=1):
+                 final_norm=True, seed=1, edit=None):
         gen = torch.Generator(device=DEV).manual_seed(seed)
         norm = lambda: types.SimpleNamespace(weight=normal(gen, HIDDEN, scale=0.1).add_(1.0), variance_epsilon=1e-6)
 
@@ -67,6 +67,8 @@ class Step:
                 self.mask[m, :min(7 + 40 * m, min(slot) // 2)] = 0
         self.x = normal(gen, rows, 1, HIDDEN)
         self.slot = torch.tensor(slot, dtype=torch.int64, device=DEV)
+        if edit is not None:
+            edit(trunk)
         self.native = NativeDecodeTrunk(trunk, held, self.x, self.mask, self.slot, final_norm=final_norm)
         self.one = self.native._trunk
 
@@ -310,6 +312,43 @@ def test_a_workspace_that_was_given_up_on_says_so(final_norm):
     workspace.zero_()
     got, cache = step.run(True)
     assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(cache, want_cache))
+
+
+def shifted(t):
+    """The same values two bytes further on."""
+    out = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("which", ["input_layernorm", "post_attention_layernorm", "norm"])
+@pytest.mark.parametrize("what", ["address", "eps"])
+def test_norms_that_the_list_refuses_stay_refused(which, what):
+    print("decode trunk: norms", which, what, flush=True)
+
+    def edit(trunk):
+        norm = trunk.norm if which == "norm" else getattr(trunk.layers[1], which)
+        if what == "address":
+            norm.weight = shifted(norm.weight)
+        else:
+            norm.variance_epsilon = -1.0
+
+    step = Step(2, edit=edit)
+    assert step.one is None
+    with pytest.raises(ValueError):
+        step.native.run()
+
+
+def test_rotary_tables_at_any_address():
+    print("decode trunk: rotary tables", flush=True)
+    want, _ = Step(2).run(False)
+
+    def edit(trunk):
+        tables = trunk.rotary_emb
+        trunk.rotary_emb = lambda *args, **kwargs: tuple(shifted(t) for t in tables(*args, **kwargs))
+
+    step = Step(2, edit=edit)
+    assert step.native.cos.data_ptr() % 4 == 2 and step.one is None
+    assert torch.equal(step.native.run(), want)
 
 
 def test_refusals():

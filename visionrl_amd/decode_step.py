@@ -424,7 +424,8 @@ class NativeDecodeTrunk:
         """The step as one launch: arguments of ``vrl_decode_trunk_bf16`` for its default and its short form, or
         ``None`` where the list is what runs (adapters, more rows or other shapes than the launch takes)."""
         records = (_lib.TrunkLayer * len(trunk.layers))()
-        inter = None
+        norm = trunk.norm.weight.data
+        inter, checked, caches = None, [(float(trunk.norm.variance_epsilon), norm)], []
         for i, (record, layer) in enumerate(zip(records, trunk.layers)):
             attn, mlp = layer.self_attn, layer.mlp
             proj = [_projection(getattr(attn, n), n) for n in ("q_proj", "k_proj", "v_proj", "o_proj")]
@@ -436,6 +437,8 @@ class NativeDecodeTrunk:
                     any(w.group_size != 128 for w in weights):
                 return None
             norms = layer.input_layernorm, layer.post_attention_layernorm
+            checked += [(float(n.variance_epsilon), n.weight.data) for n in norms]
+            caches += [cache.layers[i].keys, cache.layers[i].values]
             for name, t in zip(("q", "k", "v", "o", "gate_up", "down", "norm1", "norm2", "k_cache", "v_cache"),
                                (*(w.blob for w in weights), *(n.weight.data for n in norms), cache.layers[i].keys,
                                 cache.layers[i].values)):
@@ -443,6 +446,11 @@ class NativeDecodeTrunk:
                 setattr(record, name, t.data_ptr())
             record.eps1, record.eps2 = (float(n.variance_epsilon) for n in norms)
             record.scaling = float(attn.scaling)
+        # Its records are read on the device, where nothing can be refused: what the list's entry points refuse stays
+        # with the list, and so do rotary tables where only they can read them.
+        if not all(eps >= 0.0 and w.data_ptr() % 16 == 0 for eps, w in checked) or \
+                any(t.data_ptr() % 16 for t in caches) or any(t.data_ptr() % 4 for t in (self.cos, self.sin)):
+            return None
         desc = _lib.Trunk(n_layers=len(records), M=self.rows, hidden=self.hidden, inter=inter, n_heads=H,
                           n_kv_heads=Hkv, head_dim=D, group_size=128, L_max=self.max_len,
                           position_per_row=int(slot.numel() != 1),
@@ -454,8 +462,7 @@ class NativeDecodeTrunk:
             return None
         table = torch.frombuffer(bytearray(records), dtype=torch.uint8).to(self.device)
         workspace = torch.zeros(nbytes, dtype=torch.uint8, device=self.device)
-        norm = trunk.norm.weight.data
-        self._keep += [table, workspace, norm]
+        self._keep += [table, workspace]
         for name, t in zip(("layers", "x", "mask", "cos", "sin", "norm", "position", "workspace"),
                            (table, cur, mask, self.cos, self.sin, norm, slot, workspace)):
             setattr(desc, name, t.data_ptr())
