@@ -338,6 +338,16 @@ def test_norms_that_the_list_refuses_stay_refused(which, what):
         step.native.run()
 
 
+def test_no_layers():
+    print("decode trunk: no layers", flush=True)
+    step = Step(2, layers=0)
+    assert step.one is None
+    got = step.native.run().float()
+    x = step.x[:, 0].float()
+    want = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * step.native._keep[-1].float()
+    assert torch.allclose(got, want, rtol=2 ** -7, atol=1e-6)   # two roundings to bf16
+
+
 def test_rotary_tables_at_any_address():
     print("decode trunk: rotary tables", flush=True)
     want, _ = Step(2).run(False)

@@ -446,6 +446,8 @@ class NativeDecodeTrunk:
                 setattr(record, name, t.data_ptr())
             record.eps1, record.eps2 = (float(n.variance_epsilon) for n in norms)
             record.scaling = float(attn.scaling)
+        if inter is None:   # no layers
+            return None
         # Its records are read on the device, where nothing can be refused: what the list's entry points refuse stays
         # with the list, and so do rotary tables where only they can read them.
         if not all(eps >= 0.0 and w.data_ptr() % 16 == 0 for eps, w in checked) or \
