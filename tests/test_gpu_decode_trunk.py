@@ -338,6 +338,19 @@ def test_norms_that_the_list_refuses_stay_refused(which, what):
         step.native.run()
 
 
+@pytest.mark.parametrize("code", _lib.NOT_COOPERATIVE)
+def test_a_refused_cooperative_launch_leaves_the_step_to_the_list(monkeypatch, code):
+    print("decode trunk: not cooperative", code, flush=True)
+    step = Step(2)
+    want, want_cache = step.run(False)
+    monkeypatch.setattr(_lib.load(), "vrl_decode_trunk_bf16", lambda *args: code)
+    got, cache = step.run(True)
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(cache, want_cache))
+    monkeypatch.setattr(_lib.load(), "vrl_decode_trunk_bf16", lambda *args: 1002)   # a mistake is still one
+    with pytest.raises(ValueError):
+        step.run(True)
+
+
 def test_no_layers():
     print("decode trunk: no layers", flush=True)
     step = Step(2, layers=0)

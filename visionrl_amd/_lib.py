@@ -14,6 +14,9 @@ import threading
 from .build import LIB_PATH
 
 ABI_VERSION = 1
+# What a cooperative launch returns, and enqueues nothing, where the device or the runtime does not take it:
+# VRL_INT4_ELIMIT (checked beforehand), hipErrorCooperativeLaunchTooLarge, hipErrorNotSupported.
+NOT_COOPERATIVE = (1005, 720, 801)
 
 SYMBOLS = (
     "vrl_int4_abi_version",

@@ -1165,6 +1165,8 @@ extern "C" int vrl_decode_trunk_bf16(const vrl_trunk *trunk, void *hip_stream) {
         offset += (plan.words[i] * 8 + 255) / 256 * 256;
     }
     void *args[] = {&a};
-    return (int)hipLaunchCooperativeKernel(TRUNK_BUILDS[plan.build].kernel, dim3(plan.grid), dim3(TT), args,
-                                           (unsigned)plan.lds, reinterpret_cast<hipStream_t>(hip_stream));
+    const hipError_t e = hipLaunchCooperativeKernel(TRUNK_BUILDS[plan.build].kernel, dim3(plan.grid), dim3(TT), args,
+                                                    (unsigned)plan.lds, reinterpret_cast<hipStream_t>(hip_stream));
+    if (e != hipSuccess) (void)hipGetLastError();   // a caller may go on with the list: not left for the next check to find
+    return (int)e;
 }

@@ -492,8 +492,10 @@ class NativeDecodeTrunk:
         if self._trunk is not None:
             with ops._on(self.device):
                 rc = _lib.load().vrl_decode_trunk_bf16(ctypes.byref(self._trunk[short]), stream)
-            _lib.check(rc, "vrl_decode_trunk_bf16")
-            return self.normed
+            if rc not in _lib.NOT_COOPERATIVE:
+                _lib.check(rc, "vrl_decode_trunk_bf16")
+                return self.normed
+            self._trunk = None   # nothing was enqueued: from here on the list
         table, calls = (self._table_short, self._calls_short) if short else (self._table, self._calls)
         with ops._on(self.device):
             rc = _lib.load().vrl_decode_run_calls(table, len(table), ctypes.byref(self._failed_at), stream)
