@@ -338,6 +338,13 @@ def test_norms_that_the_list_refuses_stay_refused(which, what):
         step.native.run()
 
 
+def test_launches_says_what_run_enqueues():
+    step = Step(2, layers=3)
+    assert step.native.launches == 1
+    step.native._trunk = None
+    assert step.native.launches == 5 * 3 + 1
+
+
 @pytest.mark.parametrize("code", _lib.NOT_COOPERATIVE)
 def test_a_refused_cooperative_launch_leaves_the_step_to_the_list(monkeypatch, code):
     print("decode trunk: not cooperative", code, flush=True)

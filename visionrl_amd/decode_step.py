@@ -404,7 +404,6 @@ class NativeDecodeTrunk:
             self.final = (state["x"], state["res"], w, eps)
             self.normed = None
         self._calls = calls
-        self.launches = len(calls)
         # the same list as records of the library's own walk over it: one host call per step
         self._table = _lib.step_calls(calls)
         # The split launches leave a row with fewer than SPLIT_ATTENTION_FROM cached slots to one workgroup per
@@ -476,6 +475,11 @@ class NativeDecodeTrunk:
         short = _lib.Trunk.from_buffer_copy(desc)
         short.split_from = 0
         return desc, short
+
+    @property
+    def launches(self) -> int:
+        """Launches that :meth:`run` enqueues."""
+        return len(self._calls) if self._trunk is None else 1
 
     def short_form(self, cached_slots: int) -> bool:
         """Whether :meth:`run` has a launch list of its own for a step that finds ``cached_slots`` filled slots
