@@ -7,6 +7,7 @@ compared bit for bit: both entry points run the same kernel, only the scratch me
 """
 
 import ctypes
+import gc
 
 import numpy as np
 import pytest
@@ -19,6 +20,12 @@ from tests.test_head_sample import make_head
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+
+
+@pytest.fixture(autouse=True, scope="module")
+def cycles_of_earlier_modules():
+    """Tensors that other modules left in reference cycles are not let go between two readings of what is allocated."""
+    gc.collect()
 
 
 def call_both(lib, _lib, ops, B, K, V, G, seed, w=5.0, T=1.0):
