@@ -1,7 +1,7 @@
-"""Staging of the activations in the launches over prepacked weights: up to 16 rows go straight to LDS in pieces of 512 k.
+"""Staging of the activations in the launches over prepacked weights: few rows go straight to LDS in pieces of 512 k.
 
-Sizes at the edges of that: rows on both sides of 16, k that ends inside a piece or in the first one, more pieces than
-waves.  Reference and tolerance: a float64 product over the bit-exact dequantised weight; one bf16 rounding (2^-8 relative
+Sizes at the edges of that: rows on both sides of the lines (2, 4) and of 16, k that ends inside a piece or in the first
+one, more pieces than waves.  Reference and tolerance: a float64 product over the bit-exact dequantised weight; one bf16 rounding (2^-8 relative
 covers it) and the worst case of K fp32 additions, K 2^-24 sum |x w|.
 """
 
@@ -19,8 +19,8 @@ def _triple(gen, K, N, G, dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M", [1, 2, 7, 15, 16, 17, 32])
-@pytest.mark.parametrize("K", [128, 384, 512, 2048, 2176, 5632, 11008])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 7, 15, 16, 17, 32])
+@pytest.mark.parametrize("K", [128, 384, 512, 2048, 2176, 4096, 5632, 11008])
 @pytest.mark.parametrize("form", ["direct", "grouped"])
 def test_staged_rows(M, K, form):
     gen = torch.Generator().manual_seed(100 * M + K)

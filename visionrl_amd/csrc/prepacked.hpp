@@ -105,34 +105,8 @@ constexpr int PP_ZERO_ROW = 2;  // DevProblem::prepacked bit
 
 // natural-order staging of x[:, k0:k1) (k beyond K reads as zero), plus a row of zeros at
 // row M if the record asks for one
-// Up to 16 rows a wave takes 512 k of a row at a time, straight into LDS: all of a workgroup's requests are on their way at
-// once and no instruction divides by the row length (a step of 24 layers of 2048 with adapters at 16 rows 1345 -> 1318 us, 30
-// layers of 4096 at 8 rows 1875 -> 1860).  With more rows a workgroup's loads are bound by their rate, and the direct ones
-// are the slower (the head's call at 32 rows 17.1 against 18.1 us; a step at 32 rows 1639 against 1645).
-constexpr int STAGE_DIRECT_ROWS = 16;
 __device__ __forceinline__ void stage_x_natural(const DevProblem &p, int k0, int k1, uint16_t *xs,
                                                 int xstride, int nthreads) {
-    if (p.M <= STAGE_DIRECT_ROWS) {
-        const int pieces = (k1 - k0) / PP_SC, nwaves = nthreads / WAVE;
-        const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const int rows = p.M + ((p.prepacked & PP_ZERO_ROW) ? 1 : 0);
-        for (int m = 0, j = wave;; j += nwaves) {
-            for (; j >= pieces && m < rows; j -= pieces) ++m;
-            if (m >= rows) break;
-            const int k = k0 + j * PP_SC;
-            uint16_t *const at = xs + m * xstride + j * PP_SC;
-            const uint16_t *const from = p.x + (long)m * p.K + k;
-            if (m < p.M && k + PP_SC <= p.K) {   // wave-uniform
-                dma16(reinterpret_cast<uint8_t *>(at), reinterpret_cast<const uint8_t *>(from), lane * 16);
-            } else {
-                u32x4_t d = {0u, 0u, 0u, 0u};
-                if (m < p.M && k + lane * 8 < p.K) d = *as_global(reinterpret_cast<const u32x4_t *>(from + lane * 8));
-                *reinterpret_cast<u32x4_t *>(at + lane * 8) = d;
-            }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the compiler does not see the direct loads
-        return;
-    }
     const int words_per_row = (k1 - k0) >> 3;
     const int total = (p.M + ((p.prepacked & PP_ZERO_ROW) ? 1 : 0)) * words_per_row;
     for (int idx = threadIdx.x; idx < total; idx += nthreads) {
@@ -143,6 +117,32 @@ __device__ __forceinline__ void stage_x_natural(const DevProblem &p, int k0, int
         if (k < p.K && m < p.M) d = *as_global(reinterpret_cast<const u32x4_t *>(p.x + (long)m * p.K + k));
         *reinterpret_cast<u32x4_t *>(xs + m * xstride + (j << 3)) = d;
     }
+}
+
+// The same over all of K with loads straight to LDS: a wave takes 512 k of a row at a time, and all of a workgroup's
+// requests are on their way at once.  That is worth it while they are few: beyond, the rate of these loads is the limit
+// (one launch, x in the caches, other form against this: K = N = 2048 4.2 / 3.9 us at 2 rows, 4.2 / 4.4 at 4, 4.9 / 6.1
+// at 16; K = N = 4096 5.7 / 5.6 at 4 rows, 6.3 / 6.5 at 10, in passes of rows32_segment at 20 rows 8.2 / 9.3).
+__device__ __forceinline__ bool few_rows(const DevProblem &p) { return p.M <= (p.K >= 4096 ? 4 : 2); }
+__device__ __forceinline__ void stage_x_direct(const DevProblem &p, uint16_t *xs, int xstride, int nthreads) {
+    const int pieces = pp_nsc(p.K), nwaves = nthreads / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rows = p.M + ((p.prepacked & PP_ZERO_ROW) ? 1 : 0);
+    for (int m = 0, j = wave;; j += nwaves) {
+        for (; j >= pieces && m < rows; j -= pieces) ++m;
+        if (m >= rows) break;
+        const int k = j * PP_SC;
+        uint16_t *const at = xs + m * xstride + k;
+        const uint16_t *const from = p.x + (long)m * p.K + k;
+        if (m < p.M && k + PP_SC <= p.K) {   // wave-uniform
+            dma16(reinterpret_cast<uint8_t *>(at), reinterpret_cast<const uint8_t *>(from), lane * 16);
+        } else {
+            u32x4_t d = {0u, 0u, 0u, 0u};
+            if (m < p.M && k + lane * 8 < p.K) d = *as_global(reinterpret_cast<const u32x4_t *>(from + lane * 8));
+            *reinterpret_cast<u32x4_t *>(at + lane * 8) = d;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the compiler does not see the direct loads
 }
 
 // Residual add and RMSNorm applied while the activations are staged (plan-free launches only):
@@ -661,7 +661,11 @@ __device__ __forceinline__ void stream_segment_pp(const DevProblem &p, int t0, i
                               staged.zero_row == zero_row;  // block-uniform
         __syncthreads();
         if (threadIdx.x == 0) next_tile = t0 + WPB;
-        if (!resident) stage_x_natural(p, 0, nsc * PP_SC, xs, xstride, WPB * WAVE);
+        if (!resident) {
+            // (three layers as a grouped plan: 23.0 -> 22.3 us at 2 rows, 23.1 -> 22.4 at 4, 22.0 against 24.5 at 16)
+            if (MB == 1 && p.M <= 4) stage_x_direct(p, xs, xstride, WPB * WAVE);
+            else stage_x_natural(p, 0, nsc * PP_SC, xs, xstride, WPB * WAVE);
+        }
         __syncthreads();
         staged.x = p.x;
         staged.M = p.M;
@@ -894,7 +898,7 @@ __device__ __forceinline__ void store_tile_epi(const DevProblem &p, int tile_loc
 template <bool FUSED, int KS, int TW, int GQ, bool NORM, bool XG, bool UP = false, bool EPI = false>
 __device__ __forceinline__ void split_segment_pp(const DevProblem &p, int t0, int t1, uint8_t *smem,
                                                  const NormArgs &norm, const LoraUpArgs &up = LoraUpArgs{},
-                                                 const EpiArgs &epi = EpiArgs{}) {
+                                                 const EpiArgs &epi = EpiArgs{}, bool lora_input = false) {
     constexpr int RS = FUSED ? 2 : 1;
     static_assert(!EPI || (!FUSED && !UP), "bias, activation and residual join a plain problem");
     static_assert(!XG || (TW == 1 && !NORM), "register-fed activations: one tile per workgroup, no norm");
@@ -940,7 +944,11 @@ __device__ __forceinline__ void split_segment_pp(const DevProblem &p, int t0, in
                          t0 == 0 && (p.prepacked & PP_WRITE_H) && norm.h_out != nullptr,
                          reinterpret_cast<float *>(smem + (size_t)xrows * xstride * 2));  // the partial tiles' space, still free
         else
-            stage_x_natural(p, 0, nsc * PP_SC, xs, xstride, KS * TW * WAVE);
+            // Beside few_rows, in a decode step, where another launch has just written x (six layers of 2048, us per
+            // step): o_proj with its adapter up to 6 rows (264.5 -> 258 at 6; 263.7 against 264.6 at 8), q|k|v with
+            // adapters up to 16 (304.5 -> 301 at 16; cut into records of 16 rows and fewer: 387 against 392 at 18).
+            if (few_rows(p) || (UP && p.M <= 6) || lora_input) stage_x_direct(p, xs, xstride, KS * TW * WAVE);
+            else stage_x_natural(p, 0, nsc * PP_SC, xs, xstride, KS * TW * WAVE);
         __syncthreads();
     }
     for (int base = t0; base < t1; base += TW) {
@@ -993,7 +1001,7 @@ __device__ __forceinline__ void split_segment_pp(const DevProblem &p, int t0, in
 template <bool FUSED, int KS, int TW, bool NORM, bool XG, bool UP = false, bool EPI = false>
 __device__ __forceinline__ void split_by_group(const DevProblem &p, int t0, int t1, uint8_t *smem,
                                                const NormArgs &norm, const LoraUpArgs &up = LoraUpArgs{},
-                                               const EpiArgs &epi = EpiArgs{}) {
+                                               const EpiArgs &epi = EpiArgs{}, bool lora_input = false) {
     if constexpr (EPI) {
         if (p.G == 128) split_segment_pp<false, KS, TW, 1, NORM, XG, false, true>(p, t0, t1, smem, norm, up, epi);
         else if (p.G == 64) split_segment_pp<false, KS, TW, 2, NORM, XG, false, true>(p, t0, t1, smem, norm, up, epi);
@@ -1007,9 +1015,9 @@ __device__ __forceinline__ void split_by_group(const DevProblem &p, int t0, int 
         else if (p.G == 64) split_segment_pp<FUSED, KS, TW, 2, NORM, XG>(p, t0, t1, smem, norm);
         else split_segment_pp<FUSED, KS, TW, 4, NORM, XG>(p, t0, t1, smem, norm);
     } else {
-        if (p.G == 128) split_segment_pp<false, KS, TW, 1, NORM, XG>(p, t0, t1, smem, norm);
-        else if (p.G == 64) split_segment_pp<false, KS, TW, 2, NORM, XG>(p, t0, t1, smem, norm);
-        else split_segment_pp<false, KS, TW, 4, NORM, XG>(p, t0, t1, smem, norm);
+        if (p.G == 128) split_segment_pp<false, KS, TW, 1, NORM, XG>(p, t0, t1, smem, norm, up, epi, lora_input);
+        else if (p.G == 64) split_segment_pp<false, KS, TW, 2, NORM, XG>(p, t0, t1, smem, norm, up, epi, lora_input);
+        else split_segment_pp<false, KS, TW, 4, NORM, XG>(p, t0, t1, smem, norm, up, epi, lora_input);
     }
 }
 
@@ -1081,7 +1089,8 @@ __global__ __launch_bounds__(KS *TW *WAVE) void gemv_split_direct_kernel(DirectA
         if (k < a.n && a.recs[k].tile_begin <= g) p = a.recs[k];  // scalar selects, no indexing
     const int tiles = ((p.fused ? p.N / 2 : p.N) + 15) / 16;
     const int t0 = (g - p.tile_begin) * TW * a.rounds;
-    split_by_group<FUSED, KS, TW, NORM, XG, UP, EPI>(p, t0, min(tiles, t0 + TW * a.rounds), smem, a.norm, a.up, a.epi);
+    split_by_group<FUSED, KS, TW, NORM, XG, UP, EPI>(p, t0, min(tiles, t0 + TW * a.rounds), smem, a.norm, a.up, a.epi,
+                                                     LD && a.ld.a.M <= 16);
 }
 
 }  // namespace
