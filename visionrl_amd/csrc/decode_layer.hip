@@ -188,9 +188,9 @@ __device__ __forceinline__ void merge(Partial<VEC> &a, float m2, float l2, const
     const float ref = m == -INFINITY ? 0.0f : m;  // both empty: keep zeros, avoid inf - inf
     const float c1 = __expf(a.m - ref), c2 = __expf(m2 - ref);
     a.m = m;
-    a.l = a.l * c1 + l2 * c2;
+    a.l = two_products(a.l, c1, l2, c2);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) a.acc[i] = a.acc[i] * c1 + acc2[i] * c2;
+    for (int i = 0; i < VEC; ++i) a.acc[i] = two_products(acc2[i], c2, a.acc[i], c1);
 }
 
 
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(ATT_WAVES *WAVE) void rope_attn_decode_kernel(AttnA
     }
     if (wave == 0) {  // the new token's own slot
         float dot = 0.0f;
-        for (int d = lane; d < D; d += WAVE) dot += qs[d] * ks[d];
+        for (int d = lane; d < D; d += WAVE) dot = __builtin_fmaf(qs[d], ks[d], dot);
         dot = wave_sum(dot);
         if (lane == 0) s_new = (mask[p] && split == 0) ? dot * a.scaling : -INFINITY;  // one workgroup of a pair counts it
     }
@@ -491,17 +491,14 @@ __global__ __launch_bounds__(ATT_WAVES *WAVE) void rope_attn_decode_kernel(AttnA
         const float ref = mx == -INFINITY ? 0.0f : mx;  // nothing attendable yet: keep zeros, avoid inf - inf
         const float c0 = __expf(st.m - ref);
         st.m = mx;
-        st.l *= c0;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) st.acc[i] *= c0;
 #pragma unroll
         for (int u = 0; u < ATT_UNROLL; ++u) {
             const float w = __expf(sc[u] - ref);
-            st.l += w;
+            st.l = u ? st.l + w : __builtin_fmaf(st.l, c0, w);
 #pragma unroll
-            for (int i = 0; i < VEC / 2; ++i) {
-                st.acc[2 * i] += w * bf16_to_f32(vraw[u].w[i] & 0xFFFFu);
-                st.acc[2 * i + 1] += w * bf16_to_f32(vraw[u].w[i] >> 16);
+            for (int i = 0; i < VEC; ++i) {
+                const float v = bf16_to_f32(i & 1 ? vraw[u].w[i / 2] >> 16 : vraw[u].w[i / 2] & 0xFFFFu);
+                st.acc[i] = u ? __builtin_fmaf(w, v, st.acc[i]) : two_products(st.acc[i], c0, w, v);
             }
         }
     }
@@ -530,13 +527,12 @@ __global__ __launch_bounds__(ATT_WAVES *WAVE) void rope_attn_decode_kernel(AttnA
         float o = 0.0f, sum = 0.0f;
         if (mx != -INFINITY) {  // else every slot is masked: the output is zero
             const float cn = __expf(s_new - mx);
-            o = cn * vs[tid];
             sum = cn;
 #pragma unroll
             for (int w = 0; w < ATT_WAVES; ++w) {
                 const float c = __expf(pm[w] - mx);
-                o += c * pacc[w][tid];
-                sum += c * pl[w];
+                o = w ? __builtin_fmaf(c, pacc[w][tid], o) : two_products(cn, vs[tid], c, pacc[0][tid]);
+                sum = __builtin_fmaf(c, pl[w], sum);
             }
             if (whole) o /= sum;
         }
@@ -593,8 +589,8 @@ __global__ __launch_bounds__(ATT_WAVES *WAVE) void rope_attn_decode_kernel(AttnA
 #pragma unroll
                 for (int z = 0; z < ATTN_MAX_SPLITS; ++z) {   // index order: the same sums whoever merges
                     const float c = __expf(pm_[z] - mx);
-                    o += c * po_[z];
-                    sum += c * ps_[z];
+                    o = __builtin_fmaf(c, po_[z], o);
+                    sum = __builtin_fmaf(c, ps_[z], sum);
                 }
                 o /= sum;
             }

@@ -85,7 +85,7 @@ struct TrunkArgs {
     int32_t grid, most;                   // workgroups, and how many of them may take part
     int32_t n_layers, position_stride, M, A, KV, I, heads, kv_heads, L_max;
     int32_t nsc_a, nsc_i;                 // super-chunks of A and I
-    int32_t split_from, split_build;      // filled slots from which a pair's slots are divided in ranges; whether they ever are
+    int32_t split_from;                   // filled slots from which a pair's slots are divided in ranges
 };
 
 constexpr int SC1 = 16;   // cache-policy bit: device scope, past the die's own L2
@@ -615,7 +615,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const float v = e & 1 ? high_bf16(kv.v[b + u][e >> 1]) : low_bf16(kv.v[b + u][e >> 1]);
-                        acc[e] = u ? __builtin_fmaf(w, v, acc[e]) : __builtin_fmaf(acc[e], c0, w * v);
+                        acc[e] = u ? __builtin_fmaf(w, v, acc[e]) : two_products(acc[e], c0, w, v);
                     }
                 }
             }
@@ -628,13 +628,12 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
             step ? swap_32(l1, l2) : swap_16(l1, l2);
             mx = fmaxf(m1, m2);
             const float ref = mx == -INFINITY ? 0.0f : mx, c1 = __expf(m1 - ref), c2 = __expf(m2 - ref);
-            sum = __builtin_fmaf(l1, c1, l2 * c2);
+            sum = two_products(l1, c1, l2, c2);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float a1 = acc[e], a2 = acc[e];
                 step ? swap_32(a1, a2) : swap_16(a1, a2);
-                // (which product is rounded: as each build of rope_attn_decode_kernel came out of the compiler)
-                acc[e] = e < 5 || a.split_build ? __builtin_fmaf(a2, c2, a1 * c1) : __builtin_fmaf(a1, c1, a2 * c2);
+                acc[e] = two_products(a2, c2, a1, c1);
             }
         }
         if (ranges) {
@@ -677,8 +676,8 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
                 if (w < n) {   // uniform
                     const float2 v = *reinterpret_cast<const float2 *>(pacc + w * HEAD_DIM + col);
                     const float c = lane_of(c_w, w);
-                    o0 = w ? __builtin_fmaf(c, v.x, o0) : __builtin_fmaf(c_own, v0, c * v.x);
-                    o1 = w ? __builtin_fmaf(c, v.y, o1) : __builtin_fmaf(c_own, v1, c * v.y);
+                    o0 = w ? __builtin_fmaf(c, v.x, o0) : two_products(c_own, v0, c, v.x);
+                    o1 = w ? __builtin_fmaf(c, v.y, o1) : two_products(c_own, v1, c, v.y);
                     total = __builtin_fmaf(c, lane_of(l_w, w), total);
                 }
         return Joined{o0, o1, total, top};
@@ -1154,8 +1153,7 @@ extern "C" int vrl_decode_trunk_bf16(const vrl_trunk *trunk, void *hip_stream) {
     a.most = t.max_workgroups ? (int)std::min(t.max_workgroups, (uint32_t)plan.grid) : plan.grid;
     a.nsc_a = pp_nsc(a.A);
     a.nsc_i = pp_nsc(a.I);
-    a.split_build = t.split_from > 0;
-    a.split_from = a.split_build ? t.split_from : INT32_MAX;
+    a.split_from = t.split_from > 0 ? t.split_from : INT32_MAX;
     uint8_t *ws = static_cast<uint8_t *>(t.workspace);
     a.state = reinterpret_cast<TrunkState *>(ws);
     uint64_t **const at[6] = {&a.e_qkv, &a.e_part, &a.e_attn, &a.e_mid, &a.e_act, &a.e_out};

@@ -6,6 +6,10 @@
 
 namespace {
 
+// a b + c d with the second product rounded.  Left to the compiler either may be the fused one, build by build; the
+// attention of the launch list and that of the step as one launch have to round alike.
+__device__ __forceinline__ float two_products(float a, float b, float c, float d) { return __builtin_fmaf(a, b, c * d); }
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
