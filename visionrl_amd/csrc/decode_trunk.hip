@@ -767,12 +767,11 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
     };
 
     // ---- who takes part (wave TW - 1 sees to it): a ticket once this launch's number is known ...
-    struct Ticket { uint32_t first, gave_up, rank; };
+    struct Ticket { uint32_t first, rank; };
     auto arrive = [&](Ticket &mine) {
         TrunkState *const state = again()->state;
         if (lane == 0) {
             mine.first = __hip_atomic_load(&state->number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            mine.gave_up = __hip_atomic_load(&state->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("s_waitcnt vmcnt(0)" : "+v"(mine.first)::"memory");   // read before the ticket: the last one counts it up
             mine.rank = __hip_atomic_fetch_add(&state->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -784,6 +783,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
             const arg_ptr t = again();
             TrunkState *const state = t->state;
             const uint32_t first = mine.first, all = G, most = t->most;
+            const uint32_t gave_up = __hip_atomic_load(&state->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             uint64_t seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (mine.rank + 1 == all) {   // every workgroup has read the number: the next launch's, and a new count
                 __hip_atomic_store(&state->number, first + 8u + 8u * t->n_layers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -791,7 +791,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
             }
             uint32_t offer = mine.rank + 1 == most ? most : 0u;
             const uint64_t since = __builtin_readsteadycounter();
-            while (!mine.gave_up && (uint32_t)(seen >> 32) != first + 8u) {
+            while (!gave_up && (uint32_t)(seen >> 32) != first + 8u) {
                 if (offer) {
                     const uint64_t team = (uint64_t)(first + 8u) << 32 | offer;
                     if (__hip_atomic_compare_exchange_strong(&state->team, &seen, team, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -805,7 +805,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
                 if (waited >= TEAM_TICKS_LEAST && waited * here >= (uint64_t)t->n_layers * TEAM_TICKS) offer = here;
                 seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            joined[0] = first + 8u, joined[1] = mine.rank, joined[2] = mine.gave_up ? 0u : (uint32_t)seen;
+            joined[0] = first + 8u, joined[1] = mine.rank, joined[2] = gave_up ? 0u : (uint32_t)seen;
         }
         lds_barrier();
         number = __builtin_amdgcn_readfirstlane(joined[0]);
@@ -932,14 +932,13 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         forget();
         opaque(am), opaque(ah), opaque(akv);
         // -------------------------------------------------------------- norm, q|k|v
-        Ticket ticket{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u),
-                      __builtin_nondeterministic_value(0u)};   // (the first layer's)
+        Ticket ticket{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u)};   // (the first layer's)
         {
             Rows<MW, C::P1> x;
             Built built;
             undefined(x);
             build_ahead(P_QKV, built);
-            if (__builtin_expect(l == 0 && wave == TW - 1, 0)) arrive(ticket);
+            if (l == 0 && wave == TW - 1) arrive(ticket);
             number += 8;
             if (slots_qkv) take_rows(P1, x, L->norm1, a.e_out, number - 2, l == 0 ? again()->cur : nullptr);   // the sixth exchange of the layer before
             load(P_O, l);
@@ -948,7 +947,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
                 multiply_staged(P_QKV, built);
             }
         }
-        if (__builtin_expect(l == 0, 0)) {
+        if (l == 0) {
             const int team = settle(ticket);
             if (__builtin_expect(team != G, 0)) return share_out<C>(args, (lds_ptr)smem);
         }
