@@ -71,9 +71,13 @@ __device__ __forceinline__ uint32_t pack_bf16_rne(float lo, float hi) {
 // register.  In assembly: the compiler takes the builtin for an access of both counters and from then on waits for every
 // outstanding LDS read where it needs the first (once per MFMA step in prompt_gemm.hip).  What orders these loads against
 // the LDS reads are the waits and barriers of the kernel, as with the builtin.
+// (clang notes that it never allocates m0 itself)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(uint8_t *lds, const uint8_t *base, uint32_t off) {
     const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 }  // namespace
