@@ -27,13 +27,14 @@
 // Who takes part.  The work is laid out for one workgroup per compute unit, all of them there at once, and a workgroup takes
 // every register of its compute unit: a single wave of anything else (a collective that waits for a late rank, another
 // process, a step from another graph) keeps one of them out, for as long as it likes.  So nothing waits for a workgroup that
-// has not started.  Each takes a ticket, and the team is fixed once, by one compare-and-swap: by the last to arrive, or by one
-// that has waited for the others as long as the step would take those that are there (TEAM_TICKS).  Members are running by
+// has not started.  The team is fixed once, by one compare-and-swap: by the last to arrive, with everyone, or by one that has
+// waited for the others as long as the step would take those that are there (TEAM_TICKS), with those that have taken a ticket
+// meanwhile, which is for whoever has waited TEAM_TICKS_LEAST.  Members are running by
 // then and stay, so what one waits for comes; a workgroup that starts later finds itself left out and ends.  With everyone
 // there each has its own part of every product.  Otherwise the parts are dealt out to the members, product by product:
 // the same sums and bits, without the work ahead of its input (24 layers at 2 rows: 515 us with all 256, 838 with 255 or 128
 // of them, 6.0 ms with 16; the launch list takes 766).  The team is looked up behind the first product, before anything is
-// handed out, so that the tickets cost next to nothing.
+// handed out, so that the arrivals cost next to nothing.
 //
 // Waits are bounded all the same: a wave gives up after `budget` unsuccessful looks in total, takes NaN for what did not
 // come, hands NaN on and never waits again, so the launch ends and its output says so.  What it left behind in the workspace
@@ -64,13 +65,21 @@ constexpr uint32_t TRUNK_BUDGET = 1u << 22; // looks of about a microsecond each
 // rows), divided by those that are there, and never less than the launch itself may need to bring all of them up.
 constexpr uint32_t TEAM_TICKS = 400000, TEAM_TICKS_LEAST = 10000;
 
-// The first 256 bytes of the workspace.
+// Arrivals are counted in two levels, since those at one address are served one after the other, 27 ns each (24 layers at 2
+// rows: a single counter for 256 workgroups 526 us, this way 518; at 4 rows 632 and 623).
+constexpr int ARRIVALS = 16;
+
+// The head of the workspace.
 struct TrunkState {
     uint64_t team;       // number of a launch's first layer << 32 | workgroups that take part in it
+    uint64_t tickets;    // the same number << 32 | workgroups that gave up waiting for everyone
     uint32_t number;     // of the last exchange; the last workgroup to arrive counts it up
-    uint32_t arrived;    // tickets taken; the last workgroup to arrive puts it back
+    uint32_t complete;   // groups that have arrived; the last workgroup to arrive puts it back
     uint32_t gave_up;    // a wait over this workspace was given up
+    uint32_t pad[57];
+    struct { uint32_t arrived, pad[63]; } groups[ARRIVALS];   // of workgroups wg % n_groups; the last of a group puts it back
 };
+static_assert(sizeof(TrunkState) == 256 * (1 + ARRIVALS), "a piece of 256 bytes each");
 
 struct TrunkArgs {
     const vrl_trunk_layer *layers;
@@ -82,7 +91,7 @@ struct TrunkArgs {
     uint64_t *e_qkv, *e_part, *e_attn, *e_mid, *e_act, *e_out;
     float eps;
     uint32_t budget;
-    int32_t grid, most;                   // workgroups, and how many of them may take part
+    int32_t grid, most, n_groups;         // workgroups, how many of them may take part, groups (a power of two) they are counted in
     int32_t n_layers, position_stride, M, A, KV, I, heads, kv_heads, L_max;
     int32_t nsc_a, nsc_i;                 // super-chunks of A and I
     int32_t split_from;                   // filled slots from which a pair's slots are divided in ranges
@@ -467,6 +476,19 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
     constexpr std::integral_constant<int, C::P1> P1{};
     constexpr std::integral_constant<int, C::P2> P2{};
 
+    // ---- who takes part (lane 0 of wave TW - 1 sees to it): a workgroup counts itself once it knows this launch's number ...
+    struct Arrival { uint32_t first, rank; };
+    auto arrive = [&](Arrival &mine) {
+        TrunkState *const state = again()->state;
+        if (lane == 0) {
+            mine.first = __hip_atomic_load(&state->number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(mine.first)::"memory");   // read before it counts: the last one counts it up
+            mine.rank = __hip_atomic_fetch_add(&state->groups[wg & (again()->n_groups - 1)].arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    };
+    Arrival arrival{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u)};
+    if (!SHARED && wave == TW - 1) arrive(arrival);
+
     // ---- this workgroup's share of the attention of one (row, head), the same in every layer; so are the position, the
     // rotation and which slots count.  The order of sums is that of rope_attn_decode_kernel with sixteen waves: groups of
     // sixteen lanes visit the slots of wave w, group g: 64 u + 4 w + g, four at a time; groups, then waves.  The
@@ -766,46 +788,63 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         }
     };
 
-    // ---- who takes part (wave TW - 1 sees to it): a ticket once this launch's number is known ...
-    struct Ticket { uint32_t first, rank; };
-    auto arrive = [&](Ticket &mine) {
-        TrunkState *const state = again()->state;
+    // ---- who takes part, continued: the last of a group counts the group, the last of all finds that every workgroup has read the number: the next
+    // launch's, and new counts.  Afterwards `rank` says whether this is the last of all.
+    auto count_group = [&](Arrival &mine) {
         if (lane == 0) {
-            mine.first = __hip_atomic_load(&state->number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("s_waitcnt vmcnt(0)" : "+v"(mine.first)::"memory");   // read before the ticket: the last one counts it up
-            mine.rank = __hip_atomic_fetch_add(&state->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const arg_ptr t = again();
+            TrunkState *const state = t->state;
+            const uint32_t n = t->n_groups;
+            bool last = (mine.rank + 1) * n == (uint32_t)G;
+            if (last) {
+                __hip_atomic_store(&state->groups[wg & (n - 1)].arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                last = __hip_atomic_fetch_add(&state->complete, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == n;
+            }
+            if (last) {
+                __hip_atomic_store(&state->number, mine.first + 8u + 8u * t->n_layers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&state->complete, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            mine.rank = last;
         }
     };
-    // ... and the team: whoever offers first.  Afterwards all threads know the number; returns the team's size, 0: the
+    // ... and the team: whoever offers first, the last of all with everyone, or one that has waited with those that have taken
+    // a ticket by then (nobody takes one at first).  Afterwards all threads know the number; returns the team's size, 0: the
     // workspace is marked (by an earlier launch, so all workgroups find the same).
-    auto settle = [&](const Ticket &mine) {
+    auto settle = [&](const Arrival &mine) {
         if (wave == TW - 1 && lane == 0) {
             const arg_ptr t = again();
             TrunkState *const state = t->state;
-            const uint32_t first = mine.first, all = G, most = t->most;
+            const uint32_t now = mine.first + 8u, most = t->most;
             const uint32_t gave_up = __hip_atomic_load(&state->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             uint64_t seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (mine.rank + 1 == all) {   // every workgroup has read the number: the next launch's, and a new count
-                __hip_atomic_store(&state->number, first + 8u + 8u * t->n_layers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&state->arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            uint32_t offer = mine.rank + 1 == most ? most : 0u;
+            uint32_t offer = mine.rank && most == (uint32_t)G ? most : 0u;
+            uint32_t rank = G;   // (of a workgroup without a ticket: left out, unless everyone is in)
             const uint64_t since = __builtin_readsteadycounter();
-            while (!gave_up && (uint32_t)(seen >> 32) != first + 8u) {
+            while (!gave_up && (uint32_t)(seen >> 32) != now) {
                 if (offer) {
-                    const uint64_t team = (uint64_t)(first + 8u) << 32 | offer;
+                    const uint64_t team = (uint64_t)now << 32 | offer;
                     if (__hip_atomic_compare_exchange_strong(&state->team, &seen, team, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                              __HIP_MEMORY_SCOPE_AGENT))
                         seen = team;
                     continue;
                 }
-                const uint32_t count = __hip_atomic_load(&state->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const uint32_t here = count == 0u ? most : min(count, most);   // (0: put back, all have arrived)
                 const uint64_t waited = __builtin_readsteadycounter() - since;
-                if (waited >= TEAM_TICKS_LEAST && waited * here >= (uint64_t)t->n_layers * TEAM_TICKS) offer = here;
+                if (waited >= TEAM_TICKS_LEAST || most != (uint32_t)G) {
+                    uint64_t tickets = __hip_atomic_load(&state->tickets, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    uint32_t count = (uint32_t)(tickets >> 32) == now ? (uint32_t)tickets : 0u;
+                    if (rank == (uint32_t)G) {
+                        if (!__hip_atomic_compare_exchange_strong(&state->tickets, &tickets, (uint64_t)now << 32 | (count + 1u),
+                                                                  __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                            continue;   // another one took it
+                        rank = count++;
+                    }
+                    const uint32_t here = min(count, most);
+                    if (rank + 1 == most || (waited >= TEAM_TICKS_LEAST && waited * here >= (uint64_t)t->n_layers * TEAM_TICKS))
+                        offer = here;
+                }
                 seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            joined[0] = first + 8u, joined[1] = mine.rank, joined[2] = gave_up ? 0u : (uint32_t)seen;
+            joined[0] = now, joined[1] = gave_up ? (uint32_t)wg : rank, joined[2] = gave_up ? 0u : (uint32_t)seen;
         }
         lds_barrier();
         number = __builtin_amdgcn_readfirstlane(joined[0]);
@@ -932,13 +971,12 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         forget();
         opaque(am), opaque(ah), opaque(akv);
         // -------------------------------------------------------------- norm, q|k|v
-        Ticket ticket{__builtin_nondeterministic_value(0u), __builtin_nondeterministic_value(0u)};   // (the first layer's)
         {
             Rows<MW, C::P1> x;
             Built built;
             undefined(x);
             build_ahead(P_QKV, built);
-            if (l == 0 && wave == TW - 1) arrive(ticket);
+            if (l == 0 && wave == TW - 1) count_group(arrival);
             number += 8;
             if (slots_qkv) take_rows(P1, x, L->norm1, a.e_out, number - 2, l == 0 ? again()->cur : nullptr);   // the sixth exchange of the layer before
             load(P_O, l);
@@ -948,7 +986,7 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
             }
         }
         if (l == 0) {
-            const int team = settle(ticket);
+            const int team = settle(arrival);
             if (__builtin_expect(team != G, 0)) return share_out<C>(args, (lds_ptr)smem);
         }
         // -------------------------------------------------------------- rotary, append, attention
@@ -1076,7 +1114,7 @@ bool trunk_plan(const vrl_trunk &t, TrunkPlan &plan) {
                              (size_t)t.M * t.n_heads * STATES * STATE,
                              (size_t)t.M * A / 2, (size_t)t.M * t.hidden / 2, (size_t)t.M * t.inter / 2,
                              (size_t)t.M * t.hidden / 2};
-    plan.bytes = 256;   // TrunkState
+    plan.bytes = sizeof(TrunkState);
     for (int i = 0; i < 6; ++i) {
         plan.words[i] = words[i];
         plan.bytes += (words[i] * 8 + 255) / 256 * 256;
@@ -1150,13 +1188,15 @@ extern "C" int vrl_decode_trunk_bf16(const vrl_trunk *trunk, void *hip_stream) {
     a.budget = t.wait_limit ? t.wait_limit : TRUNK_BUDGET;
     a.grid = plan.grid;
     a.most = t.max_workgroups ? (int)std::min(t.max_workgroups, (uint32_t)plan.grid) : plan.grid;
+    a.n_groups = ARRIVALS;
+    while (plan.grid % a.n_groups) a.n_groups /= 2;
     a.nsc_a = pp_nsc(a.A);
     a.nsc_i = pp_nsc(a.I);
     a.split_from = t.split_from > 0 ? t.split_from : INT32_MAX;
     uint8_t *ws = static_cast<uint8_t *>(t.workspace);
     a.state = reinterpret_cast<TrunkState *>(ws);
     uint64_t **const at[6] = {&a.e_qkv, &a.e_part, &a.e_attn, &a.e_mid, &a.e_act, &a.e_out};
-    size_t offset = 256;
+    size_t offset = sizeof(TrunkState);
     for (int i = 0; i < 6; ++i) {
         *at[i] = reinterpret_cast<uint64_t *>(ws + offset);
         offset += (plan.words[i] * 8 + 255) / 256 * 256;
