@@ -938,17 +938,22 @@ __device__ __forceinline__ void split_segment_pp(const DevProblem &p, int t0, in
 #pragma unroll
         for (int i = 0; i < 16; ++i) xpre[0][i] = __builtin_amdgcn_raw_buffer_load_b128(xr, voff + 16u * i, 0, 0);
     } else {
+        // In a decode step another launch has just written x, and the direct loads pay for longer than few_rows has it (us
+        // per step, other form / direct): o_proj with its adapter up to 6 rows (six layers of 2048 264.5 / 258 at 6, 263.7 /
+        // 264.6 at 8); o_proj and down_proj that join the residual where K is large (eight layers of 2048, down_proj of
+        // K = 5632 321.6 / 318.7 at 6 rows, 392 / 391.6 at 16, with o_proj of K = 2048 too 366.2 against 364.8 at 12 and 394.4
+        // at 16; six of 4096 351.5 / 346.7 at 6 rows, 481.3 / 480.3 at 16); q|k|v with adapters (six layers of 2048 304.5 /
+        // 301 at 16; of 4096 409.2 / 403.3 at 6, but 531.2 / 533.6 at 12 and 534.9 / 538 at 16).
+        const bool direct = few_rows(p) || (UP && p.M <= 6) || (EPI && p.K >= 4096) || (lora_input && (p.K < 4096 || p.M <= 8));
         __syncthreads();
         if constexpr (NORM)
             stage_x_norm(p, norm, nsc * PP_SC, xs, xstride, KS * TW,
                          t0 == 0 && (p.prepacked & PP_WRITE_H) && norm.h_out != nullptr,
                          reinterpret_cast<float *>(smem + (size_t)xrows * xstride * 2));  // the partial tiles' space, still free
+        else if (direct)
+            stage_x_direct(p, xs, xstride, KS * TW * WAVE);
         else
-            // Beside few_rows, in a decode step, where another launch has just written x (six layers of 2048, us per
-            // step): o_proj with its adapter up to 6 rows (264.5 -> 258 at 6; 263.7 against 264.6 at 8), q|k|v with
-            // adapters up to 16 (304.5 -> 301 at 16; cut into records of 16 rows and fewer: 387 against 392 at 18).
-            if (few_rows(p) || (UP && p.M <= 6) || lora_input) stage_x_direct(p, xs, xstride, KS * TW * WAVE);
-            else stage_x_natural(p, 0, nsc * PP_SC, xs, xstride, KS * TW * WAVE);
+            stage_x_natural(p, 0, nsc * PP_SC, xs, xstride, KS * TW * WAVE);
         __syncthreads();
     }
     for (int base = t0; base < t1; base += TW) {
