@@ -7,7 +7,7 @@
 // of what the launch before it wrote, a round trip for its weights and their unpacking.  Here the workgroups hand their
 // results to each other through memory in words that carry their own validity, and what does not depend on the result
 // waited for is done while waiting: a wave has its 4 KB of the next product's weights loaded and rebuilt in registers, and
-// its keys and values requested, before the input arrives.  24 x (2048, 5632), 330 slots: 769 -> 513 us at 2 rows (20 us a
+// its keys and values requested, before the input arrives.  24 x (2048, 5632), 330 slots: 780 -> 518 us at 2 rows (20 us a
 // layer, about half of it the six exchanges); six layers at 4 rows and 400 slots 212 -> 176.  At 8 rows the words alone
 // are 180 KB per workgroup and down_proj, and it was slower than the launches (254 against 216), as with rows of 4096
 // (four layers, 2 rows: 205 against 197): neither is built.
@@ -29,11 +29,11 @@
 // process, a step from another graph) keeps one of them out, for as long as it likes.  So nothing waits for a workgroup that
 // has not started.  The team is fixed once, by one compare-and-swap: by the last to arrive, with everyone, or by one that has
 // waited for the others as long as the step would take those that are there (TEAM_TICKS), with those that have taken a ticket
-// meanwhile, which is for whoever has waited TEAM_TICKS_LEAST.  Members are running by
-// then and stay, so what one waits for comes; a workgroup that starts later finds itself left out and ends.  With everyone
+// meanwhile, which is for whoever has waited TEAM_TICKS_LEAST.  Members are running by then and stay, so what one waits for
+// comes; a workgroup that starts later finds itself left out and ends.  With everyone
 // there each has its own part of every product.  Otherwise the parts are dealt out to the members, product by product:
-// the same sums and bits, without the work ahead of its input (24 layers at 2 rows: 515 us with all 256, 838 with 255 or 128
-// of them, 6.0 ms with 16; the launch list takes 766).  The team is looked up behind the first product, before anything is
+// the same sums and bits, without the work ahead of its input (24 layers at 2 rows: 518 us with all 256, 834 with 255 or 128
+// of them, 6.0 ms with 16; 1.3 ms beside a kernel that keeps one out, the wait included; the launch list takes 780).  The team is looked up behind the first product, before anything is
 // handed out, so that the arrivals cost next to nothing.
 //
 // Waits are bounded all the same: a wave gives up after `budget` unsuccessful looks in total, takes NaN for what did not
@@ -64,9 +64,10 @@ constexpr uint32_t TRUNK_BUDGET = 1u << 22; // looks of about a microsecond each
 // How long a workgroup waits for the others to start, in ticks of 10 ns: what a layer takes one workgroup alone (3.9 ms at 2
 // rows), divided by those that are there, and never less than the launch itself may need to bring all of them up.
 constexpr uint32_t TEAM_TICKS = 400000, TEAM_TICKS_LEAST = 10000;
+constexpr uint32_t UNSETTLED = 0x7FFFFFFFu;
 
 // Arrivals are counted in two levels, since those at one address are served one after the other, 27 ns each (24 layers at 2
-// rows: a single counter for 256 workgroups 526 us, this way 518; at 4 rows 632 and 623).
+// rows: a single counter for 256 workgroups 526 us, this way 517; six layers at 4 rows 189 and 181).
 constexpr int ARRIVALS = 16;
 
 // The head of the workspace.
@@ -808,47 +809,69 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
         }
     };
     // ... and the team: whoever offers first, the last of all with everyone, or one that has waited with those that have taken
-    // a ticket by then (nobody takes one at first).  Afterwards all threads know the number; returns the team's size, 0: the
-    // workspace is marked (by an earlier launch, so all workgroups find the same).
+    // a ticket by then.  Afterwards all threads know the number; returns the team's size, 0: the workspace is marked (by an
+    // earlier launch, so all workgroups find the same), UNSETTLED: nobody has offered in TEAM_TICKS_LEAST, or not all may
+    // take part.
     auto settle = [&](const Arrival &mine) {
         if (wave == TW - 1 && lane == 0) {
             const arg_ptr t = again();
             TrunkState *const state = t->state;
-            const uint32_t now = mine.first + 8u, most = t->most;
+            const uint32_t now = mine.first + 8u, all = G;
             const uint32_t gave_up = __hip_atomic_load(&state->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             uint64_t seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t offer = mine.rank && most == (uint32_t)G ? most : 0u;
-            uint32_t rank = G;   // (of a workgroup without a ticket: left out, unless everyone is in)
-            const uint64_t since = __builtin_readsteadycounter();
-            while (!gave_up && (uint32_t)(seen >> 32) != now) {
-                if (offer) {
-                    const uint64_t team = (uint64_t)now << 32 | offer;
-                    if (__hip_atomic_compare_exchange_strong(&state->team, &seen, team, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT))
-                        seen = team;
-                    continue;
+            if ((uint32_t)t->most == all) {
+                const uint64_t since = __builtin_readsteadycounter();
+                while (!gave_up && (uint32_t)(seen >> 32) != now && __builtin_readsteadycounter() - since < TEAM_TICKS_LEAST) {
+                    const uint64_t everyone = (uint64_t)now << 32 | all;
+                    if (!mine.rank)
+                        seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    else if (__hip_atomic_compare_exchange_strong(&state->team, &seen, everyone, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                                  __HIP_MEMORY_SCOPE_AGENT))
+                        seen = everyone;
                 }
-                const uint64_t waited = __builtin_readsteadycounter() - since;
-                if (waited >= TEAM_TICKS_LEAST || most != (uint32_t)G) {
-                    uint64_t tickets = __hip_atomic_load(&state->tickets, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    uint32_t count = (uint32_t)(tickets >> 32) == now ? (uint32_t)tickets : 0u;
-                    if (rank == (uint32_t)G) {
-                        if (!__hip_atomic_compare_exchange_strong(&state->tickets, &tickets, (uint64_t)now << 32 | (count + 1u),
-                                                                  __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                            continue;   // another one took it
-                        rank = count++;
-                    }
-                    const uint32_t here = min(count, most);
-                    if (rank + 1 == most || (waited >= TEAM_TICKS_LEAST && waited * here >= (uint64_t)t->n_layers * TEAM_TICKS))
-                        offer = here;
-                }
-                seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            joined[0] = now, joined[1] = gave_up ? (uint32_t)wg : rank, joined[2] = gave_up ? 0u : (uint32_t)seen;
+            // (`joined[1]`: the rank in the team, for those that have no ticket)
+            joined[0] = now;
+            joined[1] = gave_up || (uint32_t)seen == all ? (uint32_t)wg : all;
+            joined[2] = gave_up ? 0u : (uint32_t)(seen >> 32) == now ? (uint32_t)seen : UNSETTLED;
         }
         lds_barrier();
         number = __builtin_amdgcn_readfirstlane(joined[0]);
         return (int)__builtin_amdgcn_readfirstlane(joined[2]);
+    };
+    // The rest of it, out of the step's way: a ticket, and the offer once the wait is long enough for those that are there.
+    auto settle_late = [&]() {
+        if (wave == TW - 1 && lane == 0) {
+            const arg_ptr t = again();
+            TrunkState *const state = t->state;
+            const uint32_t now = joined[0], most = t->most;
+            const uint64_t since = __builtin_readsteadycounter();
+            uint64_t seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t rank = G;
+            if ((uint32_t)(seen >> 32) != now) {
+                // The first one begins the count, once; then additions, which need no second try: 255 compare-and-swaps took 500 us.
+                uint64_t tickets = __hip_atomic_load(&state->tickets, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((uint32_t)(tickets >> 32) != now)
+                    (void)__hip_atomic_compare_exchange_strong(&state->tickets, &tickets, (uint64_t)now << 32, __ATOMIC_RELAXED,
+                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                rank = (uint32_t)__hip_atomic_fetch_add(&state->tickets, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            while ((uint32_t)(seen >> 32) != now) {
+                const uint32_t count = (uint32_t)__hip_atomic_load(&state->tickets, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t here = min(count, most);
+                const uint64_t waited = __builtin_readsteadycounter() - since;
+                seen = __hip_atomic_load(&state->team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((rank + 1 == most || waited * here >= (uint64_t)t->n_layers * TEAM_TICKS) && (uint32_t)(seen >> 32) != now) {
+                    const uint64_t team = (uint64_t)now << 32 | here;
+                    if (__hip_atomic_compare_exchange_strong(&state->team, &seen, team, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT))
+                        seen = team;
+                }
+            }
+            joined[1] = (uint32_t)seen == (uint32_t)G ? (uint32_t)wg : rank;   // everyone after all: each its own parts
+            joined[2] = (uint32_t)seen;
+        }
+        lds_barrier();
     };
 
     auto mark = [&]() {
@@ -859,6 +882,9 @@ __device__ __forceinline__ void trunk_step(const TrunkArgs &a, arg_ptr args, uin
     // ---- the team is not the whole grid: every product's parts are dealt out to its members, one after the other
     if constexpr (SHARED) {
         number = __builtin_amdgcn_readfirstlane(joined[0]);
+        const uint32_t found = __builtin_amdgcn_readfirstlane(joined[2]);
+        lds_barrier();   // read by all waves before it is written again
+        if (found == UNSETTLED) settle_late();
         const int rank = __builtin_amdgcn_readfirstlane(joined[1]), team = __builtin_amdgcn_readfirstlane(joined[2]);
         static_assert(TT == ROW_WORDS, "a word each");
         if (team == 0 && rank < M) {
