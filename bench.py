@@ -626,7 +626,8 @@ def ar_decode_loop(device, tokens: int = 48, only: str | None = None, batches=(1
     ``reference_style`` is the loop of vrl/models/families/janus_pro/policy.py:624-731 with the trunk's
     dynamic cache and the torch formulas for the tail, without its per-row cache copies and host
     read-backs (so a lower bound for the reference); ``static_*`` is visionrl_amd.ar_decode over the
-    trunk module, ``native_*`` the same with the trunk as visionrl_amd.decode_step (5 launches per layer, 6 with adapters).
+    trunk module, ``native_*`` the same with the trunk as visionrl_amd.decode_step (5 launches per layer, 6 with adapters; one
+    for the whole step up to 4 rows without adapters).
     """
     import types
 
@@ -1162,7 +1163,7 @@ def main():
             step_bytes = LAYERS * sum(algorithmic_bytes(2, K, N, GROUP) for _, K, N in LAYER_LINEARS) + \
                 algorithmic_bytes(2, HIDDEN, HEAD, GROUP)
             chain = {"what": "one decode step of a Janus-Pro-1B shaped policy at B=1 (2 rows): 24 dependent layers "
-                             "(five launches each), head and sampling tail, replayed from one HIP graph",
+                             "(one launch for all), head and sampling tail, replayed from one HIP graph",
                      "ms_per_step": step_ms, "GBps_of_int4_weights": step_bytes / (step_ms * 1e-3) / 1e9,
                      "cache_slots": "304 + 48 (the start of a generation); ms_per_step_at_544_slots: its middle",
                      "ms_per_step_at_544_slots": (ar_loop.get("B1_at_544_slots") or {}).get(

@@ -18,7 +18,7 @@ arguments, the same results and the same use of the random stream:
   The prompt pass and the first decode step run eagerly (the latter doubles as the warm-up a
   capture needs).
 * When the trunk's projections are prepacked int4 modules, the trunk part of the step runs as
-  five launches per layer over the same cache tensors (:mod:`visionrl_amd.decode_step`) instead
+  five launches per layer, or one for all of them (:mod:`visionrl_amd.decode_step`), over the same cache tensors instead
   of the module's some thirty tensor ops per layer; results then agree with the module path to
   bf16 roundings of the hidden states (the attention keeps fp32 probabilities), not bit for bit.
 * The tail after the head is one launch (:func:`visionrl_amd.ops.cfg_sample`) when the logits are
@@ -408,7 +408,7 @@ class StaticARSampler:
     are never written; a two-layer head runs its front as one launch with bias and GELU and its last linear
     in that call); ``embed_table`` see :meth:`embedding_table`.  With ``native`` (the default) the trunk of a decode step runs as
     :class:`visionrl_amd.decode_step.NativeDecodeTrunk` (five launches per layer, six with LoRA
-    adapters on the attention projections) when the policy went through ``apply_int4_to_policy``
+    adapters on the attention projections, one in all for few rows without adapters) when the policy went through ``apply_int4_to_policy``
     with its defaults; otherwise, and for the prompt pass, the trunk module itself is called.
     """
 

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(const uint16_t *x,
 // ---------------------------------------------------------------- rotary + cache append + attention
 constexpr int ATTN_MAX_SPLITS = 8;   // workgroups that share the cached slots of one (row, head) in the split form
 // A row with fewer cached slots than this is left to the first workgroup of each of its pairs by a split launch
-// (the exchange of the split form costs more than it saves there: a decode step at 2 rows takes 0.82 against
+// (the exchange of the split form costs more than it saves there: a decode step's launches at 2 rows take 0.82 against
 // 0.85 ms at 450 slots, 0.86 against 0.86 at 530, 0.91 against 0.86 at 610).
 constexpr int ATTN_SPLIT_FROM = 512;
 // ... and with two workgroups per pair (65 to 128 pairs: half the compute units are busy without it) from 768:

@@ -228,7 +228,7 @@ class NativeDecodeTrunk:
         # With few (row, head) pairs and a cache that grows long the attention divides a pair's cached slots
         # over several workgroups (one workspace for all layers: the launches are ordered by the stream).
         # Its exchange costs about 1.5 us per launch, which pays from about 500 cached slots on (at 2 rows a
-        # step takes 0.85 / 0.86 / 0.86 / 0.88 ms at 450 / 530 / 610 / 830 slots against 0.82 / 0.86 / 0.91 /
+        # step's list takes 0.85 / 0.86 / 0.86 / 0.88 ms at 450 / 530 / 610 / 830 slots against 0.82 / 0.86 / 0.91 /
         # 0.96 ms); the launch is recorded once for a whole generation, and while a row has fewer than 512
         # slots filled it leaves each of the row's pairs to one workgroup, as the other form does.
         # (the library's own lines: 512 slots with 8 or 4 workgroups per pair, 768 with two, where half the
